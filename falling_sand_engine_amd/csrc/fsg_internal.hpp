@@ -54,6 +54,12 @@ struct fsg_ctx {
     // the cached graph was captured with
     fsg_tuning tune{16, -1, 5, 0};
     int graph_ticks = 0, graph_occ = 0;
+    // the tick kernel's form for the prepared batch (a BatchForm) and the one
+    // the cached graph was captured with; the awake list of a batch whose
+    // worlds all skip (global chunk indices) and its two counts
+    int batch_form = 0, graph_form = 0;
+    uint32_t *d_awake = nullptr, *d_awake_n = nullptr;
+    size_t awake_cap = 0;
     // freed device blocks by size class (dev_alloc / dev_free); the cap is at
     // least 16 GiB and a quarter of the device's memory
     std::multimap<size_t, void *> cache;

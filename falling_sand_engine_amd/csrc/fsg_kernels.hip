@@ -994,6 +994,39 @@ template __global__ void k_tick_world<0, 1, 0>(DevWorld, uint32_t, int);
 template __global__ void k_tick_world<0, 0, 1>(DevWorld, uint32_t, int);
 template __global__ void k_tick_world<0, 1, 1>(DevWorld, uint32_t, int);
 
+// The wake test of one chunk by one thread, which writes the flags of a chunk
+// that sleeps.
+__device__ __forceinline__ bool wake_test(const DevWorld &w, uint64_t tick, int tile) {
+    const int tx = tile % w.tiles_x, ty = tile / w.tiles_x;
+    const uint32_t *fr = w.flags[(tick + 1) & 1];
+    const bool forced = tick == w.force_tick;
+    bool awake = chunk_awake(w, fr, tx, ty, forced);
+    // a chunk outside the zone's reach only needs a tick to copy itself
+    if (awake && !forced && !(fr[tile] & F_ANY) && zone_test(w, tx * TW - HALO, ty * TH - HALO).dead) awake = false;
+    if (!awake) w.flags[tick & 1][tile] = 0;
+    return awake;
+}
+
+// Appends the awake threads' entries to list: the workgroup (256 threads)
+// reserves its slice with one atomic on *count.
+__device__ __forceinline__ void list_awake(bool awake, uint32_t entry, uint32_t *list, uint32_t *count) {
+    __shared__ uint32_t wave_n[4], base;
+    const uint64_t m = __ballot(awake);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (lane == 0) wave_n[wv] = (uint32_t)__popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t n = wave_n[0] + wave_n[1] + wave_n[2] + wave_n[3];
+        base = n ? atomicAdd(count, n) : 0u;
+    }
+    __syncthreads();
+    if (awake) {
+        uint32_t off = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        for (int v = 0; v < wv; v++) off += wave_n[v];
+        list[off] = entry;
+    }
+}
+
 // The awake chunks of tick t = w.tick + k, listed for k_tick_list: one thread
 // per chunk runs the wake test of the skip path (and writes the flags of the
 // chunks that sleep), then each workgroup reserves its slice of the list
@@ -1003,36 +1036,11 @@ template __global__ void k_tick_world<0, 1, 1>(DevWorld, uint32_t, int);
 // reservations; the result does not depend on it (the chunks of one tick
 // are independent).
 __global__ __launch_bounds__(256) void k_wake(DevWorld w, uint32_t k) {
-    __shared__ uint32_t wave_n[4], base;
     const uint64_t tick = w.tick + k;
-    const int ntiles = w.tiles_x * w.tiles_y;
     const int tile = (int)(blockIdx.x * 256 + threadIdx.x);
     if (tile == 0) w.awake_n[(tick + 1) & 1] = 0;
-    bool awake = false;
-    if (tile < ntiles) {
-        const int tx = tile % w.tiles_x, ty = tile / w.tiles_x;
-        const uint32_t *fr = w.flags[(tick + 1) & 1];
-        const bool forced = tick == w.force_tick;
-        awake = chunk_awake(w, fr, tx, ty, forced);
-        // a chunk outside the zone's reach only needs a tick to copy itself
-        if (awake && !forced && !(fr[tile] & F_ANY) && zone_test(w, tx * TW - HALO, ty * TH - HALO).dead)
-            awake = false;
-        if (!awake) w.flags[tick & 1][tile] = 0;
-    }
-    const uint64_t m = __ballot(awake);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) wave_n[wv] = (uint32_t)__popcll(m);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t n = wave_n[0] + wave_n[1] + wave_n[2] + wave_n[3];
-        base = n ? atomicAdd(&w.awake_n[tick & 1], n) : 0u;
-    }
-    __syncthreads();
-    if (awake) {
-        uint32_t off = base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-        for (int v = 0; v < wv; v++) off += wave_n[v];
-        w.awake[off] = (uint32_t)tile;
-    }
+    const bool awake = tile < w.tiles_x * w.tiles_y && wake_test(w, tick, tile);
+    list_awake(awake, (uint32_t)tile, w.awake, &w.awake_n[tick & 1]);
 }
 
 // Skip-path tick over the awake list: workgroup i updates the i-th listed
@@ -1061,35 +1069,70 @@ template __global__ void k_tick_list<1, 1>(DevWorld, uint32_t);
 
 // Many worlds in one launch: tile_start[i] is the first global chunk index of
 // world i (prefix sums, tile_start[n] = total).
-__device__ __forceinline__ void tick_batch_chunk(const DevWorld *__restrict__ worlds,
-                                                 const uint32_t *__restrict__ tile_start, int nworlds, uint32_t k) {
-    __shared__ __align__(16) uint32_t Lmem[LH * LW + 16];  // the region, then the 16 base colours
-    __shared__ uint32_t lut[MAX_IT + 3][256];  // pair tables, scatter offsets, the phase's class table
-    uint32_t(*L)[LW] = reinterpret_cast<uint32_t(*)[LW]>(Lmem);
-    uint32_t *rgba = Lmem + LH * LW;
-    __shared__ int32_t addt[16];
-    __shared__ uint16_t queue[(NT / 64) * qcap<NT>()];
-    __shared__ uint32_t red[NT / 64];
-    const uint32_t gt = blockIdx.x;
+__device__ __forceinline__ int world_of(const uint32_t *__restrict__ tile_start, int nworlds, uint32_t gt) {
     int lo = 0, hi = nworlds - 1;
     while (lo < hi) {  // last world with tile_start <= gt
         const int mid = (lo + hi + 1) >> 1;
         if (tile_start[mid] <= gt) lo = mid;
         else hi = mid - 1;
     }
-    const DevWorld &w = worlds[lo];
-    tile_update<2, 2, 1>(w, w.tick + k, (int)(gt - tile_start[lo]), L, lut, rgba, addt, queue, red);
+    return lo;
 }
 
-// Two register budgets of the batch tick, one of the autotuner's choices:
-// five workgroups per CU (95 VGPRs) or four (up to 128).
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_tick_batch(
-    const DevWorld *__restrict__ worlds, const uint32_t *__restrict__ tile_start, int nworlds, uint32_t k) {
-    tick_batch_chunk(worlds, tile_start, nworlds, k);
+// Batch tick of the listed chunks (SK == 3) or of every chunk.  One
+// instantiation per setting that all worlds of the batch share, as for one
+// world; SK == 2, RE == 2 (read from each world) with the zone tests serves
+// the batches whose worlds differ or have a zone.  WG: workgroups per CU
+// (the register budget), one of the autotuner's choices.
+template <int SK, int RE, int ZN, int WG>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WG))) void k_tick_batch(
+    const DevWorld *__restrict__ worlds, const uint32_t *__restrict__ tile_start, int nworlds, uint32_t k,
+    const uint32_t *__restrict__ awake, const uint32_t *__restrict__ awake_n) {
+    __shared__ __align__(16) uint32_t Lmem[LH * LW + 16];  // the region, then the 16 base colours
+    __shared__ uint32_t lut[MAX_IT + 3][256];  // pair tables, scatter offsets, the phase's class table
+    uint32_t(*L)[LW] = reinterpret_cast<uint32_t(*)[LW]>(Lmem);
+    uint32_t *rgba = Lmem + LH * LW;
+    __shared__ int32_t addt[16];
+    __shared__ uint16_t queue[(NT / 64) * qcap<NT>()];
+    __shared__ __align__(16) uint32_t red[NT / 64];
+    uint32_t gt = blockIdx.x;
+    if (SK == 3) {
+        const int n = (int)awake_n[k & 1];
+        if ((int)gt >= n) return;
+        gt = awake[xcd_order((int)gt, n, 8)];
+    }
+    const int lo = world_of(tile_start, nworlds, gt);
+    const DevWorld &w = worlds[lo];
+    tile_update<SK, RE, ZN>(w, w.tick + k, (int)(gt - tile_start[lo]), L, lut, rgba, addt, queue, red);
 }
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_tick_batch4(
-    const DevWorld *__restrict__ worlds, const uint32_t *__restrict__ tile_start, int nworlds, uint32_t k) {
-    tick_batch_chunk(worlds, tile_start, nworlds, k);
+#define FSG_BATCH(SK, RE, ZN)                                                                                      \
+    template __global__ void k_tick_batch<SK, RE, ZN, 5>(const DevWorld *, const uint32_t *, int, uint32_t,        \
+                                                         const uint32_t *, const uint32_t *);                      \
+    template __global__ void k_tick_batch<SK, RE, ZN, 4>(const DevWorld *, const uint32_t *, int, uint32_t,        \
+                                                         const uint32_t *, const uint32_t *)
+FSG_BATCH(0, 0, 0);
+FSG_BATCH(0, 1, 0);
+FSG_BATCH(1, 0, 0);
+FSG_BATCH(1, 1, 0);
+FSG_BATCH(3, 0, 0);
+FSG_BATCH(3, 1, 0);
+FSG_BATCH(2, 2, 1);
+#undef FSG_BATCH
+
+// k_wake over the chunks of every world of a batch, all of which skip: the
+// list holds global chunk indices, its counts go by the parity of k (both
+// zero before k = 0).
+__global__ __launch_bounds__(256) void k_wake_batch(const DevWorld *__restrict__ worlds,
+                                                    const uint32_t *__restrict__ tile_start, int nworlds, uint32_t k,
+                                                    uint32_t *__restrict__ awake, uint32_t *__restrict__ awake_n) {
+    const uint32_t gt = blockIdx.x * 256 + threadIdx.x;
+    if (gt == 0) awake_n[(k + 1) & 1] = 0;
+    bool wake = false;
+    if (gt < tile_start[nworlds]) {
+        const int i = world_of(tile_start, nworlds, gt);
+        wake = wake_test(worlds[i], worlds[i].tick + k, (int)(gt - tile_start[i]));
+    }
+    list_awake(wake, gt, awake, &awake_n[k & 1]);
 }
 
 __global__ void k_advance(DevWorld *worlds, int nworlds, uint32_t ticks) {
@@ -1424,6 +1467,6 @@ __global__ __launch_bounds__(256) void k_stamp_compact(StampArgs a) {
         if (bits >> b & 1u) a.open[k++] = hi | (p0 + 256u * b);
 }
 
-__global__ void k_zero_u32(uint32_t *p) { *p = 0; }
+__global__ void k_zero_u32(uint32_t *p) { p[threadIdx.x] = 0; }
 
 } // namespace fsg

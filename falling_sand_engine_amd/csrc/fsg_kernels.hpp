@@ -39,10 +39,12 @@ template <int RE, int ZN>
 __global__ void k_tick_small(DevWorld w, uint32_t k);
 template <int RE, int ZN>
 __global__ void k_tick_quarter(DevWorld w, uint32_t k);
+template <int SK, int RE, int ZN, int WG>
 __global__ void k_tick_batch(const DevWorld *__restrict__ worlds, const uint32_t *__restrict__ tile_start,
-                             int nworlds, uint32_t k);
-__global__ void k_tick_batch4(const DevWorld *__restrict__ worlds, const uint32_t *__restrict__ tile_start,
-                              int nworlds, uint32_t k);
+                             int nworlds, uint32_t k, const uint32_t *__restrict__ awake,
+                             const uint32_t *__restrict__ awake_n);
+__global__ void k_wake_batch(const DevWorld *__restrict__ worlds, const uint32_t *__restrict__ tile_start,
+                             int nworlds, uint32_t k, uint32_t *__restrict__ awake, uint32_t *__restrict__ awake_n);
 __global__ void k_advance(DevWorld *worlds, int nworlds, uint32_t ticks);
 __global__ void k_temperature(const uint64_t *__restrict__ in, uint64_t *__restrict__ out, int W, int H,
                               MatTab M, int4 zone);
