@@ -176,9 +176,8 @@ void fill_pair_table(DevWorld &d) {
 // The block-class tables of the classification pass (DevWorld::ct), for a
 // world of at most 8 materials: the class of every block of 3-bit material
 // ids at every iteration, from the pair table.  bit 0: some pair relation
-// (K_SINK, K_GRISE, K_HSWAP, K_REACT); bit 1: plain (no gas or reaction in
-// the columns, no gas diagonal, no horizontal swap); bits 2-3: K_TSANDACT of
-// the top left / right cell.
+// (K_SINK, K_GRISE, K_HSWAP, K_REACT); bit 1: block_sinks; bits 2-3:
+// K_TSANDACT of the top left / right cell.
 std::vector<uint32_t> class_tables(const DevWorld &d) {
     std::vector<uint32_t> t((size_t)fsg::MAX_IT * 512, 0u);
     for (int it = 0; it < fsg::MAX_IT; it++)
@@ -188,9 +187,7 @@ std::vector<uint32_t> class_tables(const DevWorld &d) {
             const uint32_t VL = P(i0, i2), VR = P(i1, i3), DL = P(i0, i3), DR = P(i1, i2), HT = P(i0, i1),
                            HB = P(i2, i3);
             const uint32_t rel = (VL | VR | DL | DR | HT | HB) & (fsg::K_SINK | fsg::K_GRISE | fsg::K_HSWAP | fsg::K_REACT);
-            const uint32_t other = ((VL | VR) & (fsg::K_GRISE | fsg::K_REACT)) | ((DL | DR) & fsg::K_GRISE) |
-                                   ((HT | HB) & fsg::K_HSWAP);
-            const uint32_t nib = (rel ? 1u : 0u) | (other ? 0u : 2u) | (((VL >> 8) & 1u) << 2) | (((VR >> 8) & 1u) << 3);
+            const uint32_t nib = (rel ? 1u : 0u) | (fsg::block_sinks(VL, VR) ? 2u : 0u) | (((VL >> 8) & 1u) << 2) | (((VR >> 8) & 1u) << 3);
             t[(size_t)it * 512 + (i >> 3)] |= nib << ((i & 7u) * 4);
         }
     return t;
@@ -298,7 +295,11 @@ extern "C" int fsg_rule_eval(const fsg_config *cfg, int it, uint32_t r, uint32_t
         if (!fsg::block_react(M, c)) return FSG_ERR_STATE;  // the kernel queues only blocks that react
     } else {
         if (fsg::block_inert(VL, VR, DL, DR, HT, HB, movA, movB)) return 0;
-        fsg::apply_decision(fsg::block_decide(VL, VR, DL, DR, HT, HTR, HB, movA, movB, movC, movD, r, s), c);
+        const bool sinks = fsg::block_sinks(VL, VR);
+        if (!(sinks && fsg::block_sink(VL, VR, DL, DR, HTR, r, c[0], c[1], c[2], c[3])))
+            fsg::apply_decision(fsg::block_decide(VL, VR, DL, DR, HT, HTR, HB, movA, movB, movC, movD, r, s,
+                                                  !sinks && fsg::block_may_fall(VL, VR),
+                                                  fsg::block_gas_h(DL, DR, HT, HB)), c);
     }
     uint64_t o[4];
     bool ch = false;

@@ -59,7 +59,7 @@ struct DevWorld {
     // (worlds of at most 8 materials; null otherwise): word i0<<6|i1<<3|i2 of
     // table it holds, in nibble i3, the class of a block of material ids
     // i0 i1 / i2 i3 at iteration it: bit 0 some pair relation (K_SINK,
-    // K_GRISE, K_HSWAP, K_REACT), bit 1 plain, bits 2-3 K_TSANDACT of the top
+    // K_GRISE, K_HSWAP, K_REACT), bit 1 block_sinks, bits 2-3 K_TSANDACT of the top
     // left / right cell
     const uint32_t *ct;
     MatTab mat;
@@ -120,10 +120,13 @@ __host__ __device__ __forceinline__ uint32_t xform(const MatTab &, uint32_t c, u
     return m | (c & (0xFFFF0000u | C_ORG)) | C_XF;
 }
 
-// Block random words for the block whose top-left world cell is (x0, y0).
-__host__ __device__ __forceinline__ void block_hash(uint64_t key, int x0, int y0, uint32_t &r, uint32_t &s) {
-    const uint32_t pos = (uint32_t)(x0 + 1) | ((uint32_t)(y0 + 1) << 16);
-    r = lowbias32(pos ^ (uint32_t)key);
+// Block random words for the block whose top-left world cell is (x0, y0),
+// pos = (x0 + 1) | (y0 + 1) << 16; stage V uses the first one only.
+__host__ __device__ __forceinline__ uint32_t block_hash1(uint64_t key, uint32_t pos) {
+    return lowbias32(pos ^ (uint32_t)key);
+}
+__host__ __device__ __forceinline__ void block_hash(uint64_t key, uint32_t pos, uint32_t &r, uint32_t &s) {
+    r = block_hash1(key, pos);
     s = lowbias32(r ^ (uint32_t)(key >> 32));
 }
 
@@ -371,53 +374,45 @@ __host__ __device__ __forceinline__ uint32_t pair_code(const MatTab &M, int it, 
 //   bits 12-15 MOVED cleared on original cell k (bit 12 + k)
 // All intermediate values are 0/1 integers, so the stages combine with plain
 // bit operations instead of divergent branches.  Same result as block_rule
-// for blocks where no reaction fires.  GAS_H = false compiles the form for
-// blocks with no K_GRISE bit in VL, VR, DL, DR and no K_HSWAP bit in HT, HB
-// (the gas and horizontal terms are then zero).
-template <bool GAS_H = true>
+// for blocks where no reaction fires.  The caller may leave out, for a wave
+// whose blocks all allow it, stage V (vert = false: block_may_fall is false,
+// or block_sink found that no column sinks) and the gas diagonals and stage
+// H (gas_h = false: block_gas_h is false).
 __host__ __device__ __forceinline__ uint32_t block_decide(uint32_t VL, uint32_t VR, uint32_t DL, uint32_t DR,
                                                           uint32_t HT, uint32_t HTR, uint32_t HB,
                                                           uint32_t movA, uint32_t movB, uint32_t movC,
-                                                          uint32_t movD, uint32_t r, uint32_t s) {
-    if (!GAS_H) {
-        VL &= ~K_GRISE;
-        VR &= ~K_GRISE;
-        DL &= ~K_GRISE;
-        DR &= ~K_GRISE;
-        HT = 0;
-        HB = 0;
-    }
-    const uint32_t sL = VL & 1u, sR = VR & 1u, dL = DL & 1u, dR = DR & 1u, htr = HTR & 1u;
-    const uint32_t gL = (VL >> 1) & 1u, gR = (VR >> 1) & 1u, gdl = (DL >> 1) & 1u, gdr = (DR >> 1) & 1u;
+                                                          uint32_t movD, uint32_t r, uint32_t s, bool vert,
+                                                          bool gas_h) {
+    const uint32_t sL = VL & 1u, sR = VR & 1u, dL = DL & 1u, dR = DR & 1u;
     const uint32_t sandA = (VL >> 4) & 1u, sandB = (VR >> 4) & 1u;
     const uint32_t sandC = (VL >> 5) & 1u, sandD = (VR >> 5) & 1u;
-    const uint32_t airA = (VL >> 6) & 1u, airB = (DR >> 6) & 1u, airC = (VL >> 7) & 1u;
-    const uint32_t actA = (VL >> 8) & 1u, actB = (VR >> 8) & 1u;
-    const uint32_t hT = (HT >> 2) & 1u, hB = (HB >> 2) & 1u;
-    const uint32_t T1 = (r & 0xFu) == 0, T2 = (r & 0xF0u) == 0, T5 = (r & 0xC00u) == 0, T6 = (r & 0x3000u) == 0;
-    const uint32_t T3 = (r >> 8) & 1u, T4 = (r >> 9) & 1u, T7 = (r >> 14) & 1u, T8 = (r >> 15) & 1u;
-    const uint32_t UA = (r & 0xF0000u) == 0, UB = (r & 0xF00000u) == 0;  // stopped sand unsticks
-    const uint32_t S1 = (s & 0x1Fu) == 0, S2 = (s & 0x3E0u) == 0, S4 = (s & 0xFF800u) == 0;
-    const uint32_t S5 = (s & 0x300000u) == 0;
-    const uint32_t S3 = (s >> 10) & 1u, S6 = (s >> 22) & 1u, S7 = (s >> 23) & 1u, S8 = (s >> 24) & 1u;
+    const uint32_t airA = (VL >> 6) & 1u, airB = (DR >> 6) & 1u;
+    uint32_t y = 0, set = 0, nvm = 1;
 
     // V: left column, then the right column seeing the left column's result
-    const uint32_t vLs = sL & ((sandA & dL & T1) ^ 1u);
-    const uint32_t vLg = (sL ^ 1u) & gL & ((airB & T7) ^ 1u);
-    const uint32_t vL = vLs | vLg;
-    const uint32_t sinksBnewC = vL ? htr : dR;           // after a left swap, new BL is old TL
-    const uint32_t vRs = sR & ((sandB & sinksBnewC & T2) ^ 1u);
-    const uint32_t airNewA = vL ? airC : airA;           // after a left swap, new TL is old BL
-    const uint32_t vRg = (sR ^ 1u) & gR & ((airNewA & T8) ^ 1u);
-    const uint32_t vR = vRs | vRg;
-    const uint32_t vm = vL | vR;
-    uint32_t set = (vLs & sandA & T3) | ((vRs & sandB & T4) << 1) | ((vLs & sandA & T5 & sandD) << 3);
-    const uint32_t nudR = vRs & sandB & T6 & (vL ? sandA : sandC);
-    set |= vL ? nudR : (nudR << 2);
-    uint32_t y = (vL * 0x22u) | (vR * 0x88u);
+    if (vert) {
+        const uint32_t htr = HTR & 1u, gL = (VL >> 1) & 1u, gR = (VR >> 1) & 1u, airC = (VL >> 7) & 1u;
+        const uint32_t T1 = (r & 0xFu) == 0, T2 = (r & 0xF0u) == 0, T5 = (r & 0xC00u) == 0, T6 = (r & 0x3000u) == 0;
+        const uint32_t T3 = (r >> 8) & 1u, T4 = (r >> 9) & 1u, T7 = (r >> 14) & 1u, T8 = (r >> 15) & 1u;
+        const uint32_t vLs = sL & ((sandA & dL & T1) ^ 1u);
+        const uint32_t vLg = (sL ^ 1u) & gL & ((airB & T7) ^ 1u);
+        const uint32_t vL = vLs | vLg;
+        const uint32_t sinksBnewC = vL ? htr : dR;           // after a left swap, new BL is old TL
+        const uint32_t vRs = sR & ((sandB & sinksBnewC & T2) ^ 1u);
+        const uint32_t airNewA = vL ? airC : airA;           // after a left swap, new TL is old BL
+        const uint32_t vRg = (sR ^ 1u) & gR & ((airNewA & T8) ^ 1u);
+        const uint32_t vR = vRs | vRg;
+        set = (vLs & sandA & T3) | ((vRs & sandB & T4) << 1) | ((vLs & sandA & T5 & sandD) << 3);
+        const uint32_t nudR = vRs & sandB & T6 & (vL ? sandA : sandC);
+        set |= vL ? nudR : (nudR << 2);
+        y = (vL * 0x22u) | (vR * 0x88u);
+        nvm = (vL | vR) ^ 1u;
+    }
 
-    // D: sinking diagonals with sand friction, then gas diagonals
-    const uint32_t nvm = vm ^ 1u;
+    // D: sinking diagonals with sand friction
+    const uint32_t UA = (r & 0xF0000u) == 0, UB = (r & 0xF00000u) == 0;  // stopped sand unsticks
+    const uint32_t S1 = (s & 0x1Fu) == 0, S2 = (s & 0x3E0u) == 0, S4 = (s & 0xFF800u) == 0;
+    const uint32_t S5 = (s & 0x300000u) == 0, S3 = (s >> 10) & 1u;
     const uint32_t cl0 = nvm & dL, cr0 = nvm & dR;
     const uint32_t mvA = movA | UA, mvB = movB | UB;
     const uint32_t failA = cl0 & sandA & mvA & S1, failB = cr0 & sandB & mvB & S2;
@@ -431,28 +426,45 @@ __host__ __device__ __forceinline__ uint32_t block_decide(uint32_t VL, uint32_t 
     set |= (cl & sandA & UA) | ((cr & sandB & UB) << 1);  // an unstuck slider moves (S4 may clear it)
     y |= cl * (0xC3u ^ (airB * 0x44u));  // swap TL/BR, or 3-cycle TL->BR->TR->TL when TR is air
     y |= cr * (0x3Cu ^ (airA * 0x11u));  // swap TR/BL, or 3-cycle TR->BL->TL->TR when TL is air
-    const uint32_t none = nvm & (cl ^ 1u) & (cr ^ 1u);
-    const uint32_t gl0 = none & gdr, gr0 = none & gdl;
-    const uint32_t gb = gl0 & gr0;
-    const uint32_t gl = gl0 & ((gb & S6) ^ 1u), gr = gr0 & ((gb & (S6 ^ 1u)) ^ 1u);
-    y |= (gl * 0x3Cu) | (gr * 0xC3u);
-    const uint32_t rest = none & (gl ^ 1u) & (gr ^ 1u);
+    uint32_t rest = nvm & (cl ^ 1u) & (cr ^ 1u);
+
+    if (gas_h) {
+        // gas diagonals
+        const uint32_t gdl = (DL >> 1) & 1u, gdr = (DR >> 1) & 1u;
+        const uint32_t S6 = (s >> 22) & 1u, S7 = (s >> 23) & 1u, S8 = (s >> 24) & 1u;
+        const uint32_t gl0 = rest & gdr, gr0 = rest & gdl;
+        const uint32_t gb = gl0 & gr0;
+        const uint32_t gl = gl0 & ((gb & S6) ^ 1u), gr = gr0 & ((gb & (S6 ^ 1u)) ^ 1u);
+        y |= (gl * 0x3Cu) | (gr * 0xC3u);
+        rest &= (gl ^ 1u) & (gr ^ 1u);
+        // H: per row, a SOUP cell that can flow sideways moves if it faces the
+        // other cell (MOVED set: heading right), else turns and moves with
+        // p=1/16, taking the new heading; otherwise gas spreads with p=1/2
+        const uint32_t hT = (HT >> 2) & 1u, hB = (HB >> 2) & 1u;
+        const uint32_t fAB = (HT >> 9) & 1u, fBA = (HT >> 10) & 1u, fCD = (HB >> 9) & 1u, fDC = (HB >> 10) & 1u;
+        const uint32_t lT = fAB | fBA, lB = fCD | fDC;
+        const uint32_t TT = (r & 0xF000000u) == 0, TB = (r & 0xF0000000u) == 0;
+        const uint32_t goT = rest & ((lT & ((fAB & movA) | (fBA & (movB ^ 1u)) | TT)) | ((lT ^ 1u) & hT & S7));
+        const uint32_t goB = rest & ((lB & ((fCD & movC) | (fDC & (movD ^ 1u)) | TB)) | ((lB ^ 1u) & hB & S8));
+        y ^= goT * 0x05u;
+        y ^= goB * 0x50u;
+        set |= (goT & fAB) | ((goB & fCD) << 2);
+        clr |= ((goT & fBA) << 1) | ((goB & fDC) << 3);
+    }
 
     // F: an active sand top cell with no straight or in-block diagonal move stops
+    const uint32_t actA = (VL >> 8) & 1u, actB = (VR >> 8) & 1u;
     clr |= (rest & actA & (sL ^ 1u) & (dL ^ 1u)) | ((rest & actB & (sR ^ 1u) & (dR ^ 1u)) << 1);
-    // H: per row, a SOUP cell that can flow sideways moves if it faces the
-    // other cell (MOVED set: heading right), else turns and moves with
-    // p=1/16, taking the new heading; otherwise gas spreads with p=1/2
-    const uint32_t fAB = (HT >> 9) & 1u, fBA = (HT >> 10) & 1u, fCD = (HB >> 9) & 1u, fDC = (HB >> 10) & 1u;
-    const uint32_t lT = fAB | fBA, lB = fCD | fDC;
-    const uint32_t TT = (r & 0xF000000u) == 0, TB = (r & 0xF0000000u) == 0;
-    const uint32_t goT = rest & ((lT & ((fAB & movA) | (fBA & (movB ^ 1u)) | TT)) | ((lT ^ 1u) & hT & S7));
-    const uint32_t goB = rest & ((lB & ((fCD & movC) | (fDC & (movD ^ 1u)) | TB)) | ((lB ^ 1u) & hB & S8));
-    y ^= goT * 0x05u;
-    y ^= goB * 0x50u;
-    set |= (goT & fAB) | ((goB & fCD) << 2);
-    clr |= ((goT & fBA) << 1) | ((goB & fDC) << 3);
     return y | (set << 8) | (clr << 12);
+}
+
+// A column of the block may sink or its gas may rise.
+__host__ __device__ __forceinline__ bool block_may_fall(uint32_t VL, uint32_t VR) {
+    return ((VL | VR) & (K_SINK | K_GRISE)) != 0;
+}
+// Gas may rise diagonally or a row may swap.
+__host__ __device__ __forceinline__ bool block_gas_h(uint32_t DL, uint32_t DR, uint32_t HT, uint32_t HB) {
+    return (((DL | DR) & K_GRISE) | ((HT | HB) & K_HSWAP)) != 0;
 }
 
 // True if no rule can change the block for any random draw: no pair
@@ -461,6 +473,34 @@ __host__ __device__ __forceinline__ bool block_inert(uint32_t VL, uint32_t VR, u
                                                      uint32_t HT, uint32_t HB, uint32_t movA, uint32_t movB) {
     const uint32_t rel = (VL | VR | DL | DR | HT | HB) & (K_SINK | K_GRISE | K_HSWAP | K_REACT);
     return rel == 0 && ((((VL >> 8) & movA) | ((VR >> 8) & movB)) & 1u) == 0;
+}
+
+// True if the block may sink and neither gas rises nor a reaction fires in
+// its columns: if a column then sinks (block_sink), that is the block's
+// whole change, and if none does the block takes the general decision.
+__host__ __device__ __forceinline__ bool block_sinks(uint32_t VL, uint32_t VR) {
+    return ((VL | VR) & (K_SINK | K_GRISE | K_REACT)) == K_SINK;
+}
+
+// Stage V of such a block on its cells (TL, TR, BL, BR); false, with the
+// cells as they were, if no column sinks.
+__host__ __device__ __forceinline__ bool block_sink(uint32_t VL, uint32_t VR, uint32_t DL, uint32_t DR, uint32_t HTR,
+                                                    uint32_t r, uint32_t &q0, uint32_t &q1, uint32_t &q2,
+                                                    uint32_t &q3) {
+    const uint32_t sandA = VL >> 4, sandB = VR >> 4, sandC = VL >> 5, sandD = VR >> 5;  // bit 0 of each
+    const uint32_t T1 = (r & 0xFu) == 0, T2 = (r & 0xF0u) == 0, T5 = (r & 0xC00u) == 0, T6 = (r & 0x3000u) == 0;
+    // the left column, then the right column seeing the left column's result
+    const uint32_t vL = VL & ~(sandA & DL & T1) & 1u;
+    const uint32_t vR = VR & ~(sandB & (vL ? HTR : DR) & T2) & 1u;
+    // MOVED: a falling sand grain with p=1/2, a grain beside its landing with p=1/4
+    const uint32_t fL = vL & sandA, fR = vR & sandB, nudge = fR & T6;
+    const uint32_t a = q0 | ((fL & ((r >> 8) | nudge)) << 8), b = q1 | ((fR & (r >> 9)) << 8);
+    const uint32_t c = q2 | ((nudge & ~vL & sandC) << 8), d = q3 | ((fL & sandD & T5) << 8);
+    q0 = vL ? c : a;
+    q2 = vL ? a : c;
+    q1 = vR ? d : b;
+    q3 = vR ? b : d;
+    return (vL | vR) != 0;
 }
 
 // Host form of the decision's effect on q (the kernel scatters to LDS).

@@ -112,16 +112,31 @@ constexpr int qcap() { return ((36 * 36 + N - 1) / N) * 64; }
 // (need = cell_iter - it, so the region shrinks by one ring per phase and the
 // last phase leaves the one ring the temperature stencil reads).
 //
-// Two passes per wave.  The first tests every block against the pair table
-// and queues the ones some rule may change (ballot + mbcnt into the wave's
-// LDS queue Q): "plain" blocks (no reaction, no gas or horizontal relation:
-// sand over air, most of a world) from the front, the others from the back.
-// The second pass runs the random draw and the rule on the queued blocks
-// only, plain ones with the decision form that omits the gas and horizontal
-// terms, so no lane idles through the decision for an inert block.  Blocks
-// of a phase are disjoint and a wave's LDS accesses stay in order, so the
-// passes need no barrier.  With TRACK, returns the band bits of chunk cells
-// that changed.
+// Three passes.  The first tests every block against the pair table (or the
+// class table) and queues the ones some rule may change (ballot + mbcnt into
+// the wave's LDS queue Q), so no lane idles through a decision for an inert
+// block: blocks that may sink and in whose columns neither gas rises nor a
+// reaction fires ("sinking": two thirds of the active blocks or more) from
+// the front, the others from the back.  The second pass runs stage V alone
+// on the sinking blocks, with one random word: a block that sinks is then
+// done, and the few that do not (sand that skips its fall) join the others.
+// The third runs the whole decision on those.  It needs four times the
+// instructions and each wave has only part of a round of them, so in the
+// 256-thread form the workgroup's waves share them (a barrier; the phase's
+// blocks are disjoint, so who decides a block does not matter).  A wave's
+// own LDS accesses stay in order, so nothing else needs a barrier.  With
+// TRACK, returns the band bits of chunk cells that changed.
+//
+// The first pass's thread map is fixed: a thread keeps one block column and
+// every block_sweep-th block row, so its LDS address and its queue entry
+// (column | row << 8, LDS coordinates) advance by constants.
+//
+// The tick is bound by VALU issue.  Against two queues by "plain" and other
+// blocks, each decided by its wave with one whole decision, a wave of the
+// all-active 16384^2 world issues 1,494 VALU instructions instead of 1,907
+// and the tick takes 904 us instead of 957; a reacting 2048^2 world 24.8
+// instead of 27.8, a 1000x611 one (k_tick_small) 15.5 instead of 18.2.
+//
 // Block origins (LDS coordinates) whose block holds a tick-zone cell:
 // [x0, x0 + w) x [y0, y0 + h); `on` is false when every block does.
 struct ZoneBlocks {
@@ -130,17 +145,25 @@ struct ZoneBlocks {
     uint32_t w, h;
 };
 
+// Block columns of a phase (at most, over the parities and rings) for a
+// square of EXT chunk cells, and the block rows N threads take per sweep.
+template <int EXT> constexpr int block_cols() { return EXT / 2 + HALO; }
+template <int N, int EXT> constexpr int block_sweep() { return N / block_cols<EXT>(); }
+
 // EXT: the side of the square of chunk cells the tick computes, from chunk
 // coordinates (cx0, cy0): the whole chunk, or a quarter of it.
 // DIRECT: no classification; each thread decides one block at a time with
-// the general form (the same result for inert and plain blocks), for
+// the general form (the same result for inert and sinking blocks), for
 // workgroups with about as many threads as the phase has blocks, where the
 // classification pass only lengthens the chain of dependent steps.
-template <int N, bool TRACK, bool REACT, bool ZONE, int EXT = TW, bool DIRECT = false>
+// between(): called by every thread after the third pass's barrier, when
+// the class table of this phase has been read for the last time.
+template <int N, bool TRACK, bool REACT, bool ZONE, int EXT = TW, bool DIRECT = false, typename Between>
 __device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW], const uint32_t *T, int it,
                                               uint64_t key, int ox, int oy, int need, int gx0, int gy0,
-                                              bool has_wood, uint16_t *queue, const uint32_t *perm,
-                                              const ZoneBlocks &zb, const uint32_t *ct, int cx0 = 0, int cy0 = 0) {
+                                              bool has_wood, uint16_t *queue, uint32_t *qcount, const uint32_t *perm,
+                                              const ZoneBlocks &zb, const uint32_t *ct, Between between, int cx0 = 0,
+                                              int cy0 = 0) {
     static_assert(EXT == TW || !TRACK, "band tracking covers whole chunks");
     // first/last block origin (chunk coordinates) with the phase's parity
     const int xlo = cx0 - need, ylo = cy0 - need;
@@ -148,65 +171,21 @@ __device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW]
     const int x0l = (cx0 + EXT - 1 + need) - (((cx0 + EXT - 1 + need) ^ ox) & 1);
     const int y0l = (cy0 + EXT - 1 + need) - (((cy0 + EXT - 1 + need) ^ oy) & 1);
     const int nbx = ((x0l - x0f) >> 1) + 1, nby = ((y0l - y0f) >> 1) + 1;
-    const int nb = nbx * nby;
-    const uint32_t magic = (65536u + (uint32_t)nbx - 1u) / (uint32_t)nbx;  // b / nbx for b < 2^16/nbx
     const int lx0 = HALO + x0f, ly0 = HALO + y0f;
-    // LDS coordinates of block b's top-left cell, and that cell
-    auto block_xy = [&](int b, int &lx, int &ly) {
-        const int by = (int)(__umul24((uint32_t)b, magic) >> 16);
-        const int bx = b - (int)__umul24((uint32_t)by, (uint32_t)nbx);
-        lx = lx0 + 2 * bx;
-        ly = ly0 + 2 * by;
-    };
-    auto block_at = [&](int b) -> uint32_t * {
-        int lx, ly;
-        block_xy(b, lx, ly);
-        return &L[0][0] + __umul24((uint32_t)ly, (uint32_t)LW) + lx;
-    };
-    auto in_zone = [&](int b) -> bool {
-        const int by = (int)(__umul24((uint32_t)b, magic) >> 16);
-        const int bx = b - (int)__umul24((uint32_t)by, (uint32_t)nbx);
-        return (uint32_t)(lx0 + 2 * bx - zb.x0) < zb.w && (uint32_t)(ly0 + 2 * by - zb.y0) < zb.h;
+    // hash position of LDS cell (0, 0): that of a block is this plus its
+    // LDS coordinates in the two halves (both stay in 0 .. 65535 for every
+    // block that can change, whose origin is at least -1)
+    const uint32_t pos0 = (uint32_t)(gx0 + 1) + ((uint32_t)(gy0 + 1) << 16);
+    uint32_t *const L0 = &L[0][0];
+    auto in_zone = [&](int lx, int ly) -> bool {
+        return (uint32_t)(lx - zb.x0) < zb.w && (uint32_t)(ly - zb.y0) < zb.h;
     };
     const int lane = threadIdx.x & 63;
     constexpr int QCAP = qcap<N>();
-    // the wave's first block as a uniform: the compiler cannot tell that
-    // threadIdx.x & ~63 is one, and would run the loop under exec masks
+    // the wave's first thread as a uniform: the compiler cannot tell that
+    // threadIdx.x & ~63 is one, and would run loops under exec masks
     const int wb0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
     uint16_t *Q = queue + (wb0 >> 6) * QCAP;
-    int nplain = 0, nother = 0;  // wave-uniform
-    for (int b0 = wb0; b0 < nb && !DIRECT; b0 += N) {
-        const int b = b0 + lane;
-        // lanes past the last block test the last one again and queue nothing
-        const uint32_t *p0 = block_at(b < nb ? b : nb - 1);
-        const uint32_t q0 = p0[0], q1 = p0[1], q2 = p0[LW], q3 = p0[LW + 1];
-        bool act, plain;
-        if (ct) {  // one class-table read (ids < 8: at most 8 materials and no wall in the region)
-            const uint32_t nib = (ct[((q0 & 7u) << 6) | ((q1 & 7u) << 3) | (q2 & 7u)] >> ((q3 & 7u) << 2)) & 15u;
-            act = ((nib | ((nib >> 2) & (q0 >> 8)) | ((nib >> 3) & (q1 >> 8))) & 1u) != 0;
-            plain = (nib & 2u) != 0;
-        } else {
-            const uint32_t i0 = q0 & 15u, i1 = q1 & 15u, i2 = q2 & 15u, i3 = q3 & 15u;
-            const uint32_t VL = T[(i0 << 4) | i2], VR = T[(i1 << 4) | i3];
-            const uint32_t DL = T[(i0 << 4) | i3], DR = T[(i1 << 4) | i2];
-            const uint32_t HT = T[(i0 << 4) | i1], HB = T[(i2 << 4) | i3];
-            act = !block_inert(VL, VR, DL, DR, HT, HB, (q0 >> 8) & 1u, (q1 >> 8) & 1u);
-            plain = ((((VL | VR) & (K_GRISE | K_REACT)) | ((DL | DR) & K_GRISE) | ((HT | HB) & K_HSWAP)) == 0);
-        }
-        if (REACT && has_wood && (wood_hot(M, q0) || wood_hot(M, q1) || wood_hot(M, q2) || wood_hot(M, q3))) {
-            act = true;
-            plain = false;
-        }
-        act = act && b < nb;
-        if (ZONE) act = act && in_zone(b);  // workgroups on the zone's edge only
-        plain = plain && act;
-        const uint64_t mp = __builtin_amdgcn_ballot_w64(plain), mo = __builtin_amdgcn_ballot_w64(act && !plain);
-        const int bp = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mp >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mp, 0u));
-        const int bo = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mo >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mo, 0u));
-        if (act) Q[plain ? nplain + bp : QCAP - 1 - (nother + bo)] = (uint16_t)b;
-        nplain += __popcll(mp);
-        nother += __popcll(mo);
-    }
     uint32_t bands = 0;
     auto track = [&](bool wrote, int lx, int ly) {
         if (TRACK && wrote) {
@@ -226,28 +205,9 @@ __device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW]
             p0[(po >> (8 * k)) & 0xFFu] = v;
         }
     };
-    // uniform loops over the queues (rounds of 64 blocks)
-    for (int qi = 0; qi < nplain; qi += 64) {
-        const int i = qi + lane;
-        if (i >= nplain) continue;  // the last round's idle lanes (not a divergent exit)
-        int lx, ly;
-        block_xy(Q[i], lx, ly);
-        uint32_t *p0 = &L[0][0] + __umul24((uint32_t)ly, (uint32_t)LW) + lx;
-        const uint32_t q[4] = {p0[0], p0[1], p0[LW], p0[LW + 1]};
-        const uint32_t i0 = q[0] & 15u, i1 = q[1] & 15u, i2 = q[2] & 15u, i3 = q[3] & 15u;
-        uint32_t r, s;
-        block_hash(key, gx0 + lx, gy0 + ly, r, s);
-        const uint32_t dec = block_decide<false>(T[(i0 << 4) | i2], T[(i1 << 4) | i3], T[(i0 << 4) | i3],
-                                                 T[(i1 << 4) | i2], 0u, T[(i1 << 4) | i0], 0u,
-                                                 (q[0] >> 8) & 1u, (q[1] >> 8) & 1u, 0u, 0u, r, s);
-        if (dec != 0) scatter(p0, q, dec);
-        track(dec != 0, lx, ly);
-    }
-    // the general form of a block: reactions, gas and horizontal relations
-    auto general = [&](int b) {
-        int lx, ly;
-        block_xy(b, lx, ly);
-        uint32_t *p0 = &L[0][0] + __umul24((uint32_t)ly, (uint32_t)LW) + lx;
+    // the whole decision of the block at LDS (lx, ly)
+    auto general = [&](int lx, int ly) {
+        uint32_t *p0 = L0 + __umul24((uint32_t)ly, (uint32_t)LW) + lx;
         uint32_t q[4] = {p0[0], p0[1], p0[LW], p0[LW + 1]};
         const uint32_t i0 = q[0] & 15u, i1 = q[1] & 15u, i2 = q[2] & 15u, i3 = q[3] & 15u;
         const uint32_t VL = T[(i0 << 4) | i2], VR = T[(i1 << 4) | i3];
@@ -260,7 +220,7 @@ __device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW]
                                               T[(i2 << 4) | i3], (q[0] >> 8) & 1u, (q[1] >> 8) & 1u)))
             return;
         uint32_t r, s;
-        block_hash(key, gx0 + lx, gy0 + ly, r, s);
+        block_hash(key, pos0 + (uint32_t)lx + ((uint32_t)ly << 16), r, s);
         bool wrote = false;
         if (REACT && (hot || ((VL | VR) & K_REACT))) {
             if (block_react(M, q)) {
@@ -271,27 +231,130 @@ __device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW]
                 wrote = true;
             }
         } else {
-            const uint32_t dec = block_decide<true>(VL, VR, T[(i0 << 4) | i3], T[(i1 << 4) | i2], T[(i0 << 4) | i1],
-                                                    T[(i1 << 4) | i0], T[(i2 << 4) | i3], (q[0] >> 8) & 1u,
-                                                    (q[1] >> 8) & 1u, (q[2] >> 8) & 1u, (q[3] >> 8) & 1u, r, s);
+            const uint32_t DL = T[(i0 << 4) | i3], DR = T[(i1 << 4) | i2];
+            const uint32_t HT = T[(i0 << 4) | i1], HB = T[(i2 << 4) | i3];
+            // stages no block of the wave needs are left out (classified
+            // blocks that may sink come here only after they did not)
+            const bool vert = __builtin_amdgcn_ballot_w64(block_may_fall(VL, VR) && (DIRECT || !block_sinks(VL, VR)));
+            const bool gas_h = __builtin_amdgcn_ballot_w64(block_gas_h(DL, DR, HT, HB));
+            const uint32_t dec = block_decide(VL, VR, DL, DR, HT, T[(i1 << 4) | i0], HB, (q[0] >> 8) & 1u,
+                                              (q[1] >> 8) & 1u, (q[2] >> 8) & 1u, (q[3] >> 8) & 1u, r, s, vert, gas_h);
             if (dec != 0) scatter(p0, q, dec);
             wrote = dec != 0;
         }
         track(wrote, lx, ly);
     };
+    constexpr int COLS = block_cols<EXT>(), SWEEP = block_sweep<N, EXT>();
     if (DIRECT) {
-        for (int b0 = wb0; b0 < nb; b0 += N) {
-            const int b = b0 + lane;
-            if (b >= nb) continue;
-            if (ZONE && !in_zone(b)) continue;
-            general(b);
+        // sweeps of SWEEP block rows over a fixed thread map
+        const int br = (int)threadIdx.x / COLS, bc = (int)threadIdx.x - br * COLS;
+        for (int b0 = 0; b0 < nby; b0 += SWEEP) {
+            if (bc >= nbx || br >= SWEEP || b0 + br >= nby) continue;
+            const int lx = lx0 + 2 * bc, ly = ly0 + 2 * (b0 + br);
+            if (ZONE && !in_zone(lx, ly)) continue;
+            general(lx, ly);
         }
         return bands;
     }
-    for (int qi = 0; qi < nother; qi += 64) {
-        const int i = qi + lane;
-        if (i >= nother) continue;
-        general(Q[QCAP - 1 - i]);
+    int nsink = 0, nother = 0;  // wave-uniform
+    {
+        int br = (int)threadIdx.x / COLS;
+        const int bc = (int)threadIdx.x - br * COLS;
+        uint32_t e = (uint32_t)(lx0 + 2 * bc) | ((uint32_t)(ly0 + 2 * br) << 8);
+        uint32_t off = __umul24((uint32_t)(ly0 + 2 * br), (uint32_t)LW) + (uint32_t)(lx0 + 2 * bc);
+        if (bc >= nbx || br >= SWEEP) br = 1 << 20;  // never in range
+        for (int b0 = 0; b0 < nby; b0 += SWEEP, e += (uint32_t)(2 * SWEEP) << 8, off += (uint32_t)(2 * SWEEP * LW)) {
+            const bool in = br < nby - b0;
+            // lanes without a block test the region's first one and queue nothing
+            const uint32_t *p0 = L0 + (in ? off : 0u);
+            const uint32_t q0 = p0[0], q1 = p0[1], q2 = p0[LW], q3 = p0[LW + 1];
+            bool act, sink;
+            if (ct) {  // one class-table read (ids < 8: at most 8 materials and no wall in the region)
+                const uint32_t nib = ct[((q0 & 7u) << 6) | ((q1 & 7u) << 3) | (q2 & 7u)] >> ((q3 & 7u) << 2);
+                act = ((nib & 1u) | ((((nib << 6) & q0) | ((nib << 5) & q1)) & (uint32_t)MOVED)) != 0;
+                sink = (nib & 2u) != 0;
+            } else {
+                const uint32_t i0 = q0 & 15u, i1 = q1 & 15u, i2 = q2 & 15u, i3 = q3 & 15u;
+                const uint32_t VL = T[(i0 << 4) | i2], VR = T[(i1 << 4) | i3];
+                const uint32_t DL = T[(i0 << 4) | i3], DR = T[(i1 << 4) | i2];
+                const uint32_t HT = T[(i0 << 4) | i1], HB = T[(i2 << 4) | i3];
+                act = !block_inert(VL, VR, DL, DR, HT, HB, (q0 >> 8) & 1u, (q1 >> 8) & 1u);
+                sink = block_sinks(VL, VR);
+            }
+            if (REACT && has_wood && (wood_hot(M, q0) || wood_hot(M, q1) || wood_hot(M, q2) || wood_hot(M, q3))) {
+                act = true;
+                sink = false;
+            }
+            act = act && in;
+            if (ZONE) act = act && in_zone((int)(e & 0xFFu), (int)(e >> 8));  // workgroups on the zone's edge only
+            const uint64_t ma = __builtin_amdgcn_ballot_w64(act), ms = __builtin_amdgcn_ballot_w64(sink) & ma;
+            const uint64_t mo = ma & ~ms;
+            if (act) {
+                const uint32_t ks = __builtin_amdgcn_mbcnt_hi((uint32_t)(ms >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)ms, (uint32_t)nsink));
+                const uint32_t ko = __builtin_amdgcn_mbcnt_hi((uint32_t)(mo >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)mo, (uint32_t)nother));
+                Q[sink ? ks : (uint32_t)(QCAP - 1) - ko] = (uint16_t)e;
+            }
+            nsink += __popcll(ms);
+            nother += __popcll(mo);
+        }
+    }
+    // stage V on the sinking blocks, the queue's last round first: the
+    // entries that join the others take the places of entries already done
+    for (int top = nsink; top > 0; top -= 64) {
+        const int i = top - 1 - lane;
+        bool stay = false;
+        uint32_t e = 0;
+        if (i >= 0) {  // the last round's idle lanes (not a divergent exit)
+            e = Q[i];
+            const uint32_t lx = e & 0xFFu, ly = e >> 8;
+            uint32_t *p0 = L0 + __umul24(ly, (uint32_t)LW) + lx;
+            uint32_t q0 = p0[0], q1 = p0[1], q2 = p0[LW], q3 = p0[LW + 1];
+            const uint32_t i0 = q0 & 15u, i1 = q1 & 15u, i2 = q2 & 15u, i3 = q3 & 15u;
+            const uint32_t r = block_hash1(key, pos0 + lx + (ly << 16));
+            stay = !block_sink(T[(i0 << 4) | i2], T[(i1 << 4) | i3], T[(i0 << 4) | i3], T[(i1 << 4) | i2],
+                               T[(i1 << 4) | i0], r, q0, q1, q2, q3);
+            if (!stay) {
+                p0[0] = q0;
+                p0[1] = q1;
+                p0[LW] = q2;
+                p0[LW + 1] = q3;
+            }
+            track(!stay, (int)lx, (int)ly);
+        }
+        const uint64_t mo = __builtin_amdgcn_ballot_w64(stay);
+        if (stay) {
+            const uint32_t ko = __builtin_amdgcn_mbcnt_hi((uint32_t)(mo >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo((uint32_t)mo, (uint32_t)nother));
+            Q[(uint32_t)(QCAP - 1) - ko] = (uint16_t)e;
+        }
+        nother += __popcll(mo);
+    }
+    if (N == 256) {
+        // the others of all four waves, in rounds of 64 dealt to the waves
+        // in turn, starting with another wave each phase
+        if (lane == 0) qcount[wb0 >> 6] = (uint32_t)nother;
+        __syncthreads();
+        between();
+        const uint4 c = *reinterpret_cast<const uint4 *>(qcount);
+        const int n0 = __builtin_amdgcn_readfirstlane((int)c.x), n1 = n0 + __builtin_amdgcn_readfirstlane((int)c.y);
+        const int n2 = n1 + __builtin_amdgcn_readfirstlane((int)c.z), n3 = n2 + __builtin_amdgcn_readfirstlane((int)c.w);
+        for (int r0 = (((wb0 >> 6) + it) & 3) * 64; r0 < n3; r0 += 256) {
+            const int j = r0 + lane;
+            if (j >= n3) continue;
+            const int w = (j >= n0 ? 1 : 0) + (j >= n1 ? 1 : 0) + (j >= n2 ? 1 : 0);
+            const int k = j - (j >= n2 ? n2 : j >= n1 ? n1 : j >= n0 ? n0 : 0);
+            const uint32_t e = queue[w * QCAP + QCAP - 1 - k];
+            general((int)(e & 0xFFu), (int)(e >> 8));
+        }
+    } else {
+        for (int qi = 0; qi < nother; qi += 64) {
+            const int i = qi + lane;
+            if (i >= nother) continue;
+            const uint32_t e = Q[QCAP - 1 - i];
+            general((int)(e & 0xFFu), (int)(e >> 8));
+        }
     }
     return bands;
 }
@@ -601,22 +664,22 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
             const uint64_t key = splitmix64(seedmix ^ g);
             const int ox = kOX[g & 3], oy = kOY[g & 3];
             // the next iteration's class table, loaded while this phase runs
+            // and put in place when its classification is over
             const bool next_ct = use_ct && it + 1 < ci;
             if (next_ct && tab) ctv = reinterpret_cast<const uint2 *>(w.ct + (it + 1) * 512)[tid];
+            auto refill = [&]() {
+                if (next_ct && tab) reinterpret_cast<uint2 *>(lut[MAX_IT + 1])[tid] = ctv;
+            };
             if (zt.blocks.on)  // on the zone's edge: one form for every setting (the bands may go unused)
                 bands |= run_phase<N, true, RE != 0, true>(M, L, lut[it], it, key, ox, oy, ci - it, gx0, gy0, has_wood,
-                                                        queue, lut[MAX_IT], zt.blocks, ct);
+                                                        queue, red, lut[MAX_IT], zt.blocks, ct, refill);
             else if (SK != 0 && skip)
                 bands |= run_phase<N, true, RE != 0, false>(M, L, lut[it], it, key, ox, oy, ci - it, gx0, gy0, has_wood,
-                                                         queue, lut[MAX_IT], zt.blocks, ct);
+                                                         queue, red, lut[MAX_IT], zt.blocks, ct, refill);
             else if (SK != 1 && SK != 3)
                 run_phase<N, false, RE != 0, false>(M, L, lut[it], it, key, ox, oy, ci - it, gx0, gy0, has_wood, queue,
-                                                 lut[MAX_IT], zt.blocks, ct);
+                                                 red, lut[MAX_IT], zt.blocks, ct, refill);
             __syncthreads();
-            if (next_ct) {  // every wave's classification of this phase is done
-                if (tab) reinterpret_cast<uint2 *>(lut[MAX_IT + 1])[tid] = ctv;
-                __syncthreads();
-            }
         }
     }
 
@@ -774,7 +837,7 @@ static_assert(TW == 2 * QW && TH == 2 * QH && (QW & 1) == 0, "quarters of whole 
 template <int RE, int ZN, int N, bool SEP = false>
 __device__ __forceinline__ void quarter_update(const DevWorld &w, uint64_t tick, int tile, int quad,
                                                uint32_t (*L)[LW], uint32_t (*lut)[256], uint32_t *rgba,
-                                               int32_t *addt, uint16_t *queue, uint32_t *colw = nullptr) {
+                                               int32_t *addt, uint16_t *queue, uint32_t *red, uint32_t *colw = nullptr) {
     static_assert(N == 256 || N == 512 || N == 1024, "one pair-table entry per thread, write-back strips");
     const int tid = threadIdx.x;
     const MatTab &M = w.mat;
@@ -866,12 +929,12 @@ __device__ __forceinline__ void quarter_update(const DevWorld &w, uint64_t tick,
         constexpr bool DIRECT = N >= 1024;
         if (ZN && zt.blocks.on)
             run_phase<N, false, RE != 0, true, QW, DIRECT>(M, L, lut[it], it, key, kOX[g & 3], kOY[g & 3], ci - it,
-                                                           gx0, gy0, has_wood, queue, lut[MAX_IT], zt.blocks, nullptr,
-                                                           cx0, cy0);
+                                                           gx0, gy0, has_wood, queue, red, lut[MAX_IT], zt.blocks,
+                                                           nullptr, [] {}, cx0, cy0);
         else
             run_phase<N, false, RE != 0, false, QW, DIRECT>(M, L, lut[it], it, key, kOX[g & 3], kOY[g & 3], ci - it,
-                                                            gx0, gy0, has_wood, queue, lut[MAX_IT], zt.blocks, nullptr,
-                                                            cx0, cy0);
+                                                            gx0, gy0, has_wood, queue, red, lut[MAX_IT], zt.blocks,
+                                                            nullptr, [] {}, cx0, cy0);
         __syncthreads();
     }
 
@@ -943,7 +1006,7 @@ __global__ __launch_bounds__(QUARTER_NT) void k_tick_quarter(DevWorld w, uint32_
     __shared__ uint16_t queue[(QUARTER_NT / 64) * qcap<QUARTER_NT>()];
     __shared__ __align__(8) uint32_t colw[QLW * QLH];  // the window's colours
     quarter_update<RE, ZN, QUARTER_NT, true>(w, w.tick + k, (int)(blockIdx.x >> 2), (int)(blockIdx.x & 3u), L, lut,
-                                             rgba, addt, queue, colw);
+                                             rgba, addt, queue, nullptr, colw);
 }
 template __global__ void k_tick_quarter<0, 0>(DevWorld, uint32_t);
 template __global__ void k_tick_quarter<1, 0>(DevWorld, uint32_t);
@@ -972,7 +1035,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_
     uint32_t *rgba = Lmem + LH * LW;
     __shared__ int32_t addt[16];
     __shared__ uint16_t queue[(NT / 64) * qcap<NT>()];
-    __shared__ uint32_t red[NT / 64];
+    __shared__ __align__(16) uint32_t red[NT / 64];
     const int i = (int)blockIdx.x;
     if (i < nfull) {
         tile_update<SK, RE, ZN>(w, w.tick + k, xcd_order(i, nfull, (w.tiles_x & 7) ? 8 : w.tiles_x >> 3), L, lut,
@@ -986,7 +1049,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_
         const int q = i - nfull, nq = (int)gridDim.x - nfull, full = nq & ~31;
         const int c = q < full ? (q & 7) + ((q >> 5) << 3) : q >> 2;
         const int quad = q < full ? (q >> 3) & 3 : q & 3;
-        quarter_update<RE, ZN, NT>(w, w.tick + k, nfull + c, quad, L, lut, rgba, addt, queue);
+        quarter_update<RE, ZN, NT>(w, w.tick + k, nfull + c, quad, L, lut, rgba, addt, queue, red);
     }
 }
 template __global__ void k_tick_world<0, 0, 0>(DevWorld, uint32_t, int);
@@ -1055,7 +1118,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_
     uint32_t *rgba = Lmem + LH * LW;
     __shared__ int32_t addt[16];
     __shared__ uint16_t queue[(NT / 64) * qcap<NT>()];
-    __shared__ uint32_t red[NT / 64];
+    __shared__ __align__(16) uint32_t red[NT / 64];
     const uint64_t tick = w.tick + k;
     const int n = (int)w.awake_n[tick & 1];
     if ((int)blockIdx.x >= n) return;
