@@ -10,8 +10,9 @@
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <string>
 #include <new>
+#include <string>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 
@@ -228,40 +229,34 @@ int launch_tick(fsg_world *w) {
         }
         w->list_any = false;
         w->list_next = w->d.tick + 1;
-    } else if (4 * tiles <= (unsigned)w->ctx->n_cu) {
-        // at most a quarter chunk per compute unit: four workgroups per chunk
-        // (512^2 world: 9.7 us a tick instead of 11.2)
-        if (zoned) {
-            if (re) fsg::k_tick_quarter<1, 1><<<4 * tiles, fsg::QUARTER_NT, 0, st>>>(w->d, 0u);
-            else fsg::k_tick_quarter<0, 1><<<4 * tiles, fsg::QUARTER_NT, 0, st>>>(w->d, 0u);
-        } else {
-            if (re) fsg::k_tick_quarter<1, 0><<<4 * tiles, fsg::QUARTER_NT, 0, st>>>(w->d, 0u);
-            else fsg::k_tick_quarter<0, 0><<<4 * tiles, fsg::QUARTER_NT, 0, st>>>(w->d, 0u);
-        }
-    } else if (tiles <= (unsigned)w->ctx->n_cu) {
-        // at most one chunk per compute unit: 1024 threads per chunk (a 512^2
-        // world ticks in 11.4 us instead of 16.0; with more chunks than
-        // compute units the big workgroups take two rounds and lose)
-        if (zoned) {
-            if (re) fsg::k_tick_small<1, 1><<<tiles, fsg::SMALL_NT, 0, st>>>(w->d, 0u);
-            else fsg::k_tick_small<0, 1><<<tiles, fsg::SMALL_NT, 0, st>>>(w->d, 0u);
-        } else {
-            if (re) fsg::k_tick_small<1, 0><<<tiles, fsg::SMALL_NT, 0, st>>>(w->d, 0u);
-            else fsg::k_tick_small<0, 0><<<tiles, fsg::SMALL_NT, 0, st>>>(w->d, 0u);
-        }
     } else {
-        // whole chunks in full rounds of resident workgroups (five per CU),
-        // the remainder as quarters
-        const unsigned slots = 5u * (unsigned)w->ctx->n_cu;
-        const unsigned nfull = tiles <= slots ? tiles : tiles / slots * slots;
-        const unsigned grid = nfull + 4u * (tiles - nfull);
-        if (zoned) {
-            if (re) fsg::k_tick_world<0, 1, 1><<<grid, fsg::NT, 0, st>>>(w->d, 0u, (int)nfull);
-            else fsg::k_tick_world<0, 0, 1><<<grid, fsg::NT, 0, st>>>(w->d, 0u, (int)nfull);
-        } else {
-            if (re) fsg::k_tick_world<0, 1, 0><<<grid, fsg::NT, 0, st>>>(w->d, 0u, (int)nfull);
-            else fsg::k_tick_world<0, 0, 0><<<grid, fsg::NT, 0, st>>>(w->d, 0u, (int)nfull);
-        }
+        // us a tick at the lines (both sides): 64 chunks as quarters 7.6, as
+        // whole chunks of 1024 threads 10.9; 160 chunks of 1024 threads 14.9,
+        // of 512 15.0; 289 chunks of 512 threads 15.6, of 256 18.2; 484 of
+        // 512 19.6, of 256 20.1, and 1024 of 512 27.2, of 256 24.5: with
+        // more chunks per compute unit the wider workgroups take more rounds
+        const unsigned cu = (unsigned)w->ctx->n_cu;
+        const unsigned slots = (unsigned)(fsg::WGS_PER_CU - (zoned ? 1 : 0)) * cu, rest = tiles % slots;
+        // whole chunks in full rounds of resident workgroups, a remainder of
+        // at most a quarter round as quarters, which then fill one round (a
+        // larger one as whole chunks: 4096^2 world, 1024 left over, 59 us a
+        // tick instead of 68)
+        const unsigned nfull = tiles <= slots || 4 * rest > slots ? tiles : tiles - rest;
+        auto launch = [&](auto re_, auto zn_) {
+            constexpr int R = decltype(re_)::value, Z = decltype(zn_)::value;
+            if (4 * tiles <= cu)
+                fsg::k_tick_quarter<R, Z><<<4 * tiles, fsg::QUARTER_NT, 0, st>>>(w->d, 0u);
+            else if (tiles <= cu)
+                fsg::k_tick_small<R, Z, fsg::SMALL_NT><<<tiles, fsg::SMALL_NT, 0, st>>>(w->d, 0u);
+            else if (tiles <= 2 * cu)
+                fsg::k_tick_small<R, Z, fsg::MEDIUM_NT><<<tiles, fsg::MEDIUM_NT, 0, st>>>(w->d, 0u);
+            else
+                fsg::k_tick_world<R, Z><<<nfull + 4u * (tiles - nfull), fsg::NT, 0, st>>>(w->d, 0u, (int)nfull);
+        };
+        using No = std::integral_constant<int, 0>;
+        using Yes = std::integral_constant<int, 1>;
+        if (zoned) re ? launch(Yes{}, Yes{}) : launch(No{}, Yes{});
+        else re ? launch(Yes{}, No{}) : launch(No{}, No{});
     }
     HIPCHK(hipGetLastError());
     w->d.tick++;
@@ -1065,7 +1060,7 @@ int batch_form(const fsg_ctx *c, const DevWorld *dw, int n, uint64_t total) {
         const bool zoned = d.zx0 > 0 || d.zy0 > 0 || d.zx1 < d.W || d.zy1 < d.H;
         if (zoned || (d.skip != 0) != sk || (d.mat.reactions != 0) != re) return BF_ANY;
     }
-    return (!sk ? BF_PLAIN : total <= 5 * (uint64_t)c->n_cu ? BF_SKIP : BF_LIST) + (re ? 1 : 0);
+    return (!sk ? BF_PLAIN : total <= (fsg::WGS_PER_CU - 1) * (uint64_t)c->n_cu ? BF_SKIP : BF_LIST) + (re ? 1 : 0);
 }
 bool batch_listed(const fsg_ctx *c) { return c->batch_form == BF_LIST || c->batch_form == BF_LIST_REACT; }
 
@@ -1168,7 +1163,8 @@ int batch_run(fsg_ctx *c, fsg_world *const *ws, int n, int ticks, bool graph_ok)
     const unsigned tiles = c->total_tiles;
     const int T = c->tune.graph_ticks;
     const bool listed = batch_listed(c);
-    const BatchKernel kernel = c->tune.occupancy == 4 ? batch_kernel<4>(c->batch_form) : batch_kernel<5>(c->batch_form);
+    const BatchKernel kernel =
+        c->tune.occupancy == 4 ? batch_kernel<4>(c->batch_form) : batch_kernel<fsg::WGS_PER_CU>(c->batch_form);
     auto tick_launch = [&](uint32_t k) {
         if (listed)
             fsg::k_wake_batch<<<grid_for(tiles, 256), 256, 0, c->stream>>>(c->d_worlds, c->d_tile_start, n, k,

@@ -18,6 +18,8 @@
 #include "fsg_device.hpp"
 #include "fsg_kernels.hpp"
 
+#include <type_traits>
+
 namespace fsg {
 
 static_assert(NT == 256, "one pair-table entry per thread and iteration");
@@ -64,8 +66,8 @@ __device__ __forceinline__ int temp_of(const MatTab &M, const int32_t *addt, int
 // pair of cells of the LDS region (the chunk and its HALO ring) take part in
 // a rule under some random draw, can any cell change alone, or is any
 // temperature stencil of the chunk non-zero?
-template <int N>
-__device__ bool tile_unstable(const MatTab &M, const uint32_t (*L)[LW], const uint32_t *T0, const int32_t *addt,
+template <int N, typename Pair>
+__device__ bool tile_unstable(const MatTab &M, const uint32_t (*L)[LW], const Pair *T0, const int32_t *addt,
                               bool temp_enabled) {
     bool u = false;
     constexpr uint32_t KV = K_SINK | K_GRISE | K_REACT, KD = K_SINK | K_GRISE;
@@ -102,10 +104,54 @@ __device__ bool tile_unstable(const MatTab &M, const uint32_t (*L)[LW], const ui
     return u;
 }
 
-// Blocks a wave handles in one phase: at most ceil(36 * 36 / N) rounds of 64,
-// for a workgroup of N threads.
-template <int N>
-constexpr int qcap() { return ((36 * 36 + N - 1) / N) * 64; }
+// Block columns of a phase (at most, over the parities and rings) for a
+// square of EXT chunk cells, and the block rows N threads take per sweep.
+template <int EXT> constexpr int block_cols() { return EXT / 2 + HALO; }
+template <int N, int EXT> constexpr int block_sweep() { return N / block_cols<EXT>(); }
+
+// The wave's part of the block queue ends at entry queue_end(wave): room for
+// every block of a phase that its lanes see.  At 256 threads a sweep takes 7
+// of at most 36 block rows, so the sixth holds one row, all of it wave 0's.
+template <int N> constexpr int queue_end(int wave) {
+    constexpr int C = block_cols<TW>(), S = block_sweep<N, TW>(), full = C / S, rest = (C - full * S) * C;
+    static_assert(N != NT || rest <= 64, "the last sweep's blocks are wave 0's");
+    return N == NT ? (wave + 1) * full * 64 + rest : (wave + 1) * (full + (rest ? 1 : 0)) * 64;
+}
+template <int N> constexpr int queue_begin(int wave) { return wave ? queue_end<N>(wave - 1) : 0; }
+
+// A workgroup's LDS.  At 256 threads its size sets how many workgroups a
+// compute unit holds: LDS is handed out in 1280-byte steps, so six fit in
+// 160 KB up to 26,880 bytes (with the 256 bytes of a workgroup-wide OR).
+// That is why the 256-thread form keeps pair and class tables for two and
+// one iterations only, refilled while a phase runs, and why cell moves are
+// computed (scatter), not looked up.
+template <int N> struct TileLds {
+    static constexpr int PT = N == NT ? 2 : MAX_IT;  // pair tables held
+    uint32_t L[LH][LW];                              // the region
+    uint32_t rgba[16];                               // base colours
+    int32_t addt[16];
+    uint32_t ct[N == NT ? 512 : 4];                  // the phase's class table
+    alignas(16) uint32_t red[N / 64];
+    uint32_t perm[N == NT ? 4 : 256];                // cell moves by scatter mask (fill_perm)
+    using Pair = typename std::conditional<N == NT, uint16_t, uint32_t>::type;
+    Pair pair[PT][256];                              // iteration it's pair table: pair[it % PT]
+    uint16_t queue[queue_end<N>(N / 64 - 1)];
+};
+static_assert(sizeof(TileLds<NT>) + 256 <= 26880, "six workgroups per CU");
+
+// perm[y]: in byte k, the LDS offset (from the block's top-left cell) of the
+// place cell k goes to under scatter mask y, k ^ ((y >> 2k) & 3).
+template <int N> __device__ __forceinline__ void fill_perm(TileLds<N> &S) {
+    const uint32_t y = threadIdx.x;
+    if (N == NT || y >= 256) return;
+    uint32_t po = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const uint32_t d = (uint32_t)k ^ ((y >> (2 * k)) & 3u);
+        po |= ((d & 1u) + (d >> 1) * (uint32_t)LW) << (8 * k);
+    }
+    S.perm[y] = po;
+}
 
 // One Margolus phase over the blocks whose cells the rest of the tick still
 // reads: after this phase the tick needs `need` more rings around the chunk
@@ -145,11 +191,6 @@ struct ZoneBlocks {
     uint32_t w, h;
 };
 
-// Block columns of a phase (at most, over the parities and rings) for a
-// square of EXT chunk cells, and the block rows N threads take per sweep.
-template <int EXT> constexpr int block_cols() { return EXT / 2 + HALO; }
-template <int N, int EXT> constexpr int block_sweep() { return N / block_cols<EXT>(); }
-
 // EXT: the side of the square of chunk cells the tick computes, from chunk
 // coordinates (cx0, cy0): the whole chunk, or a quarter of it.
 // DIRECT: no classification; each thread decides one block at a time with
@@ -159,11 +200,9 @@ template <int N, int EXT> constexpr int block_sweep() { return N / block_cols<EX
 // between(): called by every thread after the third pass's barrier, when
 // the class table of this phase has been read for the last time.
 template <int N, bool TRACK, bool REACT, bool ZONE, int EXT = TW, bool DIRECT = false, typename Between>
-__device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW], const uint32_t *T, int it,
-                                              uint64_t key, int ox, int oy, int need, int gx0, int gy0,
-                                              bool has_wood, uint16_t *queue, uint32_t *qcount, const uint32_t *perm,
-                                              const ZoneBlocks &zb, const uint32_t *ct, Between between, int cx0 = 0,
-                                              int cy0 = 0) {
+__device__ __forceinline__ uint32_t run_phase(const MatTab &M, TileLds<N> &S, int it, uint64_t key, int ox, int oy,
+                                              int need, int gx0, int gy0, bool has_wood, const ZoneBlocks &zb,
+                                              const uint32_t *ct, Between between, int cx0 = 0, int cy0 = 0) {
     static_assert(EXT == TW || !TRACK, "band tracking covers whole chunks");
     // first/last block origin (chunk coordinates) with the phase's parity
     const int xlo = cx0 - need, ylo = cy0 - need;
@@ -176,16 +215,19 @@ __device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW]
     // LDS coordinates in the two halves (both stay in 0 .. 65535 for every
     // block that can change, whose origin is at least -1)
     const uint32_t pos0 = (uint32_t)(gx0 + 1) + ((uint32_t)(gy0 + 1) << 16);
-    uint32_t *const L0 = &L[0][0];
+    uint32_t *const L0 = &S.L[0][0];
+    const typename TileLds<N>::Pair *T = S.pair[TileLds<N>::PT == MAX_IT ? it : it & 1];
+    uint16_t *const queue = S.queue;
     auto in_zone = [&](int lx, int ly) -> bool {
         return (uint32_t)(lx - zb.x0) < zb.w && (uint32_t)(ly - zb.y0) < zb.h;
     };
     const int lane = threadIdx.x & 63;
-    constexpr int QCAP = qcap<N>();
     // the wave's first thread as a uniform: the compiler cannot tell that
     // threadIdx.x & ~63 is one, and would run loops under exec masks
     const int wb0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u));
-    uint16_t *Q = queue + (wb0 >> 6) * QCAP;
+    const int wave = wb0 >> 6;
+    uint16_t *Q = queue + queue_begin<N>(wave);
+    const int qcap = queue_end<N>(wave) - queue_begin<N>(wave);
     uint32_t bands = 0;
     auto track = [&](bool wrote, int lx, int ly) {
         if (TRACK && wrote) {
@@ -194,15 +236,17 @@ __device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW]
                 bands |= band_bits(max(cx, 0), min(cx + 1, TW - 1), max(cy, 0), min(cy + 1, TH - 1));
         }
     };
-    // perm[y] holds, in byte k, the LDS offset (from the block's top-left
-    // cell) of the destination of cell k under scatter mask y
     auto scatter = [&](uint32_t *p0, const uint32_t (&q)[4], uint32_t dec) {
-        const uint32_t po = perm[dec & 0xFFu];
+        // cell k goes to (to >> 2k) & 3; larger workgroups, whose LDS is not
+        // what limits them, read its offset from a table (512^2 world, 1024
+        // threads: 7.6 us a tick against 7.9 computed)
+        const uint32_t to = dec ^ 0xE4u, po = N == NT ? 0u : S.perm[dec & 0xFFu];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             // MOVED set on cell k (dec bit 8 + k), then cleared (bit 12 + k)
             const uint32_t v = (q[k] | ((dec >> k) & (uint32_t)MOVED)) & ~((dec >> (k + 4)) & (uint32_t)MOVED);
-            p0[(po >> (8 * k)) & 0xFFu] = v;
+            p0[N == NT ? ((to >> (2 * k)) & 1u) + __umul24((to >> (2 * k + 1)) & 1u, (uint32_t)LW)
+                       : (po >> (8 * k)) & 0xFFu] = v;
         }
     };
     // the whole decision of the block at LDS (lx, ly)
@@ -294,7 +338,7 @@ __device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW]
                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)ms, (uint32_t)nsink));
                 const uint32_t ko = __builtin_amdgcn_mbcnt_hi((uint32_t)(mo >> 32),
                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)mo, (uint32_t)nother));
-                Q[sink ? ks : (uint32_t)(QCAP - 1) - ko] = (uint16_t)e;
+                Q[sink ? ks : (uint32_t)(qcap - 1) - ko] = (uint16_t)e;
             }
             nsink += __popcll(ms);
             nother += __popcll(mo);
@@ -327,34 +371,29 @@ __device__ __forceinline__ uint32_t run_phase(const MatTab &M, uint32_t (*L)[LW]
         if (stay) {
             const uint32_t ko = __builtin_amdgcn_mbcnt_hi((uint32_t)(mo >> 32),
                                                           __builtin_amdgcn_mbcnt_lo((uint32_t)mo, (uint32_t)nother));
-            Q[(uint32_t)(QCAP - 1) - ko] = (uint16_t)e;
+            Q[(uint32_t)(qcap - 1) - ko] = (uint16_t)e;
         }
         nother += __popcll(mo);
     }
-    if (N == 256) {
-        // the others of all four waves, in rounds of 64 dealt to the waves
-        // in turn, starting with another wave each phase
-        if (lane == 0) qcount[wb0 >> 6] = (uint32_t)nother;
-        __syncthreads();
-        between();
-        const uint4 c = *reinterpret_cast<const uint4 *>(qcount);
-        const int n0 = __builtin_amdgcn_readfirstlane((int)c.x), n1 = n0 + __builtin_amdgcn_readfirstlane((int)c.y);
-        const int n2 = n1 + __builtin_amdgcn_readfirstlane((int)c.z), n3 = n2 + __builtin_amdgcn_readfirstlane((int)c.w);
-        for (int r0 = (((wb0 >> 6) + it) & 3) * 64; r0 < n3; r0 += 256) {
-            const int j = r0 + lane;
-            if (j >= n3) continue;
-            const int w = (j >= n0 ? 1 : 0) + (j >= n1 ? 1 : 0) + (j >= n2 ? 1 : 0);
-            const int k = j - (j >= n2 ? n2 : j >= n1 ? n1 : j >= n0 ? n0 : 0);
-            const uint32_t e = queue[w * QCAP + QCAP - 1 - k];
-            general((int)(e & 0xFFu), (int)(e >> 8));
-        }
-    } else {
-        for (int qi = 0; qi < nother; qi += 64) {
-            const int i = qi + lane;
-            if (i >= nother) continue;
-            const uint32_t e = Q[QCAP - 1 - i];
-            general((int)(e & 0xFFu), (int)(e >> 8));
-        }
+    // the others of all waves, in rounds of 64 dealt to the waves in turn,
+    // starting with another wave each phase
+    constexpr int NW = N / 64;
+    if (lane == 0) S.red[wave] = (uint32_t)nother;
+    __syncthreads();
+    between();
+    int upto[NW];  // others of waves 0 .. w, wave-uniform
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+        upto[w] = (w ? upto[w - 1] : 0) + __builtin_amdgcn_readfirstlane((int)S.red[w]);
+    for (int r0 = ((wave + it) & (NW - 1)) * 64; r0 < upto[NW - 1]; r0 += N) {
+        const int j = r0 + lane;
+        if (j >= upto[NW - 1]) continue;
+        int at = queue_end<N>(0) - 1 - j;  // the j-th other's entry
+#pragma unroll
+        for (int w = 0; w + 1 < NW; w++)
+            if (j >= upto[w]) at = queue_end<N>(w + 1) - 1 + upto[w] - j;
+        const uint32_t e = queue[at];
+        general((int)(e & 0xFFu), (int)(e >> 8));
     }
     return bands;
 }
@@ -490,9 +529,11 @@ __device__ __forceinline__ bool chunk_awake(const DevWorld &w, const uint32_t *f
 // the awake list k_wake built).  ZN: the tick zone is tested (1), or the
 // world's zone covers it and no zone code is compiled in (0).
 template <int SK, int RE, int ZN, int N = NT>
-__device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, int tile, uint32_t (*L)[LW],
-                                            uint32_t (*lut)[256], uint32_t *rgba, int32_t *addt,
-                                            uint16_t *queue, uint32_t *red) {
+__device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, int tile, TileLds<N> &S) {
+    uint32_t(*L)[LW] = S.L;
+    uint32_t *const rgba = S.rgba;
+    int32_t *const addt = S.addt;
+    constexpr int PT = TileLds<N>::PT;
     static_assert(N == 256 || N == 512 || N == 1024, "the load map and the write-back strips");
     constexpr int RS = rows_per_sweep<N>(), KC = sweeps<N>();
     // sweep k of this thread's rows lies in rows 1 .. LH-2 (always, unless the
@@ -535,7 +576,8 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
     // as 16-byte cell pairs) is issued before the first LDS write, so a
     // workgroup waits for one memory latency, not one per loop trip.
     const int ci = (int)M.cell_iter;
-    uint32_t pv[MAX_IT];
+    // (the first iteration's tables, or all of them where LDS holds them all)
+    uint16_t pv[MAX_IT];
     const bool tab = N == 256 || tid < 256;  // one pair-table entry per thread
 #pragma unroll
     for (int k = 0; k < MAX_IT; k++)
@@ -618,19 +660,10 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
         if (edge) wood |= (ve.x & 0xFFu) == M.wood || (ve.z & 0xFFu) == M.wood;
     }
 #pragma unroll
-    for (int k = 0; k < MAX_IT; k++)
-        if (k < ci && tab) lut[k][tid] = pv[k];
-    if (tab) {
-        // scatter offsets for mask y = tid: cell k goes to k ^ ((y >> 2k) & 3)
-        uint32_t po = 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const uint32_t d = (uint32_t)k ^ (((uint32_t)tid >> (2 * k)) & 3u);
-            po |= ((d & 1u) + (d >> 1) * (uint32_t)LW) << (8 * k);
-        }
-        lut[MAX_IT][tid] = po;
-        if (use_ct) reinterpret_cast<uint2 *>(lut[MAX_IT + 1])[tid] = ctv;
-    }
+    for (int k = 0; k < PT; k++)
+        if (k < ci && tab) S.pair[k][tid] = pv[k];
+    if (use_ct && tab) reinterpret_cast<uint2 *>(S.ct)[tid] = ctv;
+    fill_perm<N>(S);
     if (tid < 16) {
         rgba[tid] = mrgba;
         addt[tid] = madd;
@@ -645,7 +678,7 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
         // the chunk did not change last tick: if nothing in its region can
         // change now it keeps its state, and both buffers already hold it
         // (the test ignores the tick zone: it may only wake too many)
-        const bool pot = __syncthreads_or(tile_unstable<N>(M, L, lut[0], addt, M.temp_every != 0)) != 0;
+        const bool pot = __syncthreads_or(tile_unstable<N>(M, L, S.pair[0], addt, M.temp_every != 0)) != 0;
         if (!pot) {
             if (tid == 0) {
                 w.flags[tick & 1][tile] = 0;
@@ -658,27 +691,28 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
     uint32_t bands = 0;
     if (!zt.dead) {
         const uint64_t seedmix = splitmix64(w.seed);
-        const uint32_t *ct = use_ct ? lut[MAX_IT + 1] : nullptr;
+        const uint32_t *ct = use_ct ? S.ct : nullptr;
         for (int it = 0; it < ci; it++) {
             const uint64_t g = tick * (uint64_t)M.cell_iter + (uint64_t)it;
             const uint64_t key = splitmix64(seedmix ^ g);
             const int ox = kOX[g & 3], oy = kOY[g & 3];
-            // the next iteration's class table, loaded while this phase runs
-            // and put in place when its classification is over
-            const bool next_ct = use_ct && it + 1 < ci;
-            if (next_ct && tab) ctv = reinterpret_cast<const uint2 *>(w.ct + (it + 1) * 512)[tid];
+            // the next iteration's tables, loaded while this phase runs and
+            // put in place when its classification is over
+            const bool next = N == NT && it + 1 < ci;
+            if (next && use_ct) ctv = reinterpret_cast<const uint2 *>(w.ct + (it + 1) * 512)[tid];
             auto refill = [&]() {
-                if (next_ct && tab) reinterpret_cast<uint2 *>(lut[MAX_IT + 1])[tid] = ctv;
+                if (next && it == 1) S.pair[0][tid] = pv[2];
+                if (next && use_ct) reinterpret_cast<uint2 *>(S.ct)[tid] = ctv;
             };
             if (zt.blocks.on)  // on the zone's edge: one form for every setting (the bands may go unused)
-                bands |= run_phase<N, true, RE != 0, true>(M, L, lut[it], it, key, ox, oy, ci - it, gx0, gy0, has_wood,
-                                                        queue, red, lut[MAX_IT], zt.blocks, ct, refill);
+                bands |= run_phase<N, true, RE != 0, true>(M, S, it, key, ox, oy, ci - it, gx0, gy0, has_wood,
+                                                           zt.blocks, ct, refill);
             else if (SK != 0 && skip)
-                bands |= run_phase<N, true, RE != 0, false>(M, L, lut[it], it, key, ox, oy, ci - it, gx0, gy0, has_wood,
-                                                         queue, red, lut[MAX_IT], zt.blocks, ct, refill);
+                bands |= run_phase<N, true, RE != 0, false>(M, S, it, key, ox, oy, ci - it, gx0, gy0, has_wood,
+                                                            zt.blocks, ct, refill);
             else if (SK != 1 && SK != 3)
-                run_phase<N, false, RE != 0, false>(M, L, lut[it], it, key, ox, oy, ci - it, gx0, gy0, has_wood, queue,
-                                                 red, lut[MAX_IT], zt.blocks, ct, refill);
+                run_phase<N, false, RE != 0, false>(M, S, it, key, ox, oy, ci - it, gx0, gy0, has_wood, zt.blocks, ct,
+                                                    refill);
             __syncthreads();
         }
     }
@@ -768,11 +802,11 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
     }
     if (skip) {
         bands = wave_or(bands);
-        if ((tid & 63) == 0) red[tid >> 6] = bands;
+        if ((tid & 63) == 0) S.red[tid >> 6] = bands;
         __syncthreads();
         if (tid == 0) {
             uint32_t all = 0;
-            for (int k = 0; k < N / 64; k++) all |= red[k];
+            for (int k = 0; k < N / 64; k++) all |= S.red[k];
             w.flags[tick & 1][tile] = (zt.dead ? 0u : F_POT) | all;  // a dead chunk cannot change by itself
             atomicAdd(w.processed, 1ull);
         }
@@ -794,21 +828,15 @@ __device__ __forceinline__ int xcd_order(int i, int n, int g) {
     return b * run + (r & 7) * g + (r >> 3);
 }
 
-// Small worlds (at most one chunk per compute unit): the same update with
-// SMALL_NT (1024) threads per chunk.  A small world leaves compute units idle,
-// so a tick lasts one workgroup's latency; four times the waves per chunk cut
-// each wave's share of the phases and let four waves per SIMD hide each
+// Small worlds: the same update with SMALL_NT (1024) threads per chunk (at
+// most one chunk per compute unit) or MEDIUM_NT (512, at most two).  A small
+// world leaves compute units idle, so a tick lasts one workgroup's latency;
+// more waves per chunk cut each wave's share of the phases and hide each
 // other's LDS latency.
-template <int RE, int ZN>
-__global__ __launch_bounds__(SMALL_NT) void k_tick_small(DevWorld w, uint32_t k) {
-    __shared__ __align__(16) uint32_t Lmem[LH * LW + 16];  // the region, then the 16 base colours
-    __shared__ uint32_t lut[MAX_IT + 3][256];  // pair tables, scatter offsets, the phase's class table
-    uint32_t(*L)[LW] = reinterpret_cast<uint32_t(*)[LW]>(Lmem);
-    uint32_t *rgba = Lmem + LH * LW;
-    __shared__ int32_t addt[16];
-    __shared__ uint16_t queue[(SMALL_NT / 64) * qcap<SMALL_NT>()];
-    __shared__ uint32_t red[SMALL_NT / 64];
-    tile_update<0, RE, ZN, SMALL_NT>(w, w.tick + k, blockIdx.x, L, lut, rgba, addt, queue, red);
+template <int RE, int ZN, int N>
+__global__ __launch_bounds__(N) void k_tick_small(DevWorld w, uint32_t k) {
+    __shared__ __align__(16) TileLds<N> S;
+    tile_update<0, RE, ZN, N>(w, w.tick + k, blockIdx.x, S);
 }
 // Smaller worlds still (at most a quarter chunk per compute unit): each
 // chunk as four 32x32 quarters, one workgroup of QUARTER_NT threads each,
@@ -835,9 +863,12 @@ static_assert(TW == 2 * QW && TH == 2 * QH && (QW & 1) == 0, "quarters of whole 
 // region array after the phases (the chunk update's way, which keeps LDS
 // for occupancy).
 template <int RE, int ZN, int N, bool SEP = false>
-__device__ __forceinline__ void quarter_update(const DevWorld &w, uint64_t tick, int tile, int quad,
-                                               uint32_t (*L)[LW], uint32_t (*lut)[256], uint32_t *rgba,
-                                               int32_t *addt, uint16_t *queue, uint32_t *red, uint32_t *colw = nullptr) {
+__device__ __forceinline__ void quarter_update(const DevWorld &w, uint64_t tick, int tile, int quad, TileLds<N> &S,
+                                               uint32_t *colw = nullptr) {
+    uint32_t(*L)[LW] = S.L;
+    uint32_t *const rgba = S.rgba;
+    int32_t *const addt = S.addt;
+    constexpr int PT = TileLds<N>::PT, PV = PT == MAX_IT ? MAX_IT : 1;
     static_assert(N == 256 || N == 512 || N == 1024, "one pair-table entry per thread, write-back strips");
     const int tid = threadIdx.x;
     const MatTab &M = w.mat;
@@ -849,9 +880,9 @@ __device__ __forceinline__ void quarter_update(const DevWorld &w, uint64_t tick,
     const uint64_t *__restrict__ in = w.buf[tick & 1];
     uint64_t *__restrict__ out = w.buf[(tick + 1) & 1];
     const int ci = (int)M.cell_iter;
-    uint32_t pv[MAX_IT];
+    uint16_t pv[PV];
 #pragma unroll
-    for (int k = 0; k < MAX_IT; k++)
+    for (int k = 0; k < PV; k++)
         if (k < ci && tid < 256) pv[k] = w.pair[k][tid];
     uint32_t mrgba = 0;
     int32_t madd = 0;
@@ -901,18 +932,9 @@ __device__ __forceinline__ void quarter_update(const DevWorld &w, uint64_t tick,
         if (RE != 0) wood |= (v[k].x & 0xFFu) == M.wood || (v[k].z & 0xFFu) == M.wood;
     }
 #pragma unroll
-    for (int k = 0; k < MAX_IT; k++)
-        if (k < ci && tid < 256) lut[k][tid] = pv[k];
-    if (tid < 256) {
-        // scatter offsets for mask y = tid: cell k goes to k ^ ((y >> 2k) & 3)
-        uint32_t po = 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const uint32_t d = (uint32_t)k ^ (((uint32_t)tid >> (2 * k)) & 3u);
-            po |= ((d & 1u) + (d >> 1) * (uint32_t)LW) << (8 * k);
-        }
-        lut[MAX_IT][tid] = po;
-    }
+    for (int k = 0; k < PV; k++)
+        if (k < ci && tid < 256) S.pair[k][tid] = pv[k];
+    fill_perm<N>(S);
     if (tid < 16) {
         rgba[tid] = mrgba;
         addt[tid] = madd;
@@ -925,16 +947,19 @@ __device__ __forceinline__ void quarter_update(const DevWorld &w, uint64_t tick,
     for (int it = 0; it < ci && !zt.dead; it++) {
         const uint64_t g = tick * (uint64_t)M.cell_iter + (uint64_t)it;
         const uint64_t key = splitmix64(seedmix ^ g);
+        const bool next = PT != MAX_IT && it + 1 < ci;
+        if (next) pv[0] = w.pair[it + 1][tid];
+        auto refill = [&]() {
+            if (next) S.pair[(it + 1) % PT][tid] = pv[0];
+        };
         // at 1024 threads a thread per block (at most 20 x 20 a phase): no classification
         constexpr bool DIRECT = N >= 1024;
         if (ZN && zt.blocks.on)
-            run_phase<N, false, RE != 0, true, QW, DIRECT>(M, L, lut[it], it, key, kOX[g & 3], kOY[g & 3], ci - it,
-                                                           gx0, gy0, has_wood, queue, red, lut[MAX_IT], zt.blocks,
-                                                           nullptr, [] {}, cx0, cy0);
+            run_phase<N, false, RE != 0, true, QW, DIRECT>(M, S, it, key, kOX[g & 3], kOY[g & 3], ci - it, gx0, gy0,
+                                                           has_wood, zt.blocks, nullptr, refill, cx0, cy0);
         else
-            run_phase<N, false, RE != 0, false, QW, DIRECT>(M, L, lut[it], it, key, kOX[g & 3], kOY[g & 3], ci - it,
-                                                            gx0, gy0, has_wood, queue, red, lut[MAX_IT], zt.blocks,
-                                                            nullptr, [] {}, cx0, cy0);
+            run_phase<N, false, RE != 0, false, QW, DIRECT>(M, S, it, key, kOX[g & 3], kOY[g & 3], ci - it, gx0, gy0,
+                                                            has_wood, zt.blocks, nullptr, refill, cx0, cy0);
         __syncthreads();
     }
 
@@ -998,48 +1023,43 @@ __device__ __forceinline__ void quarter_update(const DevWorld &w, uint64_t tick,
 
 template <int RE, int ZN>
 __global__ __launch_bounds__(QUARTER_NT) void k_tick_quarter(DevWorld w, uint32_t k) {
-    __shared__ __align__(16) uint32_t Lmem[LH * LW + 16];  // the chunk's region layout, then the 16 base colours
-    __shared__ uint32_t lut[MAX_IT + 3][256];  // pair tables, scatter offsets
-    uint32_t(*L)[LW] = reinterpret_cast<uint32_t(*)[LW]>(Lmem);
-    uint32_t *rgba = Lmem + LH * LW;
-    __shared__ int32_t addt[16];
-    __shared__ uint16_t queue[(QUARTER_NT / 64) * qcap<QUARTER_NT>()];
+    __shared__ __align__(16) TileLds<QUARTER_NT> S;
     __shared__ __align__(8) uint32_t colw[QLW * QLH];  // the window's colours
-    quarter_update<RE, ZN, QUARTER_NT, true>(w, w.tick + k, (int)(blockIdx.x >> 2), (int)(blockIdx.x & 3u), L, lut,
-                                             rgba, addt, queue, nullptr, colw);
+    quarter_update<RE, ZN, QUARTER_NT, true>(w, w.tick + k, (int)(blockIdx.x >> 2), (int)(blockIdx.x & 3u), S, colw);
 }
 template __global__ void k_tick_quarter<0, 0>(DevWorld, uint32_t);
 template __global__ void k_tick_quarter<1, 0>(DevWorld, uint32_t);
 template __global__ void k_tick_quarter<0, 1>(DevWorld, uint32_t);
 template __global__ void k_tick_quarter<1, 1>(DevWorld, uint32_t);
 
-template __global__ void k_tick_small<0, 0>(DevWorld, uint32_t);
-template __global__ void k_tick_small<1, 0>(DevWorld, uint32_t);
-template __global__ void k_tick_small<0, 1>(DevWorld, uint32_t);
-template __global__ void k_tick_small<1, 1>(DevWorld, uint32_t);
+template __global__ void k_tick_small<0, 0, SMALL_NT>(DevWorld, uint32_t);
+template __global__ void k_tick_small<0, 0, MEDIUM_NT>(DevWorld, uint32_t);
+template __global__ void k_tick_small<1, 0, SMALL_NT>(DevWorld, uint32_t);
+template __global__ void k_tick_small<1, 0, MEDIUM_NT>(DevWorld, uint32_t);
+template __global__ void k_tick_small<0, 1, SMALL_NT>(DevWorld, uint32_t);
+template __global__ void k_tick_small<0, 1, MEDIUM_NT>(DevWorld, uint32_t);
+template __global__ void k_tick_small<1, 1, SMALL_NT>(DevWorld, uint32_t);
+template __global__ void k_tick_small<1, 1, MEDIUM_NT>(DevWorld, uint32_t);
 
-// Five workgroups per CU (at most 96 VGPRs, 28 KB of LDS each).  One
-// instantiation per (chunk skipping, reactions) setting of the world, so
-// the branches and paths a setting never takes are not compiled in.
+// Worlds of more chunks: 256 threads per chunk.  One instantiation per
+// setting of the world (reactions, tick zone), so the paths a setting never
+// takes are not compiled in.  Six workgroups per CU (at most 80 VGPRs and
+// 26.6 KB of LDS each, TileLds) hide more of each other's latency than five:
+// 16384^2 world 898 -> 845 us a tick, 4096^2 61 -> 59; a world of one round
+// gains nothing from it (2048^2: 25.1 -> 25.4 us).  The zone tests would
+// spill at 80 registers, so with them it is five.
 // Workgroups [0, nfull) update whole chunks in the XCD-aware order; the
 // chunks from nfull on are updated as quarters (four workgroups each, the
 // grid's last), so the launch's last round of workgroups is short: a chunk
 // left over from the last full round of whole chunks would hold one
 // compute unit for a whole chunk's latency while the others idle.
-template <int SK, int RE, int ZN>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_tick_world(DevWorld w, uint32_t k,
-                                                                                            int nfull) {
-    __shared__ __align__(16) uint32_t Lmem[LH * LW + 16];  // the region, then the 16 base colours
-    __shared__ uint32_t lut[MAX_IT + 3][256];  // pair tables, scatter offsets, the phase's class table
-    uint32_t(*L)[LW] = reinterpret_cast<uint32_t(*)[LW]>(Lmem);
-    uint32_t *rgba = Lmem + LH * LW;
-    __shared__ int32_t addt[16];
-    __shared__ uint16_t queue[(NT / 64) * qcap<NT>()];
-    __shared__ __align__(16) uint32_t red[NT / 64];
+template <int RE, int ZN>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WGS_PER_CU - ZN)))
+void k_tick_world(DevWorld w, uint32_t k, int nfull) {
+    __shared__ __align__(16) TileLds<NT> S;
     const int i = (int)blockIdx.x;
     if (i < nfull) {
-        tile_update<SK, RE, ZN>(w, w.tick + k, xcd_order(i, nfull, (w.tiles_x & 7) ? 8 : w.tiles_x >> 3), L, lut,
-                                rgba, addt, queue, red);
+        tile_update<0, RE, ZN>(w, w.tick + k, xcd_order(i, nfull, (w.tiles_x & 7) ? 8 : w.tiles_x >> 3), S);
     } else {
         // the four quarters of a chunk on one XCD (workgroup i runs on XCD
         // i % 8, and nfull is a multiple of 8), so they share their halo
@@ -1049,13 +1069,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_
         const int q = i - nfull, nq = (int)gridDim.x - nfull, full = nq & ~31;
         const int c = q < full ? (q & 7) + ((q >> 5) << 3) : q >> 2;
         const int quad = q < full ? (q >> 3) & 3 : q & 3;
-        quarter_update<RE, ZN, NT>(w, w.tick + k, nfull + c, quad, L, lut, rgba, addt, queue, red);
+        quarter_update<RE, ZN, NT>(w, w.tick + k, nfull + c, quad, S);
     }
 }
-template __global__ void k_tick_world<0, 0, 0>(DevWorld, uint32_t, int);
-template __global__ void k_tick_world<0, 1, 0>(DevWorld, uint32_t, int);
-template __global__ void k_tick_world<0, 0, 1>(DevWorld, uint32_t, int);
-template __global__ void k_tick_world<0, 1, 1>(DevWorld, uint32_t, int);
+template __global__ void k_tick_world<0, 0>(DevWorld, uint32_t, int);
+template __global__ void k_tick_world<1, 0>(DevWorld, uint32_t, int);
+template __global__ void k_tick_world<0, 1>(DevWorld, uint32_t, int);
+template __global__ void k_tick_world<1, 1>(DevWorld, uint32_t, int);
 
 // The wake test of one chunk by one thread, which writes the flags of a chunk
 // that sleeps.
@@ -1106,24 +1126,21 @@ __global__ __launch_bounds__(256) void k_wake(DevWorld w, uint32_t k) {
     list_awake(awake, (uint32_t)tile, w.awake, &w.awake_n[tick & 1]);
 }
 
-// Skip-path tick over the awake list: workgroup i updates the i-th listed
-// chunk, and workgroups past the list's end exit at once.  The listed
-// chunks take the first workgroups, so they start back to back and no
-// sleeping chunk holds a workgroup slot while they run.
+// Skip-path tick over the awake list (five workgroups per CU: its band
+// tracking needs more registers, and six spilled some, 50.4 -> 51.5 us on the
+// 4096^2 reacting world): workgroup i updates the i-th listed chunk, and
+// workgroups past the list's end exit at once.  The listed chunks take the
+// first workgroups, so they start back to back and no sleeping chunk holds a
+// workgroup slot while they run.
 template <int RE, int ZN>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(5))) void k_tick_list(DevWorld w, uint32_t k) {
-    __shared__ __align__(16) uint32_t Lmem[LH * LW + 16];  // the region, then the 16 base colours
-    __shared__ uint32_t lut[MAX_IT + 3][256];  // pair tables, scatter offsets, the phase's class table
-    uint32_t(*L)[LW] = reinterpret_cast<uint32_t(*)[LW]>(Lmem);
-    uint32_t *rgba = Lmem + LH * LW;
-    __shared__ int32_t addt[16];
-    __shared__ uint16_t queue[(NT / 64) * qcap<NT>()];
-    __shared__ __align__(16) uint32_t red[NT / 64];
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WGS_PER_CU - 1)))
+void k_tick_list(DevWorld w, uint32_t k) {
+    __shared__ __align__(16) TileLds<NT> S;
     const uint64_t tick = w.tick + k;
     const int n = (int)w.awake_n[tick & 1];
     if ((int)blockIdx.x >= n) return;
     // the list runs in row-major order within each reserving workgroup of k_wake
-    tile_update<3, RE, ZN>(w, tick, (int)w.awake[xcd_order(blockIdx.x, n, 8)], L, lut, rgba, addt, queue, red);
+    tile_update<3, RE, ZN>(w, tick, (int)w.awake[xcd_order(blockIdx.x, n, 8)], S);
 }
 template __global__ void k_tick_list<0, 0>(DevWorld, uint32_t);
 template __global__ void k_tick_list<1, 0>(DevWorld, uint32_t);
@@ -1146,18 +1163,14 @@ __device__ __forceinline__ int world_of(const uint32_t *__restrict__ tile_start,
 // instantiation per setting that all worlds of the batch share, as for one
 // world; SK == 2, RE == 2 (read from each world) with the zone tests serves
 // the batches whose worlds differ or have a zone.  WG: workgroups per CU
-// (the register budget), one of the autotuner's choices.
+// (the register budget), one of the autotuner's choices: four, or as many as
+// the form can have without spilling (six, with skipping five).
 template <int SK, int RE, int ZN, int WG>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WG))) void k_tick_batch(
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WG - (SK != 0 && WG == WGS_PER_CU ? 1 : 0))))
+void k_tick_batch(
     const DevWorld *__restrict__ worlds, const uint32_t *__restrict__ tile_start, int nworlds, uint32_t k,
     const uint32_t *__restrict__ awake, const uint32_t *__restrict__ awake_n) {
-    __shared__ __align__(16) uint32_t Lmem[LH * LW + 16];  // the region, then the 16 base colours
-    __shared__ uint32_t lut[MAX_IT + 3][256];  // pair tables, scatter offsets, the phase's class table
-    uint32_t(*L)[LW] = reinterpret_cast<uint32_t(*)[LW]>(Lmem);
-    uint32_t *rgba = Lmem + LH * LW;
-    __shared__ int32_t addt[16];
-    __shared__ uint16_t queue[(NT / 64) * qcap<NT>()];
-    __shared__ __align__(16) uint32_t red[NT / 64];
+    __shared__ __align__(16) TileLds<NT> S;
     uint32_t gt = blockIdx.x;
     if (SK == 3) {
         const int n = (int)awake_n[k & 1];
@@ -1166,10 +1179,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WG))) void k
     }
     const int lo = world_of(tile_start, nworlds, gt);
     const DevWorld &w = worlds[lo];
-    tile_update<SK, RE, ZN>(w, w.tick + k, (int)(gt - tile_start[lo]), L, lut, rgba, addt, queue, red);
+    tile_update<SK, RE, ZN>(w, w.tick + k, (int)(gt - tile_start[lo]), S);
 }
 #define FSG_BATCH(SK, RE, ZN)                                                                                      \
-    template __global__ void k_tick_batch<SK, RE, ZN, 5>(const DevWorld *, const uint32_t *, int, uint32_t,        \
+    template __global__ void k_tick_batch<SK, RE, ZN, 6>(const DevWorld *, const uint32_t *, int, uint32_t,        \
                                                          const uint32_t *, const uint32_t *);                      \
     template __global__ void k_tick_batch<SK, RE, ZN, 4>(const DevWorld *, const uint32_t *, int, uint32_t,        \
                                                          const uint32_t *, const uint32_t *)

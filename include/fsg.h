@@ -524,7 +524,7 @@ int fsg_perworld_step_timed(fsg_ctx *ctx, fsg_world *const *worlds, int n, int t
 typedef struct fsg_tuning {
     int32_t graph_ticks; /* ticks per captured HIP graph block: 1 (no graph), 4, 8, 16 or 32 */
     int32_t chunk_skip;  /* dirty-chunk skipping in batches: -1 each world's own setting, 0 off, 1 on */
-    int32_t occupancy;   /* tick-kernel register budget: 4 or 5 workgroups per CU */
+    int32_t occupancy;   /* tick-kernel register budget: 4 workgroups per CU, or 5: the most it can have (5 or 6) */
     int32_t reserved;    /* 0 */
 } fsg_tuning;
 

@@ -26,7 +26,7 @@ def dense(kind, W, H, seed):
 
 @pytest.mark.parametrize("kind", ["rows", (AIR, SAND), (AIR, WATER), (AIR, STEAM), (OIL, WATER, LAVA), (SAND, STONE),
                                   (AIR, SAND, WATER, STEAM, LAVA, WOOD)])
-@pytest.mark.parametrize("W,H", [(64, 64), (1152, 1024), (2100, 130)])  # each of the kernels by world size
+@pytest.mark.parametrize("W,H", [(64, 64), (2100, 130), (1152, 1024), (2100, 1100)])  # each kernel by world size
 @pytest.mark.parametrize("skip", [0, 1])
 def test_dense_phases(ctx, orc, kind, W, H, skip):
     print(f"dense {kind} {W}x{H} skip={skip}", flush=True)
