@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <vector>
@@ -60,6 +61,17 @@ struct fsg_ctx {
     int batch_form = 0, graph_form = 0;
     uint32_t *d_awake = nullptr, *d_awake_n = nullptr;
     size_t awake_cap = 0;
+    // pinned staging of small copies (copy_in / copy_out), allocated at first
+    // use: IN_SLOTS slots for uploads in flight, each reused only after the
+    // event recorded behind its last upload, and one area for downloads
+    static constexpr size_t STAGE = (size_t)1 << 20;
+    static constexpr int IN_SLOTS = 4;
+    std::mutex stage_in_mu, stage_out_mu;
+    char *h_in = nullptr, *h_out = nullptr;
+    hipEvent_t in_ev[IN_SLOTS] = {};
+    bool in_pending[IN_SLOTS] = {};
+    int in_slot = 0;
+    size_t in_used = 0;
     // freed device blocks by size class (dev_alloc / dev_free); the cap is at
     // least 16 GiB and a quarter of the device's memory
     std::multimap<size_t, void *> cache;
@@ -158,6 +170,20 @@ int dev_alloc(fsg_ctx *c, void **p, size_t bytes);
 void dev_free(void *p);
 void trim_cache(fsg_ctx *c, size_t keep);  // hipFree cached blocks down to `keep` bytes
 unsigned grid_for(size_t n, unsigned block);
+// Host -> device copy in stream order; the source may change when it returns
+// if bytes <= fsg_ctx::STAGE, else only once the stream has been synchronised.
+int copy_in(fsg_ctx *c, void *dst, const void *src, size_t bytes);
+// Device -> host copies, behind everything on the stream; waits for them.
+struct CopyOut {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+int copy_out(fsg_ctx *c, std::initializer_list<CopyOut> parts);
+// Rectangle of a device array of T (4 or 8 bytes) with rows of `pitch`
+// elements into rows of rw; waits.
+template <typename T>
+int copy_rect_out(fsg_ctx *c, T *dst, const T *src, size_t pitch, int rw, int rh);
 // Uploads the world table of a batch; *graph_ok tells whether the cached
 // graph matches this world set.
 int batch_prepare(fsg_ctx *c, fsg_world *const *ws, int n, bool *graph_ok);

@@ -213,11 +213,10 @@ extern "C" int fsg_world_physics_check(fsg_world *w, fsg_island *seeds, int n, s
     Winner *d_win = reinterpret_cast<Winner *>(scratch + b_xy + b_lists + b_out);
     std::vector<SeedOut> res((size_t)n);
     uint64_t *cur = w->d.buf[w->d.tick & 1];
-    HIPCHK(hipMemcpyAsync(d_xy, xy.data(), xy.size() * 4, hipMemcpyHostToDevice, c->stream));
+    if (int rc = fsg_impl::copy_in(c, d_xy, xy.data(), xy.size() * 4)) return rc;
     k_island_search<<<n, IT, 0, c->stream>>>(cur, W, H, solid, d_xy, d_lists, d_out);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(res.data(), d_out, b_out, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if (int rc = fsg_impl::copy_out(c, {{res.data(), d_out, b_out}})) return rc;
     // keep the first seed of each island, in seed order
     std::vector<Winner> win;
     std::unordered_set<uint32_t> gone;
@@ -250,7 +249,7 @@ extern "C" int fsg_world_physics_check(fsg_world *w, fsg_island *seeds, int n, s
             w->d_isl_pix = static_cast<uint64_t *>(pb);
         }
         const uint64_t air = (uint64_t)w->cfg.mat_air;  // Tiles_NOTHING: colour 0, temperature 0
-        HIPCHK(hipMemcpyAsync(d_win, win.data(), win.size() * sizeof(Winner), hipMemcpyHostToDevice, c->stream));
+        if (int rc = fsg_impl::copy_in(c, d_win, win.data(), win.size() * sizeof(Winner))) return rc;
         if (needed) {
             k_fill_u64<<<fsg_impl::grid_for(needed, 256), 256, 0, c->stream>>>(w->d_isl_pix, needed, air);
             HIPCHK(hipGetLastError());
@@ -284,7 +283,5 @@ extern "C" int fsg_world_island_pixels(fsg_world *w, fsg_cell *out, size_t cap) 
     if (!w->isl_pix_used) return FSG_OK;
     fsg_ctx *c = w->ctx;
     HIPCHK(hipSetDevice(c->device));
-    HIPCHK(hipMemcpyAsync(out, w->d_isl_pix, w->isl_pix_used * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return FSG_OK;
+    return fsg_impl::copy_out(c, {{out, w->d_isl_pix, w->isl_pix_used * 8}});
 }

@@ -1545,4 +1545,13 @@ __global__ __launch_bounds__(256) void k_stamp_compact(StampArgs a) {
 
 __global__ void k_zero_u32(uint32_t *p) { p[threadIdx.x] = 0; }
 
+template <typename T>
+__global__ void k_gather_rect(const T *__restrict__ src, size_t pitch, int rw, int rh, T *__restrict__ dst) {
+    const int x = blockIdx.x * 256 + threadIdx.x;
+    if (x >= rw) return;
+    for (int y = blockIdx.y; y < rh; y += gridDim.y) dst[(size_t)y * rw + x] = src[(size_t)y * pitch + x];
+}
+template __global__ void k_gather_rect<uint64_t>(const uint64_t *, size_t, int, int, uint64_t *);
+template __global__ void k_gather_rect<uint32_t>(const uint32_t *, size_t, int, int, uint32_t *);
+
 } // namespace fsg

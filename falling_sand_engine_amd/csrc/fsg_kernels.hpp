@@ -65,5 +65,8 @@ __global__ void k_stamp_step_list(StampArgs a, int op, int d);
 constexpr int STAMP_CPT = 8;  // pixels per thread of k_stamp_compact (grid x: npix / (256 * STAMP_CPT))
 __global__ void k_stamp_compact(StampArgs a);
 __global__ void k_zero_u32(uint32_t *p);
+// Rows of rw elements out of rows of `pitch`, back to back.
+template <typename T>
+__global__ void k_gather_rect(const T *__restrict__ src, size_t pitch, int rw, int rh, T *__restrict__ dst);
 
 } // namespace fsg

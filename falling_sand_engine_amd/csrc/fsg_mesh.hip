@@ -783,8 +783,7 @@ int run_mesh(fsg_world *w, const MeshSrc &src, std::vector<MeshRegionDev> &regs,
         o.regcnt = o.counters + 4;
         o.regvert = o.regcnt + nout;
         uint32_t *regbase = o.regvert + nout, *regvbase = regbase + nout;
-        HIPCHK(hipMemcpyAsync(w->d_mesh_regs, regs.data(), (size_t)n * sizeof(MeshRegionDev), hipMemcpyHostToDevice,
-                              c->stream));
+        if (int rc = fsg_impl::copy_in(c, w->d_mesh_regs, regs.data(), (size_t)n * sizeof(MeshRegionDev))) return rc;
         // pools sized from the last call, grown and the launch repeated on overflow
         uint32_t loop_cap = std::max<uint32_t>(w->mesh_loop_hint, 4096u);
         uint32_t vert_cap = std::max<uint32_t>(w->mesh_vert_hint, 65536u);
@@ -818,8 +817,7 @@ int run_mesh(fsg_world *w, const MeshSrc &src, std::vector<MeshRegionDev> &regs,
             k_mesh_emit<<<std::min<uint32_t>((loop_cap + 31) / 32, 2048u), 256, 0, c->stream>>>(o, regbase, regvbase,
                                                                                                oloops, overts);
             HIPCHK(hipGetLastError());
-            HIPCHK(hipMemcpyAsync(h.data(), o.counters, b_out, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(hipStreamSynchronize(c->stream));
+            if (int rc = fsg_impl::copy_out(c, {{h.data(), o.counters, b_out}})) return rc;
             const uint32_t *cnt = h.data(), *rc = cnt + 4;
             if (cnt[3]) return FSG_ERR_DEVICE;  // a walk that did not close: not a perimeter of a finite mask
             if (cnt[2]) {
@@ -916,8 +914,6 @@ extern "C" int fsg_world_mesh_download(fsg_world *w, fsg_mesh_loop *loops, uint3
     if ((nl && (!loops || loop_cap < nl)) || (nv && (!verts || vert_cap < nv))) return FSG_ERR_INVALID;
     fsg_ctx *c = w->ctx;
     HIPCHK(hipSetDevice(c->device));
-    if (nl) HIPCHK(hipMemcpyAsync(loops, w->d_mesh_loops, nl * sizeof(fsg_mesh_loop), hipMemcpyDeviceToHost, c->stream));
-    if (nv) HIPCHK(hipMemcpyAsync(verts, w->d_mesh_verts, nv * 2 * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return FSG_OK;
+    return fsg_impl::copy_out(c, {{loops, w->d_mesh_loops, nl * sizeof(fsg_mesh_loop)},
+                                  {verts, w->d_mesh_verts, nv * 2 * sizeof(float)}});
 }

@@ -646,7 +646,7 @@ extern "C" int fsg_world_pack(fsg_world *w, int32_t x0, int32_t y0, int32_t ncx,
     int8_t *d_phase = reinterpret_cast<int8_t *>(d_off + n + 1);
     w->pack_phase.assign(n, 0);
     if (phase) std::copy(phase, phase + n, w->pack_phase.begin());
-    HIPCHK(hipMemcpyAsync(d_phase, w->pack_phase.data(), n, hipMemcpyHostToDevice, c->stream));
+    if (int rc = fsg_impl::copy_in(c, d_phase, w->pack_phase.data(), n)) return rc;
     PackSrc s{};
     s.cells = w->d.buf[w->d.tick & 1];
     s.W = w->d.W;
@@ -673,9 +673,7 @@ extern "C" int fsg_world_pack(fsg_world *w, int32_t x0, int32_t y0, int32_t ncx,
     HIPCHK(hipGetLastError());
     w->pack_sizes.resize(2 * n);
     int64_t total = 0;
-    HIPCHK(hipMemcpyAsync(w->pack_sizes.data(), d_sizes, 2 * n * 4, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(&total, d_off + n, 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if (int rc = fsg_impl::copy_out(c, {{w->pack_sizes.data(), d_sizes, 2 * n * 4}, {&total, d_off + n, 8}})) return rc;
     if (total < 0) {
         w->pack_n = 0;
         return FSG_ERR_DEVICE;
@@ -692,9 +690,7 @@ extern "C" int fsg_world_pack_download(fsg_world *w, void *out, size_t cap) {
     if (cap < w->pack_total) return FSG_ERR_INVALID;
     fsg_ctx *c = w->ctx;
     HIPCHK(hipSetDevice(c->device));
-    HIPCHK(hipMemcpyAsync(out, w->d_pack_img, w->pack_total, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return FSG_OK;
+    return fsg_impl::copy_out(c, {{out, w->d_pack_img, w->pack_total}});
 }
 
 extern "C" int fsg_world_unpack(fsg_world *w, int32_t x0, int32_t y0, int32_t ncx, int32_t ncy, const void *images,
@@ -732,7 +728,7 @@ extern "C" int fsg_world_unpack(fsg_world *w, int32_t x0, int32_t y0, int32_t nc
             in_total += len;
         }
         if (grow(c, &w->d_pack_in, &w->pack_in_cap, std::max<size_t>(in_total, 1))) return FSG_ERR_NOMEM;
-        HIPCHK(hipMemcpyAsync(w->d_pack_in, images, in_total, hipMemcpyHostToDevice, c->stream));
+        if (int rc = fsg_impl::copy_in(c, w->d_pack_in, images, in_total)) return rc;
         src = static_cast<const uint8_t *>(w->d_pack_in);
     } else {
         int64_t o = 0;
@@ -766,16 +762,16 @@ extern "C" int fsg_world_unpack(fsg_world *w, int32_t x0, int32_t y0, int32_t nc
     d.moved = (map.flags & FSG_PACK_NO_MOVED) ? 0u : 1u;
     d.n = (int)n;
     std::memcpy(d.from_file, map.from_file, sizeof(d.from_file));
-    HIPCHK(hipMemcpyAsync(d_desc, desc.data(), 2 * n * sizeof(DecDesc), hipMemcpyHostToDevice, c->stream));
+    if (int rc = fsg_impl::copy_in(c, d_desc, desc.data(), 2 * n * sizeof(DecDesc))) return rc;
     if (b_l2 + b_bg) HIPCHK(hipMemsetAsync(dec + b_desc + b_st, 0, b_l2 + b_bg, c->stream));  // failed chunks: 0
     uint8_t *raw = static_cast<uint8_t *>(w->d_pack_raw);
     k_pack_decode<<<(unsigned)((2 * n + DW - 1) / DW), 64 * DW, 0, c->stream>>>(src, d_desc, raw, d_bst, (int)(2 * n));
     k_pack_cells<<<(unsigned)n, 256, 0, c->stream>>>(raw, d_bst, d, d_cst);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(status, d_cst, n * 4, hipMemcpyDeviceToHost, c->stream));
-    if (layer2) HIPCHK(hipMemcpyAsync(layer2, d.l2, b_l2, hipMemcpyDeviceToHost, c->stream));
-    if (background) HIPCHK(hipMemcpyAsync(background, d.bg, b_bg, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if (int rc = fsg_impl::copy_out(c, {{status, d_cst, n * 4},
+                                        {layer2, d.l2, layer2 ? b_l2 : 0},
+                                        {background, d.bg, background ? b_bg : 0}}))
+        return rc;
     if (phase) std::copy(ph.begin(), ph.end(), phase);
     // new cells, as after fsg_world_upload
     w->d.force_tick = w->d.tick;

@@ -635,8 +635,9 @@ extern "C" int fsg_world_particles_add(fsg_world *w, const fsg_particle *p, size
     fsg_ctx *c = w->ctx;
     HIPCHK(hipSetDevice(c->device));
     if (int rc = grow_lists(w, w->npart + n)) return rc;
-    HIPCHK(hipMemcpyAsync(w->d_part + w->npart, p, n * sizeof(fsg_particle), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    const size_t bytes = n * sizeof(fsg_particle);
+    if (int rc = fsg_impl::copy_in(c, w->d_part + w->npart, p, bytes)) return rc;
+    if (bytes > fsg_ctx::STAGE) HIPCHK(hipStreamSynchronize(c->stream));
     w->npart += n;
     return FSG_OK;
 }
@@ -682,8 +683,7 @@ extern "C" int fsg_world_particles_tick(fsg_world *w, size_t *alive, size_t *lan
             k_ph_round<<<(n - final_n + 255) / 256, 256, 0, st>>>(ra);
             HIPCHK(hipGetLastError());
             uint32_t h[3];
-            HIPCHK(hipMemcpyAsync(h, b.cnt, 12, hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
+            if (int rc = fsg_impl::copy_out(c, {{h, b.cnt, 12}})) return rc;
             if (h[0] == 0) {  // no landing changed: every outcome is the sequential one
                 final_n = n;
                 break;
@@ -727,8 +727,7 @@ extern "C" int fsg_world_particles_tick(fsg_world *w, size_t *alive, size_t *lan
         k_pc_scatter<<<nb, 1024, 0, st>>>(w->d_part, w->d_part_alive, n, b.blk, w->d_part2);
         HIPCHK(hipGetLastError());
         unsigned long long h[2] = {0, 0};
-        HIPCHK(hipMemcpyAsync(h, w->d_part_cnt, 16, hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
+        if (int rc = fsg_impl::copy_out(c, {{h, w->d_part_cnt, 16}})) return rc;
         nl = h[0];
         std::swap(w->d_part, w->d_part2);  // the survivors, in order, are the list
         w->npart = (size_t)(uint32_t)h[1];
@@ -743,10 +742,8 @@ extern "C" int fsg_world_particles_get(fsg_world *w, fsg_particle *out, size_t c
     fsg_ctx *c = w->ctx;
     HIPCHK(hipSetDevice(c->device));
     const size_t k = std::min(cap, w->npart);
-    if (k) {
-        HIPCHK(hipMemcpyAsync(out, w->d_part, k * sizeof(fsg_particle), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-    }
+    if (k)
+        if (int rc = fsg_impl::copy_out(c, {{out, w->d_part, k * sizeof(fsg_particle)}})) return rc;
     if (n) *n = w->npart;
     return FSG_OK;
 }

@@ -220,8 +220,7 @@ extern "C" int fsg_world_render(fsg_world *w, const fsg_render_params *p, fsg_re
     HIPCHK(hipGetLastError());
     if (stats) {
         unsigned long long rep[NREP * REP_STRIDE], h[17] = {};
-        HIPCHK(hipMemcpyAsync(rep, tally, tally_bytes, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
+        if (int rc = fsg_impl::copy_out(c, {{rep, tally, tally_bytes}})) return rc;
         for (int r = 0; r < NREP; r++)
             for (int k = 0; k < 17; k++) h[k] += rep[r * REP_STRIDE + k];
         for (int m = 0; m < 16; m++) {
@@ -249,8 +248,5 @@ extern "C" int fsg_world_layer_download(fsg_world *w, uint32_t layer, int x0, in
     fsg_ctx *c = w->ctx;
     HIPCHK(hipSetDevice(c->device));
     const uint32_t *src = w->d_layer[li] + (size_t)y0 * w->d.W + x0;
-    HIPCHK(hipMemcpy2DAsync(out, (size_t)rw * 4, src, (size_t)w->d.W * 4, (size_t)rw * 4, (size_t)rh,
-                            hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return FSG_OK;
+    return fsg_impl::copy_rect_out(c, out, src, (size_t)w->d.W, rw, rh);
 }
