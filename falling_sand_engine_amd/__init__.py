@@ -206,6 +206,8 @@ class Context:
         self.close()
 
 
+_EDIT = np.dtype([("x", np.int32), ("y", np.int32), ("cell", np.uint64)])  # a CellEdit
+
 MIRROR_PAGE = 64  # side of the getTile mirror's pages
 
 
@@ -377,8 +379,8 @@ class World:
         check(lib().fsg_world_stamp_bodies(self.handle, barr, nb, px.ctypes.data, px.size, C.byref(res)),
               "fsg_world_stamp_bodies")
         n = min(res.displaced, displaced_cap)
-        displaced = [(disp[i].x, disp[i].y,
-                      make_cell(disp[i].cell.mat, disp[i].cell.temp, disp[i].cell.rgba)) for i in range(n)]
+        d = np.frombuffer(disp, _EDIT, n)
+        displaced = list(zip(d["x"].tolist(), d["y"].tolist(), d["cell"].tolist()))
         return {"placed": res.placed, "unplaced": res.unplaced, "displaced": res.displaced,
                 "displaced_cells": displaced, "hits_sand": list(hs)[:nb], "hits_soup": list(hw)[:nb]}
 

@@ -153,7 +153,10 @@ struct fsg_world {
     std::vector<fsg_body> bodies;
     fsg::StampWorld *d_sw = nullptr;  // one-entry stamp table on the device
     fsg::StampWorld sw_host{};
-    std::vector<uint32_t> pix_body_host;
+    std::vector<uint32_t> body_order;  // bodies by their first pixel
+    uint32_t *d_order = nullptr;
+    void *d_sres = nullptr;            // the stamp's result (fsg::StampRes)
+    size_t sres_cap = 0;
 };
 
 
@@ -194,13 +197,15 @@ fsg::StampWorld stamp_world_of(fsg_world *w, uint32_t pix_start);
 // Stamp (or unstamp) claim rounds over a device table of n worlds.
 // max_npix: the largest pixel count of one world (the launch's x extent).
 // save: the claim slots of the spare buffer are restored afterwards.
+// res: the stamp's result (one world; no counts: not wanted).
 int stamp_rounds(fsg_ctx *c, const fsg::StampWorld *d_table, int n, uint32_t total, uint32_t max_npix,
-                 const MatTab &M, bool unstamp, bool save);
+                 const MatTab &M, bool unstamp, bool save, const fsg::StampRes &res = fsg::StampRes{});
 // Enqueues w's census (counts [0,16), checksum [16], processed chunks [17])
 // into host[18], valid after the context's stream is synchronised.
 int stats_enqueue(fsg_world *w, unsigned long long *host);
 // Uploads pixels/bodies of a world for stamping (validates them).
-int set_bodies(fsg_world *w, const fsg_body *bodies, int nb, const fsg_cell *pixels, size_t npix);
+int set_bodies(fsg_world *w, const fsg_body *bodies, int nb, const fsg_cell *pixels, size_t npix,
+               uint32_t *zero = nullptr, uint32_t nzero = 0);
 // Looks up the device address of fsg_world_set_cells_noalloc's array on the
 // current device (once per device).
 int noalloc_setup(int device);

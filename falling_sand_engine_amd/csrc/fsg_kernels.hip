@@ -1372,8 +1372,9 @@ __device__ __forceinline__ void mark_tiles_wave(uint32_t *flags, bool on, uint32
 // the atomicMin to the earlier round's claim still in the slot -- so the
 // earliest round and then the lowest pixel win, as a round-by-round pass
 // over the pixels gives.  With save the slots' contents (the state before
-// the last tick) are first copied out, and k_claims_clear clears them in a
-// launch of its own, after every copy; k_claims_restore puts them back.
+// the last tick) are taken out by the exchange that clears them: of the
+// pixels sharing a slot one gets its cell and the others ~0, which no cell
+// is; k_claims_restore puts the cells back.
 __device__ __forceinline__ void slot_at(const StampWorld &W, uint64_t t, int d, bool live, bool &on, int &wx,
                                         int &wy) {
     wx = (int)(uint32_t)t + kDX[d];
@@ -1384,6 +1385,7 @@ __device__ __forceinline__ void slot_at(const StampWorld &W, uint64_t t, int d, 
 __global__ void k_claims_init(StampArgs a, int save) {
     const StampWorld &W = a.worlds[blockIdx.y];
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p == 0 && blockIdx.y == 0) *a.nopen = 0;
     const bool in = p < W.npix;
     uint64_t t = NOT_LIVE;
     if (in) {
@@ -1396,44 +1398,113 @@ __global__ void k_claims_init(StampArgs a, int save) {
         bool on;
         int wx, wy;
         slot_at(W, t, d, live, on, wx, wy);
-        if (save) {
-            if (on) W.save[5 * (size_t)p + d] = W.claims[(size_t)wy * W.W + wx];
-            continue;
+        uint64_t *slot = &W.claims[(size_t)wy * W.W + wx];
+        if (on && save) {
+            W.save[5 * (size_t)p + d] = atomicExch(reinterpret_cast<unsigned long long *>(slot), ~0ull);
+        } else if (on) {
+            *slot = ~0ull;
         }
-        if (on) W.claims[(size_t)wy * W.W + wx] = ~0ull;
         if (W.flags) mark_tiles_wave(W.flags, on, on ? (uint32_t)((wy / TH) * W.tiles_x + wx / TW) : 0u);
     }
 }
 
-__global__ void k_claims_clear(StampArgs a) {
+// The body of pixel p: the last one in order whose first pixel is at or
+// before p, if p is one of its pixels (bodies do not overlap).
+__global__ __launch_bounds__(256) void k_pix_body(const fsg_body *bodies, const uint32_t *order, uint32_t nb,
+                                                  uint32_t npix, uint32_t *pix_body, uint32_t *zero, uint32_t nzero) {
+    const uint32_t p = blockIdx.x * 256 + threadIdx.x;
+    if (p < nzero) zero[p] = 0;
+    if (p >= npix) return;
+    uint32_t b = 0xFFFFFFFFu;
+    if (nb && bodies[order[0]].pixel_offset <= p) {
+        uint32_t lo = 0, hi = nb - 1;
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi + 1) >> 1;
+            if (bodies[order[mid]].pixel_offset <= p) lo = mid;
+            else hi = mid - 1;
+        }
+        const fsg_body &B = bodies[order[lo]];
+        if (p - B.pixel_offset < (uint32_t)B.mat_w * (uint32_t)B.mat_h) b = order[lo];
+    }
+    pix_body[p] = b;
+}
+
+// The saved slots put back and, with r.count, the stamp's result: the pixels
+// placed and unplaced, the displaced ones per workgroup (k_displaced lists
+// them) and per body (one atomic per body and wave).
+__global__ __launch_bounds__(256) void k_claims_restore(StampArgs a, StampRes r) {
+    __shared__ uint32_t cnt[3];
     const StampWorld &W = a.worlds[blockIdx.y];
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t p = blockIdx.x * 256 + threadIdx.x;
     const bool in = p < W.npix;
-    const uint64_t t = in ? W.tgt[p] : NOT_LIVE;
-    const bool live = in && (uint32_t)t != NOT_LIVE;
-    for (int d = 0; d < 5; d++) {
-        bool on;
-        int wx, wy;
-        slot_at(W, t, d, live, on, wx, wy);
-        if (on) W.claims[(size_t)wy * W.W + wx] = ~0ull;
-        if (W.flags) mark_tiles_wave(W.flags, on, on ? (uint32_t)((wy / TH) * W.tiles_x + wx / TW) : 0u);
+    if (in && W.save) {
+        const uint64_t t = W.tgt[p];
+        const bool live = (uint32_t)t != NOT_LIVE;
+        for (int d = 0; d < 5; d++) {
+            bool on;
+            int wx, wy;
+            slot_at(W, t, d, live, on, wx, wy);
+            const uint64_t v = on ? W.save[5 * (size_t)p + d] : ~0ull;
+            if (v != ~0ull) W.claims[(size_t)wy * W.W + wx] = v;
+        }
     }
+    if (!r.count) return;
+    if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t b = in ? W.pix_body[p] : 0xFFFFFFFFu;
+    const bool live = b != 0xFFFFFFFFu && W.bodies[b].enabled && !bit(a.mat.air, cid(W.pixels[p]));
+    const uint32_t st = live ? W.state[p] : 0u;
+    const uint64_t mp = __ballot(live && st), mu = __ballot(live && !st), md = __ballot(st >= 2);
+    const int lane = threadIdx.x & 63;
+    if (lane == 0) {
+        if (mp) atomicAdd(&cnt[0], (uint32_t)__popcll(mp));
+        if (mu) atomicAdd(&cnt[1], (uint32_t)__popcll(mu));
+        if (md) atomicAdd(&cnt[2], (uint32_t)__popcll(md));
+    }
+    for (uint64_t m = md; m;) {  // a wave's pixels are one or two bodies'
+        const int leader = __builtin_ctzll(m);
+        const uint32_t b0 = (uint32_t)__shfl((int)b, leader, 64);
+        const uint64_t same = __ballot(b == b0) & md, sand = __ballot(st == 2) & same;
+        if (lane == leader) {
+            if (sand) atomicAdd(&r.hits[b0], (uint32_t)__popcll(sand));
+            if (same != sand) atomicAdd(&r.hits[r.nb + b0], (uint32_t)__popcll(same & ~sand));
+        }
+        m &= ~same;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3 && cnt[threadIdx.x]) atomicAdd(&r.count[threadIdx.x], cnt[threadIdx.x]);
+    if (threadIdx.x == 0) r.block[blockIdx.x] = cnt[2];
 }
 
-// Every pixel that saved a slot writes the saved value back; pixels sharing
-// a slot saved the same value, so the writes agree.
-__global__ void k_claims_restore(StampArgs a) {
-    const StampWorld &W = a.worlds[blockIdx.y];
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= W.npix || !W.save) return;
-    const uint64_t t = W.tgt[p];
-    const bool live = (uint32_t)t != NOT_LIVE;
-    for (int d = 0; d < 5; d++) {
-        bool on;
-        int wx, wy;
-        slot_at(W, t, d, live, on, wx, wy);
-        if (on) W.claims[(size_t)wy * W.W + wx] = W.save[5 * (size_t)p + d];
+// The displaced cells in pixel order: a workgroup per workgroup of
+// k_claims_restore, which adds up the counts before its own.
+__global__ __launch_bounds__(256) void k_displaced(StampWorld W, StampRes r) {
+    __shared__ uint32_t sum[4], wn[4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (r.block[blockIdx.x] == 0) return;
+    uint32_t before = 0;
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += 256) before += r.block[i];
+    for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
+    const uint32_t p = blockIdx.x * 256 + threadIdx.x;
+    const bool on = p < W.npix && W.state[p] >= 2;
+    const uint64_t m = __ballot(on);
+    if (lane == 0) {
+        sum[wv] = before;
+        wn[wv] = (uint32_t)__popcll(m);
     }
+    __syncthreads();
+    uint32_t at = sum[0] + sum[1] + sum[2] + sum[3];
+    for (int k = 0; k < wv; k++) at += wn[k];
+    at += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    if (!on || at >= r.cap) return;
+    const uint64_t xy = W.disp_xy[p], c = W.disp[p];
+    fsg_cell_edit e;
+    e.x = (int32_t)(uint32_t)xy;
+    e.y = (int32_t)(uint32_t)(xy >> 32);
+    e.cell.mat = (uint16_t)c;
+    e.cell.temp = (int16_t)(uint16_t)(c >> 16);
+    e.cell.rgba = (uint32_t)(c >> 32);
+    r.list[at] = e;
 }
 
 // The per-pixel steps of a claim round (d: round).  Each runs in two launch
@@ -1491,6 +1562,30 @@ __global__ void k_stamp_step(StampArgs a, int op, int d) {
     PixelRef ref;
     if (!pixel_ref(a, ref)) return;
     stamp_step(a, ref, op, d);
+}
+
+// Round 0's resolve with the compaction of the pixels it leaves open: one
+// reservation per 256 pixels, for batches small enough that those atomics
+// are few (k_stamp_compact reserves per 2048).
+__global__ __launch_bounds__(256) void k_stamp_resolve0(StampArgs a, int op) {
+    __shared__ uint32_t wn[4], base_s;
+    PixelRef ref;
+    const bool in = pixel_ref(a, ref);
+    if (in) stamp_step(a, ref, op, 0);
+    const bool open = in && !ref.w->state[ref.p] && (uint32_t)ref.w->tgt[ref.p] != NOT_LIVE;
+    const uint64_t m = __ballot(open);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (lane == 0) wn[wv] = (uint32_t)__popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t t = wn[0] + wn[1] + wn[2] + wn[3];
+        base_s = t ? atomicAdd(a.nopen, t) : 0u;
+    }
+    __syncthreads();
+    if (!open) return;
+    uint32_t k = base_s + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    for (int w = 0; w < wv; w++) k += wn[w];
+    a.open[k] = (uint64_t)blockIdx.y << 32 | ref.p;
 }
 
 __global__ void k_stamp_step_list(StampArgs a, int op, int d) {

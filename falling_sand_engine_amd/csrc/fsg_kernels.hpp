@@ -33,6 +33,15 @@ struct StampArgs {
     uint32_t *nopen;           // their count
 };
 
+// Result of one world's stamp, in device memory.
+struct StampRes {
+    uint32_t *count;           // [0] placed, [1] unplaced, [2] displaced
+    uint32_t *hits;            // [nb] displaced SAND per body, then [nb] displaced SOUP
+    uint32_t *block;           // displaced pixels per workgroup of k_claims_restore
+    fsg_cell_edit *list;       // displaced cells in pixel order, at most cap
+    uint32_t nb, cap;
+};
+
 template <int RE, int ZN>
 __global__ void k_tick_world(DevWorld w, uint32_t k, int nfull);
 template <int RE, int ZN, int N>
@@ -55,12 +64,17 @@ __global__ void k_stats(const uint64_t *__restrict__ cells, size_t n, unsigned l
 __global__ void k_fill(uint64_t *cells, size_t n, uint64_t v);
 __global__ void k_copy(const uint4 *__restrict__ src, uint4 *__restrict__ dst, size_t n16);
 __global__ void k_set_cells(uint64_t *cells, int W, int H, const int32_t *xy, const uint64_t *vals, size_t n);
+// The body of every pixel (bodies' indices in order of their first pixel),
+// and `zero` words of zeroed result.
+__global__ void k_pix_body(const fsg_body *bodies, const uint32_t *order, uint32_t nb, uint32_t npix,
+                           uint32_t *pix_body, uint32_t *zero, uint32_t nzero);
 __global__ void k_claims_init(StampArgs a, int save);
-__global__ void k_claims_clear(StampArgs a);
-__global__ void k_claims_restore(StampArgs a);
+__global__ void k_claims_restore(StampArgs a, StampRes r);
+__global__ void k_displaced(StampWorld W, StampRes r);
 // Per-pixel steps of a stamp claim round (k_stamp_step, k_stamp_step_list).
 enum StampOp { OP_PROPOSE = 1, OP_RESOLVE, OP_UNPROPOSE, OP_UNRESOLVE, OP_UNFINISH };
 __global__ void k_stamp_step(StampArgs a, int op, int d);
+__global__ void k_stamp_resolve0(StampArgs a, int op);
 __global__ void k_stamp_step_list(StampArgs a, int op, int d);
 constexpr int STAMP_CPT = 8;  // pixels per thread of k_stamp_compact (grid x: npix / (256 * STAMP_CPT))
 __global__ void k_stamp_compact(StampArgs a);
