@@ -70,26 +70,33 @@ __device__ __forceinline__ bool is_air(const uint64_t *cells, uint32_t airmask, 
     return (airmask >> (uint32_t)(cells[i] & 15u)) & 1u;
 }
 
-// Landings seen by particle `self`: keys[h] = landing cell (EMPTY: free slot),
-// vals[h] = lowest index of a particle that landed there with a non-air tile.
-// keys == nullptr: no landings.
+// Landings seen by particle `self`: slots[h].x = landing cell (EMPTY: free slot),
+// .y = lowest index of a particle that landed there with a non-air tile.
+// slots == nullptr: no landings.
 constexpr uint32_t EMPTY = 0xFFFFFFFFu;
 struct View {
-    const uint32_t *keys, *vals;
+    const uint2 *slots;
     uint32_t mask, self;
 };
 
 __device__ __forceinline__ uint32_t slot_of(uint32_t cell, uint32_t mask) { return fsg::lowbias32(cell) & mask; }
 
+// Whether an earlier particle landed in cell i; q: the slot at i's hash, h.
+__device__ __forceinline__ bool taken(const View &v, uint32_t i, uint32_t h, uint2 q) {
+    for (;;) {  // the table is at most half full
+        if (q.x == EMPTY) return false;
+        if (q.x == i) return q.y < v.self;
+        h = (h + 1) & v.mask;
+        q = v.slots[h];
+    }
+}
+
 // An air cell of the grid that no earlier particle has filled.
 __device__ __forceinline__ bool free_cell(const uint64_t *cells, uint32_t airmask, const View &v, int i) {
     if (!is_air(cells, airmask, i)) return false;
-    if (!v.keys) return true;
-    for (uint32_t h = slot_of((uint32_t)i, v.mask);; h = (h + 1) & v.mask) {  // the table is at most half full
-        const uint32_t k = v.keys[h];
-        if (k == EMPTY) return true;
-        if (k == (uint32_t)i) return v.vals[h] >= v.self;
-    }
+    if (!v.slots) return true;
+    const uint32_t h = slot_of((uint32_t)i, v.mask);
+    return !taken(v, (uint32_t)i, h, v.slots[h]);
 }
 
 // Which 8 x 8 blocks of the grid hold an air cell, found on demand: two bits
@@ -129,9 +136,151 @@ __device__ bool block_has_air(const AirMap &am, const uint64_t *cells, int W, in
     return air;
 }
 
-// One particle's tick against the grid (the reference's loop body).
+// Bit planes of the grid for the rounds (which only read it): one bit per cell
+// that holds air, and one per cell that some landing of the view is in, so
+// that a step of a path is two loads that stay in the L2 and the view's hash
+// is searched only where a landing is.
+struct BitMaps {
+    const uint32_t *air;     // null: not built
+    const uint32_t *landed;  // null: no landings
+    int wpr;                 // words per row
+};
+
+// free_cell for a cell (x, y) of the grid, from its words of the planes.
+__device__ __forceinline__ bool free_word(uint32_t a, uint32_t l, const View &v, int x, int y, int W) {
+    if (!((a >> (x & 31)) & 1u)) return false;
+    if (!((l >> (x & 31)) & 1u)) return true;
+    const uint32_t i = (uint32_t)(x + y * W), h = slot_of(i, v.mask);
+    return !taken(v, i, h, v.slots[h]);
+}
+
+__device__ __forceinline__ bool free_bit(const BitMaps &bm, const View &v, int x, int y, int W) {
+    const size_t w = (size_t)y * bm.wpr + (x >> 5);
+    return free_word(bm.air[w], bm.landed ? bm.landed[w] : 0u, v, x, y, W);
+}
+
+// Index of offset (x, y) on the spiral: ring r starts right of its lower right
+// corner and runs up the right side, left along the top, down the left side
+// and right along the bottom.
+__device__ __forceinline__ uint32_t spiral_index(int x, int y) {
+    const int r = max(abs(x), abs(y));
+    const int side = (x == r && y > -r) ? y + r - 1 : y == r ? 3 * r - 1 - x : x == -r ? 5 * r - 1 - y : 7 * r - 1 + x;
+    return r ? (uint32_t)((2 * r - 1) * (2 * r - 1) + side) : 0u;
+}
+
+// First cell on the spiral among row y's cells `b` (bit k: offset k - 15), as
+// index << 5 | bit; NO_CELL if b is empty.  The row's middle |x| <= |y| is part
+// of one ring's top, walked leftwards, or bottom, walked rightwards; the rest
+// are rings further out, on whose right side they come before the left.
+constexpr uint32_t NO_CELL = 0xFFFFu;
+__device__ __forceinline__ uint32_t first_of_row(uint32_t b, int y) {
+    if (!b) return NO_CELL;
+    const int a = abs(y);
+    const uint32_t hi = (a >= 16 ? 0u : ~1u << (15 + a)), lo = a >= 15 ? 0u : (1u << (15 - a)) - 1u;
+    const uint32_t mid = b & ~(hi | lo);
+    int k;
+    if (mid) {
+        k = y > 0 ? 31 - __builtin_clz(mid) : __builtin_ctz(mid);
+    } else {
+        const int r = (b & hi) ? __builtin_ctz(b & hi) : 99, l = (b & lo) ? 31 - __builtin_clz(b & lo) : -99;
+        k = r - 15 <= 15 - l ? r : l;
+    }
+    return spiral_index(k - 15, y) << 5 | (uint32_t)k;
+}
+
+// The landing search from the planes.  The 32 x 32 offsets of the spiral are a
+// window of the air plane: its rows go into LDS with each row's first cell on
+// the spiral beside them (`rows`, `firsts`: the lane's columns), so the next
+// candidate is a minimum over 32 numbers instead of a walk of up to 1024
+// steps; one taken by an earlier landing is removed from its row.  Walking the
+// window's bits in spiral order instead: 65 us a round for 40 000 particles on
+// 4096^2, with this 24; reading the grid's cells in spiral order: 233.
+// (int)(x + offset) is (int)x + offset for all offsets unless a sum rounds up
+// to the next integer, which the largest sum shows; sums in (-1, 0) give cell 0
+// again, right before or after its own offset or later.  Returns the landing
+// cell or -1, and grows the box over what it read.
+__device__ __forceinline__ int search_bits(PState &s, float cx0, float cy0, int W, int H, const View &view,
+                                           const BitMaps &bm, uint32_t *rows, uint16_t *firsts) {
+    const int mx = (int)cx0, my = (int)cy0;
+    int land = -1, reach = 16;
+    if ((int)(cx0 + 16.0f) == mx + 16 && (int)(cy0 + 16.0f) == my + 16 && max(mx, my) < (1 << 23) - 16) {
+        const int ox = mx - 15, w0 = max(ox, 0) >> 5, sh = max(ox, 0) & 31, up = max(-ox, 0);
+        const bool two = w0 + 1 < bm.wpr;
+        uint32_t best = ~0u;
+        for (int r0 = 0; r0 < 32; r0 += 8) {
+            uint32_t lo[8], hi[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const int y = my - 15 + r0 + u;
+                const bool in = y >= 0 && y < H;
+                const uint32_t *q = bm.air + (size_t)max(y, 0) * bm.wpr + w0;
+                lo[u] = in ? q[0] : 0u;
+                hi[u] = (in && two) ? q[1] : 0u;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const uint32_t b = (uint32_t)((((uint64_t)hi[u] << 32) | lo[u]) >> sh) << up;
+                const uint32_t f = first_of_row(b, r0 + u - 15);
+                rows[(r0 + u) * 256] = b;
+                firsts[(r0 + u) * 256] = (uint16_t)f;
+                best = min(best, f << 5 | (uint32_t)(r0 + u));
+            }
+        }
+        // one candidate, then four at a time: their slots are loaded together
+        for (int some = 1; (best >> 5) != NO_CELL && land < 0; some = 4) {
+            int at[4];
+            uint32_t h[4];
+            uint2 q[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                at[u] = -1;
+                q[u] = make_uint2(EMPTY, 0u);
+                if (u >= some || (best >> 5) == NO_CELL) continue;
+                const int row = (int)(best & 31u), k = (int)(best >> 5 & 31u);
+                at[u] = row << 5 | k;
+                if (!view.slots) break;  // every air cell is free
+                const uint32_t i = (uint32_t)(mx + k - 15 + (my + row - 15) * W);
+                h[u] = slot_of(i, view.mask);
+                q[u] = view.slots[h[u]];
+                const uint32_t b = rows[row * 256] & ~(1u << k);
+                rows[row * 256] = b;
+                firsts[row * 256] = (uint16_t)first_of_row(b, row - 15);
+                best = ~0u;
+#pragma unroll
+                for (int r = 0; r < 32; r++) best = min(best, (uint32_t)firsts[r * 256] << 5 | (uint32_t)r);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                if (at[u] < 0 || land >= 0) continue;
+                const int x = (at[u] & 31) - 15, y = (at[u] >> 5) - 15;
+                const uint32_t i = (uint32_t)(mx + x + (my + y) * W);
+                if (view.slots && taken(view, i, h[u], q[u])) continue;
+                land = (int)i;
+                reach = max(abs(x), abs(y));
+            }
+        }
+    } else {
+        Spiral sp;
+        for (int k = 0; k < NSPIRAL && land < 0; k++) {
+            const int cx = (int)(cx0 + (float)sp.x), cy = (int)(cy0 + (float)sp.y);
+            sp.next();
+            if (cx < 0 || cy < 0 || cx >= W || cy >= H) continue;  // the reference reads out of range here
+            if (free_bit(bm, view, cx, cy, W)) land = cx + cy * W;
+        }
+    }
+    // everything read lies within the ring reached (a cell more for rounding)
+    grow_box(s, max(mx - reach - 1, 0), max(my - reach - 1, 0));
+    grow_box(s, min(mx + reach + 1, W - 1), min(my + reach + 1, H - 1));
+    return land;
+}
+
+// One particle's tick against the grid (the reference's loop body).  BITS: the
+// cells are read from the planes bm (rows, firsts: the lane's columns of the
+// search window in LDS), else from the grid and the on-demand map am.
+template <bool BITS>
 __device__ void move_particle(PState &s, const uint64_t *cells, int W, int H, uint32_t airmask, int4 zone,
-                              const View &view, const AirMap &am) {
+                              const View &view, const AirMap &am, const BitMaps &bm = BitMaps{},
+                              uint32_t *rows = nullptr, uint16_t *firsts = nullptr) {
 #pragma clang fp contract(off)
     fsg_particle c = s.p;
     s.kind = 0;
@@ -166,7 +315,22 @@ __device__ void move_particle(PState &s, const uint64_t *cells, int W, int H, ui
     const int div = (int)((fabsf(c.vx) + fabsf(c.vy)) + 1.0f);
     const float dvx = c.vx / (float)div, dvy = c.vy / (float)div;
     bool done = false;
+    // BITS: the plane's words of the next four steps are loaded together
+    constexpr int AHEAD = 4;
+    uint32_t wa[AHEAD], wl[AHEAD];
     for (int k = 0; k < div && !done; k++) {
+        if (BITS && (k & (AHEAD - 1)) == 0) {
+            float qx = c.x, qy = c.y;
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) {
+                qx += dvx;
+                qy += dvy;
+                const bool in = !(qx < 0.0f || (int)qx >= W || qy < 0.0f || (int)qy >= H);
+                const size_t wd = in ? (size_t)(int)qy * bm.wpr + ((int)qx >> 5) : 0;
+                wa[u] = bm.air[wd];
+                wl[u] = bm.landed ? bm.landed[wd] : 0u;
+            }
+        }
         c.x += dvx;
         c.y += dvy;
         if (c.x < 0.0f || (int)c.x >= W || c.y < 0.0f || (int)c.y >= H) {
@@ -176,7 +340,10 @@ __device__ void move_particle(PState &s, const uint64_t *cells, int W, int H, ui
         const int px = (int)c.x, py = (int)c.y;
         if (c.flags & FSG_PARTICLE_PHASE) continue;
         grow_box(s, px, py);
-        if (free_cell(cells, airmask, view, px + py * W)) continue;
+        const int u = k & (AHEAD - 1);
+        if (BITS ? free_word(u == 0 ? wa[0] : u == 1 ? wa[1] : u == 2 ? wa[2] : wa[3],
+                             u == 0 ? wl[0] : u == 1 ? wl[1] : u == 2 ? wl[2] : wl[3], view, px, py, W)
+                 : free_cell(cells, airmask, view, px + py * W)) continue;
         if (c.in_object_state <= 1) c.in_object_state = 2;  // no OBJECT cells on this grid
         done = true;
         if (c.flags & FSG_PARTICLE_TEMPORARY) {
@@ -184,7 +351,17 @@ __device__ void move_particle(PState &s, const uint64_t *cells, int W, int H, ui
             return;
         }
         grow_box(s, lx, ly);
-        if (!free_cell(cells, airmask, view, lx + ly * W)) {
+        if (!(BITS ? free_bit(bm, view, lx, ly, W) : free_cell(cells, airmask, view, lx + ly * W))) {
+            if (BITS) {
+                s.land = search_bits(s, c.x, c.y, W, H, view, bm, rows, firsts);
+                if (s.land >= 0) {
+                    s.kind = 2;
+                    return;
+                }
+                c.vy = -4.0f;
+                c.y -= 16.0f;
+                continue;
+            }
             // SB offsets at a time: their cells are loaded together, then
             // tested in spiral order.  After the first SB, a 5 x 5 mask of the
             // 8 x 8 blocks the spiral can reach says which hold an air cell;
@@ -268,7 +445,7 @@ __global__ __launch_bounds__(PT) void k_particles(PArgs a) {
     const int t = threadIdx.x;
     uint32_t base = a.start;
     unsigned long long nl = 0;
-    const View none{nullptr, nullptr, 0u, 0u};
+    const View none{nullptr, 0u, 0u};
     const AirMap am{a.airbits, a.air_wpr};
     while (base < a.n) {  // base is the same in every thread
         const uint32_t i = base + (uint32_t)t;
@@ -276,7 +453,7 @@ __global__ __launch_bounds__(PT) void k_particles(PArgs a) {
         const bool mine = i < a.n;
         if (mine) {
             s.p = a.p[i];
-            move_particle(s, a.cells, a.W, a.H, a.airmask, a.zone, none, am);
+            move_particle<false>(s, a.cells, a.W, a.H, a.airmask, a.zone, none, am);
         }
         land_at[t] = (mine && s.kind == 2) ? s.land : -1;
         if (t == 0) first_bad = PT;
@@ -330,37 +507,94 @@ __global__ void k_u32_fill(uint32_t *p, uint32_t n, uint32_t v) {
     if (i < n) p[i] = v;
 }
 
-__global__ void k_ph_clear(uint32_t *keys, uint32_t *vals, uint32_t cap, uint32_t val0, uint32_t *cnt) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < cap) {
-        keys[i] = EMPTY;
-        vals[i] = val0;
+// The landings of a round: a hash of landing cell -> lowest index and, where the
+// planes are built, the bit plane of its cells.
+struct Table {
+    uint2 *slots;
+    uint32_t *landed;
+};
+
+struct PrepArgs {
+    const uint64_t *cells;
+    int W, H;
+    uint32_t airmask;
+    uint32_t *bits;  // the air plane (null: not built)
+    int wpr;
+    uint32_t bit_words, hcap, n, ncnt;
+    Table t[2];
+    int32_t *vkey;
+    uint32_t *cnt;
+    unsigned long long *totals;
+};
+
+// Start of a pass, one launch: the air plane from the grid (a wave takes 64
+// columns of eight rows, so its loads are independent: bound by the read, 23
+// us for 4096^2, 5.7 TB/s), empty tables, no landings, counters at zero.
+__global__ __launch_bounds__(256) void k_ph_prep(PrepArgs a) {
+    const uint32_t i0 = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
+    if (a.bits) {
+        constexpr int R = 8;
+        const int lane = threadIdx.x & 63;
+        const uint32_t nbx = (uint32_t)a.wpr / 2, nby = ((uint32_t)a.H + R - 1) / R;
+        for (uint32_t b = blockIdx.x * 4 + (threadIdx.x >> 6); b < nbx * nby; b += gridDim.x * 4) {
+            const uint32_t by = b / nbx, bx = b - by * nbx;
+            const int x = (int)bx * 64 + lane, y0 = (int)by * R;
+            uint32_t m[R];
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                m[r] = (x < a.W && y0 + r < a.H) ? (uint32_t)a.cells[(size_t)(y0 + r) * a.W + x] & 15u : 32u;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const uint64_t q = __ballot(m[r] < 32u && ((a.airmask >> (m[r] & 31u)) & 1u));
+                if (y0 + r < a.H && lane < 2) a.bits[(size_t)(y0 + r) * a.wpr + 2 * bx + lane] = (uint32_t)(q >> (32 * lane));
+            }
+        }
+        for (uint32_t i = i0; i < a.bit_words; i += step) a.t[0].landed[i] = a.t[1].landed[i] = 0;
     }
-    if (i < 4 && cnt) cnt[i] = i == 1 ? 0xFFFFFFFFu : 0u;  // [0] changes, [1] first change, [2] changed cells
+    for (uint32_t i = i0; i < a.hcap; i += step)
+        a.t[0].slots[i] = a.t[1].slots[i] = make_uint2(EMPTY, EMPTY);
+    for (uint32_t i = i0; i < a.n; i += step) a.vkey[i] = -1;
+    for (uint32_t i = i0; i < a.ncnt; i += step) a.cnt[i] = (i & 3u) == 1u ? 0xFFFFFFFFu : 0u;
+    if (i0 < 2) a.totals[i0] = 0;
+}
+
+// An empty table for the cells' last writers.
+__global__ void k_ph_clear(uint2 *slots, uint32_t cap) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < cap) slots[i] = make_uint2(EMPTY, 0u);
 }
 
 // Adds the landings of particles [0, n): key[i] is a cell or -1.  MAX keeps
 // the highest index per cell (the last writer), else the lowest.
+// prev: the counters of the round before (null: none); nothing to add if it
+// changed no landing.
 template <bool MAX>
-__global__ void k_ph_insert(const int32_t *key, uint32_t n, uint32_t *keys, uint32_t *vals, uint32_t mask) {
+__global__ void k_ph_insert(const int32_t *key, uint32_t n, Table t, uint32_t mask, int wpr, int W,
+                            const uint32_t *prev) {
+    if (prev && prev[0] == 0) return;
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t *landed = t.landed;
     if (i >= n || key[i] < 0) return;
     const uint32_t c = (uint32_t)key[i];
+    if (landed) {
+        const uint32_t y = c / (uint32_t)W, x = c - y * (uint32_t)W;
+        atomicOr(&landed[(size_t)y * wpr + (x >> 5)], 1u << (x & 31u));
+    }
     for (uint32_t h = slot_of(c, mask);; h = (h + 1) & mask) {  // capacity >= 2n: a slot is always found
-        const uint32_t prev = atomicCAS(&keys[h], EMPTY, c);
-        if (prev == EMPTY || prev == c) {
-            if (MAX) atomicMax(&vals[h], i);
-            else atomicMin(&vals[h], i);
+        const uint32_t old = atomicCAS(&t.slots[h].x, EMPTY, c);
+        if (old == EMPTY || old == c) {
+            if (MAX) atomicMax(&t.slots[h].y, i);
+            else atomicMin(&t.slots[h].y, i);
             return;
         }
     }
 }
 
-__device__ __forceinline__ uint32_t ph_lookup(const uint32_t *keys, const uint32_t *vals, uint32_t mask, uint32_t c) {
+__device__ __forceinline__ uint32_t ph_lookup(const uint2 *slots, uint32_t mask, uint32_t c) {
     for (uint32_t h = slot_of(c, mask);; h = (h + 1) & mask) {
-        const uint32_t k = keys[h];
-        if (k == c) return vals[h];
-        if (k == EMPTY) return EMPTY;
+        const uint2 q = slots[h];
+        if (q.x == c) return q.y;
+        if (q.x == EMPTY) return EMPTY;
     }
 }
 
@@ -369,52 +603,83 @@ struct RoundArgs {
     PRes *res;
     int32_t *vkey;          // per particle: its non-air landing cell of the last round, or -1
     int32_t *wkey;          // per particle: its landing cell (any tile), or -1
-    uint32_t start, n;
+    uint32_t n;
     const uint64_t *cells;
     int W, H;
     uint32_t airmask;
     int4 zone;
-    View view;              // self is set per particle
+    uint32_t mask, hcap;    // of the tables
+    Table view;             // the last round's landings (slots null: none)
+    Table clear;            // the table before it, emptied here for the next round (slots null: it is empty)
     uint32_t *cnt;          // [0] landings that changed, [1] first particle whose landing changed,
                             // [2] cells appended to chg
-    const int32_t *prev_chg;  // cells whose landing changed in the last round (null: move every particle)
-    uint32_t prev_nchg;
+    const uint32_t *prev;   // cnt of the last round (null: the first round)
+    uint32_t *air_tiles;    // set if a particle landed with an air tile
+    const int32_t *prev_chg;  // cells whose landing changed in the last round
     int32_t *chg;           // this round's changed cells
     AirMap am;
+    BitMaps bm;
 };
 
-// One round: particles [start, n) against the grid and the view.  A
+// One round: the particles from the first one whose landing changed against the
+// grid and the view.  The round's kernels read the counters of the one before
+// on the device, so several are enqueued at a time; after one that changed
+// nothing the others end at once.  Bound by a lane's chain of loads and the
+// search: 21 us for 40 000 particles on 4096^2, three rounds a pass (233 with
+// the grid's own cells, and a look by the host after each).  A
 // particle none of whose read cells changed its landing in the last round
 // reads what it read then, so its outcome stands and it is not moved again.
 constexpr uint32_t MAX_CHG = 4096;  // changed cells a round tests against (more: every particle moves)
 
+template <bool BITS>
 __global__ __launch_bounds__(256) void k_ph_round(RoundArgs a) {
+    __shared__ uint32_t rows[BITS ? 32 * 256 : 1];
+    __shared__ uint16_t firsts[BITS ? 32 * 256 : 1];
     __shared__ int2 cl[MAX_CHG];  // the changed cells as (x, y), staged once per workgroup
-    const uint32_t i = a.start + blockIdx.x * blockDim.x + threadIdx.x;
-    if (a.prev_chg) {
-        for (uint32_t k = threadIdx.x; k < a.prev_nchg; k += blockDim.x) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t start = 0;
+    if (a.prev) {
+        if (a.prev[0] == 0) return;
+        start = a.prev[1];
+    }
+    if (a.clear.slots) {
+        for (uint32_t h = i; h < a.hcap; h += gridDim.x * blockDim.x) {
+            const uint32_t c = a.clear.slots[h].x;
+            if (c == EMPTY) continue;
+            if (a.clear.landed) {
+                const uint32_t y = c / (uint32_t)a.W, x = c - y * (uint32_t)a.W;
+                a.clear.landed[(size_t)y * a.bm.wpr + (x >> 5)] = 0;
+            }
+            a.clear.slots[h] = make_uint2(EMPTY, EMPTY);
+        }
+    }
+    if (blockIdx.x * blockDim.x + blockDim.x <= start) return;
+    // a long list of changes costs more to test than to move all
+    if (a.prev && a.prev[2] <= MAX_CHG) {
+        const uint32_t nchg = a.prev[2];
+        for (uint32_t k = threadIdx.x; k < nchg; k += blockDim.x) {
             const int c = a.prev_chg[k];
             const int cy = c / a.W;
             cl[k] = make_int2(c - cy * a.W, cy);
         }
         __syncthreads();
-        if (i >= a.n) return;
+        if (i >= a.n || i < start) return;
         const PRes &o = a.res[i];
         bool hit = false;
         if (o.bx0 <= o.bx1) {
-            for (uint32_t k = 0; k < a.prev_nchg; k++) {
+            for (uint32_t k = 0; k < nchg; k++) {
                 const int2 q = cl[k];
                 hit |= q.x >= o.bx0 && q.x <= o.bx1 && q.y >= o.by0 && q.y <= o.by1;
             }
         }
         if (!hit) return;
     }
-    if (i >= a.n) return;
+    if (i >= a.n || i < start) return;
     PState s;
     s.p = a.p[i];
-    View v = a.view;
-    v.self = i;
-    move_particle(s, a.cells, a.W, a.H, a.airmask, a.zone, v, a.am);
+    const View v{a.view.slots, a.mask, i};
+    move_particle<BITS>(s, a.cells, a.W, a.H, a.airmask, a.zone, v, a.am, a.bm, rows + (BITS ? threadIdx.x : 0),
+                        firsts + (BITS ? threadIdx.x : 0));
     PRes r;
     r.p = s.p;
     r.kind = s.kind;
@@ -425,6 +690,7 @@ __global__ __launch_bounds__(256) void k_ph_round(RoundArgs a) {
     r.by1 = s.by1;
     a.res[i] = r;
     const bool solid = s.kind == 2 && !((a.airmask >> (uint32_t)(s.p.tile.mat & 15u)) & 1u);
+    if (s.kind == 2 && !solid) *a.air_tiles = 1u;
     const int32_t k = solid ? s.land : -1;
     const int32_t old = a.vkey[i];
     if (k != old) {
@@ -447,21 +713,25 @@ struct ApplyArgs {
     uint64_t *cells;
     int W, H, tiles_x;
     uint32_t *flags;
-    const uint32_t *keys, *vals;  // last writer per landing cell
+    const uint2 *slots;     // last writer per landing cell (null: a cell has one)
     uint32_t mask;
     unsigned long long *landed;
+    uint32_t *blk;          // survivors per block of 1024 particles (null: not counted)
 };
 
-// Final outcomes: the last particle landing in a cell writes it (an earlier
-// one can only have carried an air tile, which a later landing replaces).
-__global__ __launch_bounds__(256) void k_ph_apply(ApplyArgs a) {
+// Final outcomes.  A cell that a particle with a tile other than air lands in
+// is free to none after it, so cells have one writer unless air tiles
+// landed: then the last one writes.
+__global__ __launch_bounds__(1024) void k_ph_apply(ApplyArgs a) {
+    __shared__ uint32_t wsum[16];
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    bool keep = false;
     unsigned long long nl = 0;
     if (i < a.n) {
         const PRes r = a.res[i];
         if (r.kind == 2) {
             nl = 1;
-            if (ph_lookup(a.keys, a.vals, a.mask, (uint32_t)r.land) == i) {
+            if (!a.slots || ph_lookup(a.slots, a.mask, (uint32_t)r.land) == i) {
                 const fsg_cell &tl = r.p.tile;
                 a.cells[r.land] = (uint64_t)tl.mat | ((uint64_t)(uint16_t)tl.temp << 16) | ((uint64_t)tl.rgba << 32);
                 if (a.flags) {
@@ -470,16 +740,28 @@ __global__ __launch_bounds__(256) void k_ph_apply(ApplyArgs a) {
                 }
             }
         }
-        a.alive[i] = r.kind == 0 && !(r.p.y > (float)a.H);  // erase_if(y > height), world.cpp:2190
+        keep = r.kind == 0 && !(r.p.y > (float)a.H);  // erase_if(y > height), world.cpp:2190
+        a.alive[i] = keep;
         if (r.kind == 0) a.p[i] = r.p;
     }
     for (int off = 32; off > 0; off >>= 1) nl += __shfl_xor(nl, off, 64);
     if ((threadIdx.x & 63) == 0 && nl) atomicAdd(a.landed, nl);
+    if (!a.blk) return;
+    const uint64_t m = __ballot(keep);
+    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = (uint32_t)__popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (int k = 0; k < 16; k++) t += wsum[k];
+        a.blk[blockIdx.x] = t;
+    }
 }
 
 // ---- survivors in list order ---------------------------------------------------
-// Counts per 1024-particle block, an exclusive scan of the counts in one
-// workgroup, then each block writes its survivors from its offset.
+// Counts per 1024-particle block (from k_ph_apply, or k_pc_count where the
+// batch walk ended the pass), then each block writes its survivors from its
+// offset: the sum of the counts before it, which it makes itself for up to
+// 1024 blocks; above, one workgroup scans the counts first.
 __global__ __launch_bounds__(1024) void k_pc_count(const uint8_t *alive, uint32_t n, uint32_t *blk) {
     __shared__ uint32_t wsum[16];
     const uint32_t i = blockIdx.x * 1024 + threadIdx.x;
@@ -518,17 +800,26 @@ __global__ __launch_bounds__(1024) void k_pc_scan(uint32_t *blk, uint32_t nb, ui
 }
 
 __global__ __launch_bounds__(1024) void k_pc_scatter(const fsg_particle *in, const uint8_t *alive, uint32_t n,
-                                                     const uint32_t *blk, fsg_particle *out) {
-    __shared__ uint32_t wsum[16];
+                                                     const uint32_t *blk, bool scanned, fsg_particle *out,
+                                                     uint32_t *total) {
+    __shared__ uint32_t wsum[16], before[16];
     const uint32_t i = blockIdx.x * 1024 + threadIdx.x;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const bool keep = i < n && alive[i];
     const uint64_t m = __ballot(keep);
     if (lane == 0) wsum[wv] = (uint32_t)__popcll(m);
+    if (!scanned) {
+        uint32_t v = threadIdx.x < blockIdx.x ? blk[threadIdx.x] : 0u;
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        if (lane == 0) before[wv] = v;
+    }
     __syncthreads();
-    uint32_t off = blk[blockIdx.x];
+    uint32_t off = scanned ? blk[blockIdx.x] : 0u;
+    if (!scanned)
+        for (int k = 0; k < 16; k++) off += before[k];
     for (int k = 0; k < wv; k++) off += wsum[k];
     if (keep) out[off + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = in[i];
+    if (!scanned && blockIdx.x == gridDim.x - 1 && threadIdx.x == 1023) *total = off + wsum[15];
 }
 
 using fsg_impl::dev_alloc;
@@ -561,18 +852,44 @@ int grow_lists(fsg_world *w, size_t want) {
     return FSG_OK;
 }
 
+// Rounds before a list whose landings keep changing goes to the batch walk: as
+// many as the walk would need batches for the list, as a round and a batch
+// take about the same time and a round moves every particle (300 000 on 1024^2,
+// most of them in packed heaps: 133 ms a pass with 24 rounds, 9 with 256;
+// 20 heaps of 150 particles: 12 ms with 24, 59 with 256).  Three are enqueued
+// before the host looks at their counters, then six at a time (a spray over
+// terrain takes three; a round that has nothing to do costs about 5 us, a
+// look 20).
+constexpr int MAX_ROUNDS = 256, MIN_ROUNDS = 24;
+constexpr int ROUNDS_AHEAD = 3, LATER_AHEAD = 6;
+constexpr uint32_t CNT_WORDS = 4 * MAX_ROUNDS + 4;  // four a round, then: air tiles landed
+
 // Round buffers for `n` particles, carved from one block: results, the two
-// landing keys, the compaction's block offsets, counters, and the landing
-// hash (capacity the power of two >= 2n, so it is at most half full).
+// landing keys, the compaction's block offsets, counters, and two landing
+// tables (capacity the power of two >= 2n, so they are at most half full).
 struct RoundBufs {
     PRes *res;
     int32_t *vkey, *wkey, *chg[2];
-    uint32_t *blk, *cnt, *keys, *vals, *air;
+    uint32_t *blk, *cnt, *air;
+    Table t[2];
     uint32_t hcap, air_words;
     int air_wpr;
+    uint32_t *bits;  // the grid's air plane (null: not built), of bit_words, as each table's
+    uint32_t bit_words;
+    int bit_wpr;
 };
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// The planes' build reads the whole grid (22 us for 4096^2) and the passes they
+// are for are bounded by one lane's chain of loads whatever their number, so
+// up to 2^25 cells they are always built (a pass of 10 particles on 4096^2
+// took 206 us with the on-demand map, of 1000 745; with the planes and the
+// launches below 84 and 115), and above for one particle per 2^17 cells.
+bool want_planes(const fsg_world *w, size_t n) {
+    const size_t cells = (size_t)w->d.W * w->d.H;
+    return cells <= (size_t)1 << 25 || n >= cells >> 17;
+}
 
 int round_bufs(fsg_world *w, size_t n, RoundBufs &b) {
     uint32_t hcap = 1024;
@@ -581,14 +898,27 @@ int round_bufs(fsg_world *w, size_t n, RoundBufs &b) {
     const int nbx = (w->d.W + 7) / 8, nby = (w->d.H + 7) / 8;
     b.air_wpr = (nbx + 15) / 16;
     b.air_words = (uint32_t)((size_t)b.air_wpr * nby);
-    const size_t sz = align256(n * sizeof(PRes)) + 2 * align256(n * 4) + 2 * align256(n * 8) + align256(nb * 4) + 256 +
-                      2 * align256((size_t)hcap * 4) + align256((size_t)b.air_words * 4);
+    b.bit_wpr = 2 * ((w->d.W + 63) / 64);
+    bool planes = want_planes(w, n);
+    b.bit_words = planes ? (uint32_t)((size_t)b.bit_wpr * w->d.H) : 0u;
+    size_t sz = align256(n * sizeof(PRes)) + 2 * align256(n * 4) + 2 * align256(n * 8) + align256(nb * 4) +
+                align256(CNT_WORDS * 4) + 2 * align256((size_t)hcap * 8) + align256((size_t)b.air_words * 4) +
+                3 * align256((size_t)b.bit_words * 4);
     if (w->pround_cap < sz) {
         void *q = nullptr;
-        if (dev_alloc(w->ctx, &q, sz)) return FSG_ERR_NOMEM;
-        dev_free(w->d_pround);
-        w->d_pround = q;
-        w->pround_cap = sz;
+        int rc = dev_alloc(w->ctx, &q, sz);
+        if (rc && planes) {  // short of memory: without the planes
+            planes = false;
+            sz -= 3 * align256((size_t)b.bit_words * 4);
+            b.bit_words = 0;
+            rc = w->pround_cap < sz ? dev_alloc(w->ctx, &q, sz) : FSG_OK;
+        }
+        if (rc) return FSG_ERR_NOMEM;
+        if (q) {
+            dev_free(w->d_pround);
+            w->d_pround = q;
+            w->pround_cap = sz;
+        }
     }
     char *c = static_cast<char *>(w->d_pround);
     b.res = reinterpret_cast<PRes *>(c);
@@ -604,18 +934,24 @@ int round_bufs(fsg_world *w, size_t n, RoundBufs &b) {
     b.blk = reinterpret_cast<uint32_t *>(c);
     c += align256(nb * 4);
     b.cnt = reinterpret_cast<uint32_t *>(c);
-    c += 256;
-    b.keys = reinterpret_cast<uint32_t *>(c);
-    c += align256((size_t)hcap * 4);
-    b.vals = reinterpret_cast<uint32_t *>(c);
-    c += align256((size_t)hcap * 4);
+    c += align256(CNT_WORDS * 4);
+    for (Table &t : b.t) {
+        t.slots = reinterpret_cast<uint2 *>(c);
+        c += align256((size_t)hcap * 8);
+    }
     b.air = reinterpret_cast<uint32_t *>(c);
+    c += align256((size_t)b.air_words * 4);
+    uint32_t *plane[3];
+    for (uint32_t *&q : plane) {
+        q = planes ? reinterpret_cast<uint32_t *>(c) : nullptr;
+        c += align256((size_t)b.bit_words * 4);
+    }
+    b.bits = plane[0];
+    b.t[0].landed = plane[1];
+    b.t[1].landed = plane[2];
     b.hcap = hcap;
     return FSG_OK;
 }
-
-// Rounds before a list whose landings keep changing goes to the batch walk.
-constexpr int MAX_ROUNDS = 24;
 
 }  // namespace
 
@@ -664,43 +1000,71 @@ extern "C" int fsg_world_particles_tick(fsg_world *w, size_t *alive, size_t *lan
         uint64_t *cells = w->d.buf[w->d.tick & 1];
         // landings wake their chunks for the next tick (no flags: it processes every chunk)
         uint32_t *flags = w->flags_valid ? w->d.flags[(w->d.tick + 1) & 1] : nullptr;
-        HIPCHK(hipMemsetAsync(w->d_part_cnt, 0, 16, st));
-        HIPCHK(hipMemsetAsync(b.vkey, 0xFF, (size_t)n * 4, st));  // -1: no landing yet
-        const unsigned hg = (b.hcap + 255) / 256;
-        k_u32_fill<<<(b.air_words + 255) / 256, 256, 0, st>>>(b.air, b.air_words, 0u);
-        RoundArgs ra{w->d_part, b.res, b.vkey, b.wkey, 0u, n, cells, w->d.W, w->d.H, airmask, zone,
-                     View{nullptr, nullptr, b.hcap - 1, 0u}, b.cnt, nullptr, 0u, b.chg[0], AirMap{b.air, b.air_wpr}};
+        const unsigned ng = (n + 255) / 256;
+        {
+            PrepArgs pa{cells, w->d.W, w->d.H, airmask, b.bits, b.bit_wpr, b.bit_words, b.hcap, n, CNT_WORDS,
+                        {b.t[0], b.t[1]}, b.vkey, b.cnt, w->d_part_cnt};
+            // a workgroup per four wave tiles of the plane, up to 16 a CU
+            const size_t tiles = b.bits ? (size_t)(b.bit_wpr / 2) * ((w->d.H + 7) / 8) : 0;
+            const size_t g = std::max<size_t>((tiles + 3) / 4, std::max<size_t>(ng, b.hcap / 256));
+            k_ph_prep<<<(unsigned)std::min<size_t>(g, (size_t)c->n_cu * 16), 256, 0, st>>>(pa);
+        }
+        const unsigned ag = (b.air_words + 255) / 256;
+        if (!b.bits) k_u32_fill<<<ag, 256, 0, st>>>(b.air, b.air_words, 0u);
         uint32_t final_n = 0;  // particles [0, final_n) have their outcomes
-        for (int round = 0; round < MAX_ROUNDS; round++) {
-            k_ph_clear<<<hg, 256, 0, st>>>(b.keys, b.vals, b.hcap, EMPTY, b.cnt);
-            if (round > 0) {
-                k_ph_insert<false><<<(n + 255) / 256, 256, 0, st>>>(b.vkey, n, b.keys, b.vals, b.hcap - 1);
-                ra.view.keys = b.keys;
-                ra.view.vals = b.vals;
+        uint32_t h[CNT_WORDS];
+        // the walk's time is at least that of its batches, so rounds may take as many
+        const int most = (int)std::min<size_t>(MAX_ROUNDS, std::max<size_t>(MIN_ROUNDS, n / PT));
+        for (int round = 0; round < most && final_n < n;) {
+            const int first = round;
+            for (; round < std::min(first + (first ? LATER_AHEAD : ROUNDS_AHEAD), most); round++) {
+                RoundArgs ra{};
+                ra.p = w->d_part;
+                ra.res = b.res;
+                ra.vkey = b.vkey;
+                ra.wkey = b.wkey;
+                ra.n = n;
+                ra.cells = cells;
+                ra.W = w->d.W;
+                ra.H = w->d.H;
+                ra.airmask = airmask;
+                ra.zone = zone;
+                ra.mask = b.hcap - 1;
+                ra.hcap = b.hcap;
+                ra.cnt = b.cnt + 4 * round;
+                ra.air_tiles = b.cnt + 4 * MAX_ROUNDS;
+                ra.prev_chg = b.chg[(round + 1) & 1];
+                ra.chg = b.chg[round & 1];
+                ra.am = AirMap{b.air, b.air_wpr};
+                ra.bm = BitMaps{b.bits, nullptr, b.bit_wpr};
+                if (round > 0) {
+                    ra.prev = ra.cnt - 4;
+                    ra.view = b.t[round & 1];
+                    ra.bm.landed = ra.view.landed;
+                    if (round > 1) ra.clear = b.t[(round + 1) & 1];
+                    k_ph_insert<false><<<ng, 256, 0, st>>>(b.vkey, n, ra.view, ra.mask, b.bit_wpr, w->d.W, ra.prev);
+                }
+                if (b.bits) k_ph_round<true><<<ng, 256, 0, st>>>(ra);
+                else k_ph_round<false><<<ng, 256, 0, st>>>(ra);
             }
-            ra.start = final_n;
-            ra.chg = b.chg[round & 1];
-            k_ph_round<<<(n - final_n + 255) / 256, 256, 0, st>>>(ra);
             HIPCHK(hipGetLastError());
-            uint32_t h[3];
-            if (int rc = fsg_impl::copy_out(c, {{h, b.cnt, 12}})) return rc;
-            if (h[0] == 0) {  // no landing changed: every outcome is the sequential one
-                final_n = n;
-                break;
-            }
-            final_n = h[1];  // the particles before the first changed landing are final
-            // the next round moves only particles that read a changed cell
-            // (a long list of changes costs more to test than to move all)
-            ra.prev_chg = h[2] <= MAX_CHG ? b.chg[round & 1] : nullptr;
-            ra.prev_nchg = h[2];
+            if (int rc = fsg_impl::copy_out(c, {{h, b.cnt, sizeof h}})) return rc;
+            for (int r = first; r < round && final_n < n; r++)
+                // no landing changed: every outcome is the sequential one; else
+                // the particles before the first changed landing are final
+                final_n = h[4 * r] == 0 ? n : h[4 * r + 1];
         }
         if (final_n > 0) {
-            // the last particle landing in a cell writes it
-            k_ph_clear<<<hg, 256, 0, st>>>(b.keys, b.vals, b.hcap, 0u, nullptr);
-            k_ph_insert<true><<<(final_n + 255) / 256, 256, 0, st>>>(b.wkey, final_n, b.keys, b.vals, b.hcap - 1);
             ApplyArgs aa{w->d_part, b.res, w->d_part_alive, final_n, cells, w->d.W, w->d.H, w->d.tiles_x, flags,
-                         b.keys, b.vals, b.hcap - 1, w->d_part_cnt};
-            k_ph_apply<<<(final_n + 255) / 256, 256, 0, st>>>(aa);
+                         nullptr, b.hcap - 1, w->d_part_cnt, final_n == n ? b.blk : nullptr};
+            if (h[4 * MAX_ROUNDS]) {  // air tiles: the last particle landing in a cell writes it
+                const Table t{b.t[0].slots, nullptr};
+                k_ph_clear<<<(b.hcap + 255) / 256, 256, 0, st>>>(t.slots, b.hcap);
+                k_ph_insert<true><<<(final_n + 255) / 256, 256, 0, st>>>(b.wkey, final_n, t, b.hcap - 1, 0, w->d.W,
+                                                                         nullptr);
+                aa.slots = t.slots;
+            }
+            k_ph_apply<<<(final_n + 1023) / 1024, 1024, 0, st>>>(aa);
         }
         if (final_n < n) {
             // the rest, in order, by the batch walk over the grid the prefix left
@@ -719,18 +1083,20 @@ extern "C" int fsg_world_particles_tick(fsg_world *w, size_t *alive, size_t *lan
             a.landed = w->d_part_cnt;
             a.airbits = b.air;
             a.air_wpr = b.air_wpr;
+            if (b.bits) k_u32_fill<<<ag, 256, 0, st>>>(b.air, b.air_words, 0u);
             k_particles<<<1, PT, 0, st>>>(a);
         }
         const uint32_t nb = (n + 1023) / 1024;
-        k_pc_count<<<nb, 1024, 0, st>>>(w->d_part_alive, n, b.blk);
-        k_pc_scan<<<1, 1024, 0, st>>>(b.blk, nb, reinterpret_cast<uint32_t *>(w->d_part_cnt + 1));
-        k_pc_scatter<<<nb, 1024, 0, st>>>(w->d_part, w->d_part_alive, n, b.blk, w->d_part2);
+        uint32_t *total = reinterpret_cast<uint32_t *>(w->d_part_cnt + 1);
+        if (final_n < n) k_pc_count<<<nb, 1024, 0, st>>>(w->d_part_alive, n, b.blk);
+        if (nb > 1024) k_pc_scan<<<1, 1024, 0, st>>>(b.blk, nb, total);
+        k_pc_scatter<<<nb, 1024, 0, st>>>(w->d_part, w->d_part_alive, n, b.blk, nb > 1024, w->d_part2, total);
         HIPCHK(hipGetLastError());
-        unsigned long long h[2] = {0, 0};
-        if (int rc = fsg_impl::copy_out(c, {{h, w->d_part_cnt, 16}})) return rc;
-        nl = h[0];
+        unsigned long long sums[2] = {0, 0};
+        if (int rc = fsg_impl::copy_out(c, {{sums, w->d_part_cnt, 16}})) return rc;
+        nl = sums[0];
         std::swap(w->d_part, w->d_part2);  // the survivors, in order, are the list
-        w->npart = (size_t)(uint32_t)h[1];
+        w->npart = (size_t)(uint32_t)sums[1];
     }
     if (alive) *alive = w->npart;
     if (landed) *landed = (size_t)nl;
