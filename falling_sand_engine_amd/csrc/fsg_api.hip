@@ -294,7 +294,29 @@ int launch_tick(fsg_world *w) {
     // a zone smaller than the world takes the kernels that test it
     const bool zoned = w->d.zx0 > 0 || w->d.zy0 > 0 || w->d.zx1 < w->d.W || w->d.zy1 < w->d.H;
     hipStream_t st = w->ctx->stream;
-    if (sk) {
+    using No = std::integral_constant<int, 0>;
+    using Yes = std::integral_constant<int, 1>;
+    const unsigned cu = (unsigned)w->ctx->n_cu;
+    if (sk && tiles <= 10 * cu) {
+        // skipping, tested by each workgroup.  us a tick (test and list as two
+        // launches of 256 threads / this): 64 chunks of 1024 threads 22.4 /
+        // 16.8, 256 29.8 / 18.3; 484 of 512 threads 30.6 / 22.3, 784 33.2 /
+        // 26.1 (of 256 threads 30.7); 1024 of 256 threads, all awake, 33.0 (of
+        // 512 34.0; half asleep 35.1 / 32.6); 2500 44.1 / 42.8.  From two
+        // rounds of resident workgroups on the sleeping ones' slots cost as
+        // much as the second launch: 4096 54.0 / 55.8, 16384 65 / 86.
+        auto launch = [&](auto re_, auto zn_) {
+            constexpr int R = decltype(re_)::value, Z = decltype(zn_)::value;
+            if (tiles <= cu)
+                fsg::k_tick_small<1, R, Z, fsg::SMALL_NT><<<tiles, fsg::SMALL_NT, 0, st>>>(w->d, 0u);
+            else if (2 * tiles <= 7 * cu)
+                fsg::k_tick_small<1, R, Z, fsg::MEDIUM_NT><<<tiles, fsg::MEDIUM_NT, 0, st>>>(w->d, 0u);
+            else
+                fsg::k_tick_small<1, R, Z, fsg::NT><<<tiles, fsg::NT, 0, st>>>(w->d, 0u);
+        };
+        if (zoned) re ? launch(Yes{}, Yes{}) : launch(No{}, Yes{});
+        else re ? launch(Yes{}, No{}) : launch(No{}, No{});
+    } else if (sk) {
         // the awake chunks listed, then one workgroup per listed chunk; the
         // count of this tick's parity must start at zero (a tick run another
         // way, or a jump of the tick counter, leaves it stale)
@@ -315,7 +337,6 @@ int launch_tick(fsg_world *w) {
         // of 512 15.0; 289 chunks of 512 threads 15.6, of 256 18.2; 484 of
         // 512 19.6, of 256 20.1, and 1024 of 512 27.2, of 256 24.5: with
         // more chunks per compute unit the wider workgroups take more rounds
-        const unsigned cu = (unsigned)w->ctx->n_cu;
         const unsigned slots = (unsigned)(fsg::WGS_PER_CU - (zoned ? 1 : 0)) * cu, rest = tiles % slots;
         // whole chunks in full rounds of resident workgroups, a remainder of
         // at most a quarter round as quarters, which then fill one round (a
@@ -327,14 +348,12 @@ int launch_tick(fsg_world *w) {
             if (4 * tiles <= cu)
                 fsg::k_tick_quarter<R, Z><<<4 * tiles, fsg::QUARTER_NT, 0, st>>>(w->d, 0u);
             else if (tiles <= cu)
-                fsg::k_tick_small<R, Z, fsg::SMALL_NT><<<tiles, fsg::SMALL_NT, 0, st>>>(w->d, 0u);
+                fsg::k_tick_small<0, R, Z, fsg::SMALL_NT><<<tiles, fsg::SMALL_NT, 0, st>>>(w->d, 0u);
             else if (tiles <= 2 * cu)
-                fsg::k_tick_small<R, Z, fsg::MEDIUM_NT><<<tiles, fsg::MEDIUM_NT, 0, st>>>(w->d, 0u);
+                fsg::k_tick_small<0, R, Z, fsg::MEDIUM_NT><<<tiles, fsg::MEDIUM_NT, 0, st>>>(w->d, 0u);
             else
                 fsg::k_tick_world<R, Z><<<nfull + 4u * (tiles - nfull), fsg::NT, 0, st>>>(w->d, 0u, (int)nfull);
         };
-        using No = std::integral_constant<int, 0>;
-        using Yes = std::integral_constant<int, 1>;
         if (zoned) re ? launch(Yes{}, Yes{}) : launch(No{}, Yes{});
         else re ? launch(Yes{}, No{}) : launch(No{}, No{});
     }

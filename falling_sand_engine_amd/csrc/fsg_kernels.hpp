@@ -44,7 +44,7 @@ struct StampRes {
 
 template <int RE, int ZN>
 __global__ void k_tick_world(DevWorld w, uint32_t k, int nfull);
-template <int RE, int ZN, int N>
+template <int SK, int RE, int ZN, int N>
 __global__ void k_tick_small(DevWorld w, uint32_t k);
 template <int RE, int ZN>
 __global__ void k_tick_quarter(DevWorld w, uint32_t k);
