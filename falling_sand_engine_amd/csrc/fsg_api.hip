@@ -1205,6 +1205,24 @@ BatchKernel batch_kernel(int form) {
     }
 }
 
+template <int N>
+BatchKernel batch_small_kernel(int form) {
+    switch (form) {
+    case BF_PLAIN: return fsg::k_tick_batch_small<0, 0, N>;
+    case BF_PLAIN_REACT: return fsg::k_tick_batch_small<0, 1, N>;
+    case BF_SKIP: return fsg::k_tick_batch_small<1, 0, N>;
+    default: return fsg::k_tick_batch_small<1, 1, N>;
+    }
+}
+
+// Threads per chunk of a batch, by the lines of one world's tick.
+unsigned batch_threads(const fsg_ctx *c) {
+    const uint64_t cu = (uint64_t)c->n_cu, t = c->total_tiles;
+    const bool plain = c->batch_form == BF_PLAIN || c->batch_form == BF_PLAIN_REACT;
+    if (!plain && c->batch_form != BF_SKIP && c->batch_form != BF_SKIP_REACT) return fsg::NT;
+    return t <= cu ? fsg::SMALL_NT : 2 * t <= (plain ? 4 : 7) * cu ? fsg::MEDIUM_NT : fsg::NT;
+}
+
 int batch_prepare(fsg_ctx *c, fsg_world *const *ws, int n, bool *graph_ok) {
     for (int i = 0; i < n; i++)
         if (!ws[i] || ws[i]->ctx != c) return FSG_ERR_INVALID;
@@ -1290,13 +1308,16 @@ int batch_run(fsg_ctx *c, fsg_world *const *ws, int n, int ticks, bool graph_ok)
     const unsigned tiles = c->total_tiles;
     const int T = c->tune.graph_ticks;
     const bool listed = batch_listed(c);
+    const unsigned threads = batch_threads(c);
     const BatchKernel kernel =
-        c->tune.occupancy == 4 ? batch_kernel<4>(c->batch_form) : batch_kernel<fsg::WGS_PER_CU>(c->batch_form);
+        threads == fsg::SMALL_NT ? batch_small_kernel<fsg::SMALL_NT>(c->batch_form)
+        : threads == fsg::MEDIUM_NT ? batch_small_kernel<fsg::MEDIUM_NT>(c->batch_form)
+        : c->tune.occupancy == 4 ? batch_kernel<4>(c->batch_form) : batch_kernel<fsg::WGS_PER_CU>(c->batch_form);
     auto tick_launch = [&](uint32_t k) {
         if (listed)
             fsg::k_wake_batch<<<grid_for(tiles, 256), 256, 0, c->stream>>>(c->d_worlds, c->d_tile_start, n, k,
                                                                            c->d_awake, c->d_awake_n);
-        kernel<<<tiles, fsg::NT, 0, c->stream>>>(c->d_worlds, c->d_tile_start, n, k, c->d_awake, c->d_awake_n);
+        kernel<<<tiles, threads, 0, c->stream>>>(c->d_worlds, c->d_tile_start, n, k, c->d_awake, c->d_awake_n);
     };
     // both counts of the awake list start at zero; each tick's wake launch
     // clears the other one, and a graph has an even number of ticks

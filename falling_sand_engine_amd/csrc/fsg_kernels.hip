@@ -513,6 +513,9 @@ __device__ __forceinline__ ZoneTest zone_test(const DevWorld &w, int gx0, int gy
 // Wake test of the skip path: the chunk may change by itself (F_POT), changed
 // last tick (F_ANY: its two state buffers differ), a neighbour changed inside
 // the band the chunk's region overlaps, or the tick is forced.
+// ONE: the chunk's own flags first, which mostly decide (for the test by a
+// workgroup; a wave of 64 chunks' tests needs the neighbours' anyway).
+template <bool ONE>
 __device__ __forceinline__ bool chunk_awake(const DevWorld &w, const uint32_t *fr, int tx, int ty, bool forced) {
     // every load is issued before the first is waited for
     auto fl = [&](int dx, int dy, uint32_t bits) -> uint32_t {
@@ -521,6 +524,7 @@ __device__ __forceinline__ bool chunk_awake(const DevWorld &w, const uint32_t *f
         const uint32_t f = fr[in ? ny * w.tiles_x + nx : ty * w.tiles_x + tx];
         return in ? f & bits : 0u;
     };
+    if (ONE && (forced || (fr[ty * w.tiles_x + tx] & (F_POT | F_ANY)))) return true;
     const uint32_t any = fl(0, 0, F_POT | F_ANY) | fl(0, -1, F_S) | fl(0, 1, F_N) | fl(-1, 0, F_E) | fl(1, 0, F_W) |
                          fl(-1, -1, F_SE) | fl(1, -1, F_SW) | fl(-1, 1, F_NE) | fl(1, 1, F_NW);
     return forced || any != 0;
@@ -566,7 +570,7 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
         const uint32_t *fr = w.flags[(tick + 1) & 1];
         const uint32_t self = fr[tile];
         const bool forced = tick == w.force_tick;
-        sleeps = SK != 3 && !chunk_awake(w, fr, tx, ty, forced);
+        sleeps = SK != 3 && !chunk_awake<!LATE>(w, fr, tx, ty, forced);
         // both state buffers hold this chunk unless it changed last tick
         prev_changed = forced || (self & F_ANY);
         sleeps |= zt.dead && !prev_changed;
@@ -1098,7 +1102,7 @@ __device__ __forceinline__ bool wake_test(const DevWorld &w, uint64_t tick, int 
     const int tx = tile % w.tiles_x, ty = tile / w.tiles_x;
     const uint32_t *fr = w.flags[(tick + 1) & 1];
     const bool forced = tick == w.force_tick;
-    bool awake = chunk_awake(w, fr, tx, ty, forced);
+    bool awake = chunk_awake<false>(w, fr, tx, ty, forced);
     // a chunk outside the zone's reach only needs a tick to copy itself
     if (awake && !forced && !(fr[tile] & F_ANY) && zone_test(w, tx * TW - HALO, ty * TH - HALO).dead) awake = false;
     if (!awake) w.flags[tick & 1][tile] = 0;
@@ -1210,6 +1214,32 @@ FSG_BATCH(3, 0, 0);
 FSG_BATCH(3, 1, 0);
 FSG_BATCH(2, 2, 1);
 #undef FSG_BATCH
+
+// Batches of few chunks, with the wider workgroups of small worlds: such a tick
+// lasts one chunk's latency (us a tick with 256 / these threads: 64 chunks with
+// skipping 25.5 / 18.3, without 16.8 / 14.5; 512 29.3 / 22.5 and 22.4 / 20.2; 896
+// with skipping 33.1 / 28.4; 640 without 24.6 / 24.6).
+template <int SK, int RE, int N>
+__global__ __launch_bounds__(N) void k_tick_batch_small(const DevWorld *__restrict__ worlds,
+                                                        const uint32_t *__restrict__ tile_start, int nworlds,
+                                                        uint32_t k, const uint32_t *, const uint32_t *) {
+    __shared__ __align__(16) TileLds<N> S;
+    const int lo = world_of(tile_start, nworlds, blockIdx.x);
+    const DevWorld &w = worlds[lo];
+    tile_update<SK, RE, 0, N>(w, w.tick + k, (int)(blockIdx.x - tile_start[lo]), S);
+}
+#define FSG_BATCH_SMALL(SK, RE, N)                                                                                   \
+    template __global__ void k_tick_batch_small<SK, RE, N>(const DevWorld *, const uint32_t *, int, uint32_t,        \
+                                                           const uint32_t *, const uint32_t *)
+FSG_BATCH_SMALL(0, 0, SMALL_NT);
+FSG_BATCH_SMALL(0, 1, SMALL_NT);
+FSG_BATCH_SMALL(1, 0, SMALL_NT);
+FSG_BATCH_SMALL(1, 1, SMALL_NT);
+FSG_BATCH_SMALL(0, 0, MEDIUM_NT);
+FSG_BATCH_SMALL(0, 1, MEDIUM_NT);
+FSG_BATCH_SMALL(1, 0, MEDIUM_NT);
+FSG_BATCH_SMALL(1, 1, MEDIUM_NT);
+#undef FSG_BATCH_SMALL
 
 // k_wake over the chunks of every world of a batch, all of which skip: the
 // list holds global chunk indices, its counts go by the parity of k (both

@@ -48,6 +48,9 @@ template <int SK, int RE, int ZN, int N>
 __global__ void k_tick_small(DevWorld w, uint32_t k);
 template <int RE, int ZN>
 __global__ void k_tick_quarter(DevWorld w, uint32_t k);
+template <int SK, int RE, int N>
+__global__ void k_tick_batch_small(const DevWorld *__restrict__ worlds, const uint32_t *__restrict__ tile_start,
+                                   int nworlds, uint32_t k, const uint32_t *, const uint32_t *);
 template <int SK, int RE, int ZN, int WG>
 __global__ void k_tick_batch(const DevWorld *__restrict__ worlds, const uint32_t *__restrict__ tile_start,
                              int nworlds, uint32_t k, const uint32_t *__restrict__ awake,
