@@ -25,11 +25,13 @@
 // (material, temperature, alpha, padding) all become matches.  The last 12
 // bytes of a block are literals, as the format requires.
 //
-// Decoding: one wave per block (fsg_lz4.hpp), four waves per workgroup, into
-// a record staging area; then one workgroup per chunk checks every record and
+// Decoding: one wave per block (fsg_lz4.hpp), four waves per workgroup, or for
+// few blocks a workgroup each (fsg_lz4_wide.hpp), into a record staging area;
+// then one workgroup per chunk checks every record and
 // writes the cells.
 #include "fsg_internal.hpp"
 #include "fsg_lz4.hpp"
+#include "fsg_lz4_wide.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -505,6 +507,93 @@ __global__ __launch_bounds__(64 * DW) __attribute__((amdgpu_waves_per_eu(8))) vo
     if (lane == 0) result[v] = r;
 }
 
+// The group policy of the wide decode: this thread.
+struct WideGroup {
+    int t;
+    template <class T>
+    struct Reg {
+        T v;
+        __device__ T &operator[](int) { return v; }
+    };
+    template <class F>
+    __device__ void each(F f) {
+        f(t);
+    }
+    __device__ void sync() { __syncthreads(); }
+    __device__ uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+    __device__ void min(uint32_t *p, uint32_t v) { atomicMin(p, v); }
+    __device__ void or_(uint32_t *p, uint32_t v) { atomicOr(p, v); }
+    // the sequences on the chain from the wave's entry
+    __device__ void chain(Reg<uint32_t> &nx, Reg<int> &entry, Reg<uint64_t> &mask) {
+        const int seg = __builtin_amdgcn_readfirstlane(t & ~63);
+        uint64_t m = 0;
+        for (int at = __builtin_amdgcn_readfirstlane(entry.v); at >= 0 && at < 64;) {
+            const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)nx.v, at);
+            if (to == fsg_lz4::STOP) break;
+            m |= 1ull << at;
+            at = (int)to - seg;
+        }
+        mask.v = m;
+    }
+    // the wave's running sum, along rows of 16 lanes, then across them
+    __device__ int inclusive(int v) {
+        v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1
+        v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);   // row_shr:2
+        v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);   // row_shr:4
+        v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);   // row_shr:8
+        v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+        v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+        return v;
+    }
+    template <class F>
+    __device__ void prefix(F f, Reg<int> &before, uint32_t *sums) {
+        const int v = f(t), s = inclusive(v);
+        before.v = s - v;
+        if ((t & 63) == 63) sums[t >> 6] = (uint32_t)s;
+    }
+    __device__ int waves_before(int, const uint32_t *sums, int &total) {
+        constexpr int NW = fsg_lz4::WT / 64;
+        const int s = inclusive((t & 63) < NW ? (int)sums[t & 63] : 0), wv = __builtin_amdgcn_readfirstlane(t >> 6);
+        total = __builtin_amdgcn_readlane(s, NW - 1);
+        return wv ? __builtin_amdgcn_readlane(s, wv - 1) : 0;
+    }
+    // a thread's word where it has one, the wave's threads for more
+    __device__ void cover(int, int *p, int v, int a, int b) {
+        if (b - a == 1) p[a] = v;
+        for (uint64_t m = __ballot(b - a > 1); m; m &= m - 1) {
+            const int k = __builtin_ctzll(m);
+            const int kv = __builtin_amdgcn_readlane(v, k), ka = __builtin_amdgcn_readlane(a, k),
+                      kb = __builtin_amdgcn_readlane(b, k);
+            for (int w = ka + (t & 63); w < kb; w += 64) p[w] = kv;
+        }
+    }
+};
+
+// A workgroup per block (fsg_lz4_wide.hpp): about 22 000 cycles a batch of 1 KB of
+// block, a third of them the output bytes' lookups (VALU issue), a sixth the
+// barriers, the rest LDS latency of the parse and the chains.
+__global__ __launch_bounds__(fsg_lz4::WT) void k_pack_decode_wide(const uint8_t *in, const DecDesc *desc, uint8_t *out,
+                                                                  int32_t *result) {
+    __shared__ __align__(16) fsg_lz4::WideLds S;
+    const DecDesc d = desc[blockIdx.x];
+    WideGroup g{(int)threadIdx.x};
+    int r = -1;
+    if (d.n >= 0) r = fsg_lz4::decode_wide(in + d.off, d.n, out + d.dst, d.cap, S, g);
+    if (threadIdx.x == 0) result[blockIdx.x] = r;
+}
+
+// A workgroup per block up to six blocks per compute unit (two at a time are
+// resident, and half of an unpack's blocks are short), else a wave per block.
+// Unpack of 1 chunk 3.3 ms by waves, 1.1 by workgroups; of 256 (512 blocks) 3.7
+// and 1.3; of 576 3.8 and 2.8; of 1024 3.8 and 4.1, as a workgroup does more
+// work for a block than a wave.
+void launch_decode(const fsg_ctx *c, const uint8_t *in, const DecDesc *desc, uint8_t *out, int32_t *result, int n) {
+    if (n <= 6 * c->n_cu)
+        k_pack_decode_wide<<<(unsigned)n, fsg_lz4::WT, 0, c->stream>>>(in, desc, out, result);
+    else
+        k_pack_decode<<<(unsigned)((n + DW - 1) / DW), 64 * DW, 0, c->stream>>>(in, desc, out, result, n);
+}
+
 // Little-endian u32 at a 4-byte aligned staging address (records are 12 or
 // 4 bytes and each chunk's staging starts at a multiple of 4).
 __device__ __forceinline__ uint32_t ld32(const uint8_t *p) { return *reinterpret_cast<const uint32_t *>(p); }
@@ -765,7 +854,7 @@ extern "C" int fsg_world_unpack(fsg_world *w, int32_t x0, int32_t y0, int32_t nc
     if (int rc = fsg_impl::copy_in(c, d_desc, desc.data(), 2 * n * sizeof(DecDesc))) return rc;
     if (b_l2 + b_bg) HIPCHK(hipMemsetAsync(dec + b_desc + b_st, 0, b_l2 + b_bg, c->stream));  // failed chunks: 0
     uint8_t *raw = static_cast<uint8_t *>(w->d_pack_raw);
-    k_pack_decode<<<(unsigned)((2 * n + DW - 1) / DW), 64 * DW, 0, c->stream>>>(src, d_desc, raw, d_bst, (int)(2 * n));
+    launch_decode(c, src, d_desc, raw, d_bst, (int)(2 * n));
     k_pack_cells<<<(unsigned)n, 256, 0, c->stream>>>(raw, d_bst, d, d_cst);
     HIPCHK(hipGetLastError());
     if (int rc = fsg_impl::copy_out(c, {{status, d_cst, n * 4},
@@ -811,9 +900,8 @@ extern "C" int fsg_lz4_decode_blocks(fsg_ctx *c, const void *src, size_t src_len
     if (src_len) HIPCHK(hipMemcpyAsync(d_src.p, src, src_len, hipMemcpyHostToDevice, c->stream));
     if (out_len) HIPCHK(hipMemcpyAsync(d_out.p, out, out_len, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(d_desc.p, desc.data(), (size_t)n * sizeof(DecDesc), hipMemcpyHostToDevice, c->stream));
-    k_pack_decode<<<(unsigned)((n + DW - 1) / DW), 64 * DW, 0, c->stream>>>(
-        static_cast<const uint8_t *>(d_src.p), static_cast<const DecDesc *>(d_desc.p),
-        static_cast<uint8_t *>(d_out.p), static_cast<int32_t *>(d_res.p), n);
+    launch_decode(c, static_cast<const uint8_t *>(d_src.p), static_cast<const DecDesc *>(d_desc.p),
+                  static_cast<uint8_t *>(d_out.p), static_cast<int32_t *>(d_res.p), n);
     HIPCHK(hipGetLastError());
     if (out_len) HIPCHK(hipMemcpyAsync(out, d_out.p, out_len, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipMemcpyAsync(result, d_res.p, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
