@@ -18,7 +18,7 @@
 // block format decodes the same, so the encoder uses one that parallelises:
 // every byte is compared with the byte one record back and one record row
 // (128 records) back, runs of equal bytes of 4 or more become matches with
-// that offset, and the rest are literals.  A thread parses one record row;
+// that offset, and the rest are literals.  A wave parses one record row;
 // matches do not cross rows, literal runs do (a prefix scan over the rows
 // gives each row the literals carried into it).  Runs of identical cells,
 // identical rows, and the fields that repeat between neighbouring records
@@ -47,8 +47,7 @@ constexpr int CAPA = bound(NA), CAPB = bound(NB);
 constexpr size_t SLOT = ((size_t)CAPA + CAPB + 255) & ~(size_t)255;  // encoder output per chunk
 constexpr size_t RAW = (size_t)NA + NB;          // decoder output per chunk
 constexpr int HDR = 17;
-constexpr int KX = 0, KL = 1, KU = 2;            // byte kinds: literal, as one record back, as one row back
-constexpr int PT = 256;                          // encoder threads (one per record row of block A)
+constexpr int PT = 1024;                         // encoder threads
 
 struct PackSrc {
     const uint64_t *cells;  // world grid
@@ -105,92 +104,91 @@ __device__ __forceinline__ uint32_t eqmask(uint64_t x) {
 
 __device__ __forceinline__ int extlen(int v) { return v >= 15 ? (v - 15) / 255 + 1 : 0; }
 
-// Records of every row staged at a time, per column block (LDS, coalesced
-// loads: consecutive threads read consecutive cells of a row).  One thread
-// per row reading its own records touched 64 cache lines per wave load:
-// 17.1 ms for 16384 chunks, against 12.1 ms staged 4 columns at a time (8:
-// 13.9 ms, 16: 18.8, 2: 15.7; the staging's LDS sets the occupancy).
-constexpr int CB = 4;
+constexpr int ROWS = NA / (CW * RA);  // most record rows of a block: 256
 
-// Parses the block's record rows, thread t taking row t (bytes
-// [t*128*R, (t+1)*128*R) of an n-byte block) into runs and handing each match
-// to the sink; returns the literal bytes pending at the row's end.  Every
-// thread of the workgroup calls it (the rows' records are staged in LDS by
-// all of them, CB columns at a time); threads t >= rows only stage.
-template <int R, class Rec, class Sink>
-__device__ int walk_row(int rows, int n, const Rec &rec, uint64_t (*stage)[CB], Sink &sink) {
-    constexpr uint32_t FULL = (1u << R) - 1;
-    const int t = threadIdx.x;
-    const bool mine = t < rows;
-    const int i0 = t * CW;
-    const int forced = n - fsg_lz4::MFLIMIT;  // bytes from here on are literals
-    uint64_t left = mine && i0 > 0 ? rec(i0 - 1) : 0ull;
-    int kind = -1, len = 0, pend = 0;
-    auto close = [&](int end) {
-        if (kind != KX && len >= fsg_lz4::MINMATCH) {
-            sink.match(pend, end - len, len, kind == KL ? R : CW * R);
-            pend = 0;
-        } else {
-            pend += len;
-        }
-    };
-    for (int jb = 0; jb < CW; jb += CB) {
-        __syncthreads();  // the last column block's readers are done
-        for (int k = t; k < rows * CB; k += PT) {
-            const int r = k / CB, c = k - r * CB;
-            stage[r][c] = rec(r * CW + jb + c);
-        }
-        __syncthreads();
-        if (!mine) continue;
-        sink.window(i0 + jb, stage[t], left);
-        for (int jj = 0; jj < CB; jj++) {
-            const int j = jb + jj, i = i0 + j;
-            const uint64_t v = stage[t][jj];
-            const uint32_t mL = i > 0 ? eqmask<R>(v ^ left) : 0u;
-            const uint32_t mU = i >= CW ? eqmask<R>(v ^ stage[t - 1][jj]) : 0u;  // the row above: thread t - 1's
-            left = v;
-            const int p0 = i * R;
-            uint32_t live = FULL;
-            if (p0 + R > forced) live = p0 >= forced ? 0u : ((1u << (forced - p0)) - 1u);
-            const uint32_t isL = mL & live, isU = mU & ~mL & live;
-            const uint32_t same = kind == KL ? isL : kind == KU ? isU : kind == KX ? (~(isL | isU) & FULL) : 0u;
-            if (same == FULL) {
-                len += R;
-                continue;
-            }
-            // runs of one kind inside the record, found with bit scans
-            const uint32_t isX = ~(isL | isU) & FULL;
-            for (int b = 0; b < R;) {
-                const int k = (isL >> b & 1u) ? KL : (isU >> b & 1u) ? KU : KX;
-                const uint32_t m = k == KL ? isL : k == KU ? isU : isX;
-                const int run = min(R - b, __builtin_ctz(~(m >> b)));  // bytes of kind k from b on
-                if (k == kind) {
-                    len += run;
-                } else {
-                    if (kind >= 0) close(p0 + b);
-                    kind = k;
-                    len = run;
-                }
-                b += run;
-            }
-        }
+// One record row parsed by a wave, two records (W bytes) a lane.  The lanes
+// compare their bytes with the record before and the row above and keep the
+// two answers as bit masks; runs of equal kind start where a mask changes, and
+// a run's end, the last match before a lane and the next one after it are
+// found by ballots.  Positions are bytes from the row's start.
+template <int R>
+struct RowParse {
+    static constexpr int W = 2 * R, S = CW * R;
+    uint32_t word[W / 4];      // the lane's bytes
+    uint32_t lmask, start;     // bytes that equal the record before; run starts
+    uint32_t match;            // starts of match runs (4 bytes or more, not literals)
+    int next;                  // first run start past the lane
+    int pe;                    // end of the last match that starts before the lane (-1: none)
+    uint64_t lanes;            // lanes in which a match starts
+
+    // End of the run that starts at bit b of the lane.
+    __device__ int end_of(int lane, int b) const {
+        const uint32_t m = start & ~((2u << b) - 1u);
+        return m ? lane * W + __builtin_ctz(m) : next;
     }
-    if (mine) close((i0 + CW) * R);
-    return pend;
-}
-// Pass 1: the sizes of the sequences whose match lies in the row.
-struct Sizer {
-    bool hm = false;
-    int lead = 0, rest = 0;
-    __device__ void window(int, const uint64_t *, uint64_t) {}
-    __device__ void match(int pend, int, int ml, int) {
-        if (!hm) {
-            hm = true;
-            lead = pend;
-            rest += 3 + extlen(ml - 4);
-        } else {
-            rest += 1 + extlen(pend) + pend + 2 + extlen(ml - 4);
+    template <class Rec>
+    __device__ void parse(int row, int lane, int n, const Rec &rec) {
+        constexpr uint32_t FULL = (1u << W) - 1u;
+        const int i = row * CW + 2 * lane;
+        const uint64_t v0 = rec(i), v1 = rec(i + 1);
+        const uint64_t u0 = row ? rec(i - CW) : 0ull, u1 = row ? rec(i + 1 - CW) : 0ull;
+        uint64_t left = __shfl_up(v1, 1, 64);
+        const uint64_t wrap = __shfl(u1, 63, 64);  // the row above's last record comes before this row's first
+        if (lane == 0) left = wrap;
+        uint32_t mL = eqmask<R>(v1 ^ v0) << R, mU = 0;
+        if (i > 0) mL |= eqmask<R>(v0 ^ left);
+        if (row) mU = eqmask<R>(v0 ^ u0) | eqmask<R>(v1 ^ u1) << R;
+        const int p0 = i * R, forced = n - fsg_lz4::MFLIMIT;  // bytes from forced on are literals
+        const uint32_t live = p0 + W <= forced ? FULL : p0 >= forced ? 0u : (1u << (forced - p0)) - 1u;
+        lmask = mL & live;
+        const uint32_t umask = mU & ~mL & live;
+        const uint32_t before = __shfl_up(((lmask >> (W - 1)) & 1u) | ((umask >> (W - 1)) & 1u) << 1, 1, 64);
+        start = ((lmask ^ (lmask << 1 | (before & 1u))) | (umask ^ (umask << 1 | (before >> 1 & 1u)))) & FULL;
+        if (lane == 0) start |= 1u;
+        const uint64_t any = __ballot(start != 0), above = any & ~((2ull << lane) - 1ull);
+        const int first = lane * W + (start ? __builtin_ctz(start) : 0);
+        const int nf = __shfl(first, above ? __builtin_ctzll(above) : 0, 64);
+        next = above ? nf : S;
+        match = 0;
+        int lme = 0;
+        for (uint32_t m = start & (lmask | umask); m; m &= m - 1) {
+            const int b = __builtin_ctz(m), e = end_of(lane, b);
+            if (e - (lane * W + b) < fsg_lz4::MINMATCH) continue;
+            match |= 1u << b;
+            lme = e;
         }
+        lanes = __ballot(match != 0);
+        const uint64_t below = lanes & ((1ull << lane) - 1ull);
+        const int pl = __shfl(lme, below ? 63 - __builtin_clzll(below) : 0, 64);
+        pe = below ? pl : -1;
+        auto put = [&](int k, uint64_t v) {
+            if (R == RB) {
+                word[k] = (uint32_t)v;
+            } else {
+                word[3 * k] = (uint32_t)v & 0xFFu;
+                word[3 * k + 1] = (uint32_t)(v >> 32);
+                word[3 * k + 2] = ((uint32_t)v >> 16) | ((uint32_t)v & 0xFF00u) << 8;
+            }
+        };
+        put(0, v0);
+        put(1, v1);
+    }
+    // Bytes of the lane's sequences; the row's first one without its literals
+    // and their length bytes.
+    __device__ int size(int lane) const {
+        int sum = 0, prev = pe;
+        for (uint32_t m = match; m; m &= m - 1) {
+            const int b = __builtin_ctz(m), at = lane * W + b, e = end_of(lane, b), ll = prev < 0 ? 0 : at - prev;
+            sum += 3 + extlen(ll) + ll + extlen(e - at - fsg_lz4::MINMATCH);
+            prev = e;
+        }
+        return sum;
+    }
+    __device__ uint32_t byte(int b) const {
+        uint32_t w = word[0];
+#pragma unroll
+        for (int k = 1; k < W / 4; k++) w = (b >> 2) == k ? word[k] : w;
+        return w >> (8 * (b & 3)) & 0xFFu;
     }
 };
 
@@ -217,133 +215,152 @@ __device__ __forceinline__ int put_len(const Out &o, int oc, int v) {
     return oc;
 }
 
-// Copies raw block bytes [p, p + cnt) to output position at.
-template <int R, class Rec>
-__device__ void put_raw(const Out &o, int at, int p, int cnt, const Rec &rec) {
-    if (cnt <= 0) return;
-    int i = p / R, b = p - i * R;
-    uint64_t v = rec(i);
-    for (int k = 0; k < cnt; k++) {
-        o.put(at + k, rbyte<R>(v, b));
-        if (++b == R && k + 1 < cnt) {
-            b = 0;
-            v = rec(++i);
-        }
+// Sums over the wave's lanes up to and with this one.
+__device__ __forceinline__ int wave_sum(int v, int lane) {
+    for (int d = 1; d < 64; d <<= 1) {
+        const int o = __shfl_up(v, d, 64);
+        v += lane >= d ? o : 0;
     }
+    return v;
 }
 
-// Record i from the thread's staged column block (records base .. base +
-// CB - 1, LDS) or the record just before it (a register) when it lies there,
-// else from the block's source.
-template <class Rec>
-struct Near {
-    const Rec *rec;
-    int base = 0;
-    const uint64_t *win = nullptr;
-    uint64_t prev = 0;
-    __device__ uint64_t operator()(int i) const {
-        const int d = i - base;
-        return win && d >= 0 && d < CB ? win[d] : win && d == -1 ? prev : (*rec)(i);
+// Exclusive sums over the rows; every thread of the workgroup calls it.
+__device__ __forceinline__ int rows_before(int v, int *sums, int *total) {
+    const int t = threadIdx.x, lane = t & 63;
+    const int s = wave_sum(v, lane);
+    if (lane == 63 && t < ROWS) sums[t >> 6] = s;
+    __syncthreads();
+    int b = 0, all = 0;
+    for (int w = 0; w < ROWS / 64; w++) {
+        b += w < (t >> 6) ? sums[w] : 0;
+        all += sums[w];
     }
-};
+    *total = all;
+    __syncthreads();
+    return b + s - v;
+}
 
-// Pass 2: writes the row's sequences.
-template <int R, class Rec>
-struct Writer {
-    Out o;
-    int oc, carry;
-    bool first = true;
-    Near<Rec> near;
-    __device__ void window(int base, const uint64_t *win, uint64_t prev) {
-        near.base = base;
-        near.win = win;
-        near.prev = prev;
-    }
-    __device__ void match(int pend, int mstart, int ml, int off) {
-        const int ll = first ? carry + pend : pend;
-        o.put(oc++, (uint32_t)((min(ll, 15) << 4) | min(ml - 4, 15)));
-        oc = put_len(o, oc, ll);
-        put_raw<R>(o, oc + (ll - pend), mstart - pend, pend, near);  // carried bytes come from earlier rows
-        oc += ll;
-        o.put(oc++, (uint32_t)off & 0xFFu);
-        o.put(oc++, (uint32_t)off >> 8);
-        oc = put_len(o, oc, ml - 4);
-        first = false;
-    }
-};
-
+// A workgroup of PT threads encodes a block: its waves take the record rows in
+// turn, first for the rows' sizes, then to write them.  Bound by the VALU work of
+// the run loops, whose trips are the lane's with the most runs.  (A thread per
+// row walking its records: 1095 us for 256 chunks, so 190; a pack of 16384
+// chunks 11.0 ms, so 10.7.)
 template <int R, class Rec>
 __device__ void encode_block(int n, const Rec &rec, uint8_t *out, int cap, int32_t *size_out) {
-    constexpr int S = CW * R;
-    const int rows = n / S, L = rows - 1, t = threadIdx.x;
-    __shared__ int hm[PT], lead[PT], trail[PT], size[PT], carry[PT], start[PT], nxt[PT];
-    __shared__ int total;
-    __shared__ uint64_t stage[PT][CB];
-    Sizer sz;
-    const int pend = walk_row<R>(rows, n, rec, stage, sz);
-    if (t < rows) {
-        hm[t] = sz.hm;
-        lead[t] = sz.hm ? sz.lead : S;
-        trail[t] = pend;
-    }
-    __syncthreads();
-    if (t == 0) {
-        int c = 0;
-        for (int u = 0; u < rows; u++) {
-            carry[u] = c;
-            c = trail[u] + (hm[u] ? 0 : c);
-        }
-        int nx = L;
-        for (int u = L; u >= 0; u--) {
-            nxt[u] = nx;
-            if (hm[u]) nx = u;
+    constexpr int S = CW * R, NW = PT / 64;
+    const int rows = n / S, L = rows - 1, t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    __shared__ int hm[ROWS], lead[ROWS], trail[ROWS], rest[ROWS], carry[ROWS], start[ROWS], nxt[ROWS], sums[ROWS / 64];
+    __shared__ int psum[ROWS + 1];
+    __shared__ uint64_t has[ROWS / 64];
+    for (int r = wv; r < rows; r += NW) {
+        RowParse<R> p;
+        p.parse(r, lane, n, rec);
+        const int sum = wave_sum(p.size(lane), lane);
+        const uint64_t lanes = p.lanes;
+        // the row's first match, and the end of its last one
+        int b = p.match ? lane * RowParse<R>::W + __builtin_ctz(p.match) : 0;
+        int e = p.match ? p.end_of(lane, 31 - __builtin_clz(p.match)) : 0;
+        b = __shfl(b, lanes ? __builtin_ctzll(lanes) : 0, 64);
+        e = __shfl(e, lanes ? 63 - __builtin_clzll(lanes) : 0, 64);
+        if (lane == 63) {
+            hm[r] = lanes != 0;
+            lead[r] = lanes ? b : S;
+            trail[r] = lanes ? S - e : S;
+            rest[r] = sum;
         }
     }
     __syncthreads();
-    if (t < rows) {
-        int s = 0;
-        if (hm[t]) s = sz.rest + extlen(carry[t] + lead[t]) + carry[t] + lead[t];
+    const bool mine = t < rows;
+    int total;
+    const int ps = rows_before(mine ? trail[t] : 0, sums, &total);
+    const uint64_t hb = __ballot(mine && hm[t]);
+    if (t < ROWS) {
+        psum[t] = ps;
+        if (lane == 0) has[wv] = hb;
+    }
+    __syncthreads();
+    int sz = 0;
+    if (mine) {
+        // the literals carried into a row: the trailing ones since the last row with a match
+        int prev = 0, nx = L;
+        for (int w = t >> 6; w >= 0; w--) {
+            const uint64_t m = w == (t >> 6) ? has[w] & ((1ull << lane) - 1ull) : has[w];
+            if (m) {
+                prev = 64 * w + 63 - __builtin_clzll(m);
+                break;
+            }
+        }
+        for (int w = t >> 6; w < ROWS / 64; w++) {
+            const uint64_t m = w == (t >> 6) ? has[w] & ~((2ull << lane) - 1ull) : has[w];
+            if (m) {
+                nx = 64 * w + __builtin_ctzll(m);
+                break;
+            }
+        }
+        const int c = ps - psum[prev];
+        carry[t] = c;
+        nxt[t] = nx;
+        if (hm[t]) sz = rest[t] + extlen(c + lead[t]) + c + lead[t];
         if (t == L) {
-            const int llf = hm[t] ? pend : carry[t] + S;
-            s += 1 + extlen(llf) + llf;
+            const int llf = hm[t] ? trail[t] : c + S;
+            sz += 1 + extlen(llf) + llf;
         }
-        size[t] = s;
     }
-    __syncthreads();
-    if (t == 0) {
-        int o = 0;
-        for (int u = 0; u < rows; u++) {
-            start[u] = o;
-            o += size[u];
-        }
-        total = o;
-    }
+    const int at0 = rows_before(sz, sums, &total);
+    if (mine) start[t] = at0;
     __syncthreads();
     if (total > cap) {  // cannot happen for these parses (sizes stay under the LZ4 bound)
         if (t == 0) *size_out = -1;
         return;
     }
     const Out o{out, cap};
-    Writer<R, Rec> w{o, t < rows ? start[t] : 0, t < rows ? carry[t] : 0, true, Near<Rec>{&rec}};
-    walk_row<R>(rows, n, rec, stage, w);
-    if (t < rows) {
-        const int row0 = t * S, tstart = row0 + S - pend;  // first trailing literal byte
-        if (t == L) {
-            // the last sequence: literals only
-            const int llf = hm[t] ? pend : carry[t] + S;
-            int oc = w.oc;
-            o.put(oc++, (uint32_t)(min(llf, 15) << 4));
-            oc = put_len(o, oc, llf);
-            put_raw<R>(o, oc + (llf - pend), tstart, pend, w.near);  // the last staged block, or the source
+    for (int r = wv; r < rows; r += NW) {
+        RowParse<R> p;
+        p.parse(r, lane, n, rec);
+        constexpr int W = RowParse<R>::W;
+        const int sum = wave_sum(p.size(lane), lane), rowsum = __shfl(sum, 63, 64);
+        const int ll1 = carry[r] + lead[r], skip = extlen(ll1) + ll1;  // the first sequence's literals
+        // where the row's trailing literals go: byte b of the row to tail + b
+        int tail;
+        if (r == L) {
+            const int llf = hm[r] ? trail[r] : carry[r] + S;
+            int oc = start[r] + (hm[r] ? rowsum + skip : 0);
+            if (lane == 0) {
+                o.put(oc, (uint32_t)(min(llf, 15) << 4));
+                put_len(o, oc + 1, llf);
+            }
+            oc += 1 + extlen(llf);
+            tail = oc + (llf - trail[r]) - (S - trail[r]);
         } else {
-            // trailing literals belong to the first sequence of the next row with a match
-            // (or to the last sequence)
-            const int u = nxt[t];
-            const int ll0 = carry[u] + lead[u];
-            const int lit_out = start[u] + 1 + extlen(ll0);
-            const int lit_raw = u * S - carry[u];
-            put_raw<R>(o, lit_out + (tstart - lit_raw), tstart, pend, w.near);
+            const int u = nxt[r], ll0 = carry[u] + lead[u];
+            tail = start[u] + 1 + extlen(ll0) + carry[u] + (r - u) * S;
         }
+        // the lane's sequences, and where each one's literals go
+        int oc = start[r] + (sum - p.size(lane)) + (p.pe < 0 ? 0 : skip);
+        auto base_of = [&](int prev, int at) { return prev < 0 ? oc + 1 + extlen(ll1) + carry[r]
+                                                               : oc + 1 + extlen(at - prev) - prev; };
+        // the literals past the lane's last match belong to the next lane with one
+        const int fb = p.match ? base_of(p.pe, lane * W + __builtin_ctz(p.match)) : 0;
+        const uint64_t above = p.lanes & ~((2ull << lane) - 1ull);
+        const int nb = __shfl(fb, above ? __builtin_ctzll(above) : 0, 64);
+        int prev = p.pe, from = max(p.pe - lane * W, 0);
+        auto literals = [&](int a, int b, int base) {
+            for (int k = a; k < b; k++) o.put(base + lane * W + k, p.byte(k));
+        };
+        for (uint32_t m = p.match; m; m &= m - 1) {
+            const int b = __builtin_ctz(m), at = lane * W + b, e = p.end_of(lane, b);
+            const int ll = prev < 0 ? ll1 : at - prev, ml = e - at - fsg_lz4::MINMATCH;
+            literals(from, b, base_of(prev, at));
+            o.put(oc, (uint32_t)(min(ll, 15) << 4 | min(ml, 15)));
+            oc = put_len(o, oc + 1, ll) + ll;
+            const int off = (p.lmask >> b & 1u) ? R : S;
+            o.put(oc++, (uint32_t)off & 0xFFu);
+            o.put(oc++, (uint32_t)off >> 8);
+            oc = put_len(o, oc, ml);
+            prev = e;
+            from = e - lane * W;
+        }
+        literals(from, W, above ? nb : tail);
     }
     if (t == 0) *size_out = total;
 }
@@ -370,7 +387,7 @@ __global__ __launch_bounds__(PT) void k_pack_encode(PackSrc s, uint8_t *slots, i
 // Image offsets (exclusive scan of 17 + A + B over the chunks); off[n] = total,
 // or -1 when a block failed.  One workgroup.
 __global__ __launch_bounds__(1024) void k_pack_offsets(const int32_t *sizes, int n, int64_t *off) {
-    __shared__ int64_t part[1024];
+    __shared__ int64_t part[16];
     __shared__ int bad;
     const int t = threadIdx.x, per = (n + 1023) / 1024, a = min(n, t * per), b = min(n, a + per);
     if (t == 0) bad = 0;
@@ -380,19 +397,19 @@ __global__ __launch_bounds__(1024) void k_pack_offsets(const int32_t *sizes, int
         if (sizes[2 * c] < 0 || sizes[2 * c + 1] < 0) bad = 1;
         s += HDR + sizes[2 * c] + sizes[2 * c + 1];
     }
-    part[t] = s;
-    __syncthreads();
-    if (t == 0) {
-        int64_t o = 0;
-        for (int k = 0; k < 1024; k++) {
-            const int64_t v = part[k];
-            part[k] = o;
-            o += v;
-        }
-        off[n] = bad ? -1 : o;
+    int64_t sum = s;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t v = __shfl_up(sum, d, 64);
+        sum += (t & 63) >= d ? v : 0;
     }
+    if ((t & 63) == 63) part[t >> 6] = sum;
     __syncthreads();
-    int64_t o = part[t];
+    int64_t o = sum - s, all = 0;
+    for (int w = 0; w < 16; w++) {
+        o += w < (t >> 6) ? part[w] : 0;
+        all += part[w];
+    }
+    if (t == 0) off[n] = bad ? -1 : all;
     for (int c = a; c < b; c++) {
         off[c] = o;
         o += HDR + sizes[2 * c] + sizes[2 * c + 1];
@@ -403,10 +420,28 @@ __device__ __forceinline__ void put_i32(uint8_t *p, int32_t v) {
     for (int k = 0; k < 4; k++) p[k] = (uint8_t)((uint32_t)v >> (8 * k));
 }
 
-// Writes each chunk's image: header, then block A, then block B.
+// Thread t of nt copies its share of len bytes: aligned words of the
+// destination, each from the two aligned words of the source it lies in (the
+// word past the last byte is read: encoder slots have room behind them).
+__device__ __forceinline__ void copy_words(uint8_t *dst, const uint8_t *src, int len, int t, int nt) {
+    const int head = min(len, (int)(-(uintptr_t)dst & 3)), words = (len - head) >> 2, done = head + 4 * words;
+    if (t < head) dst[t] = src[t];
+    if (t < len - done) dst[done + t] = src[done + t];
+    const int sh = (int)((uintptr_t)(src + head) & 3);
+    const uint32_t *p = reinterpret_cast<const uint32_t *>(src + head - sh);
+    uint32_t *q = reinterpret_cast<uint32_t *>(dst + head);
+    for (int k = t; k < words; k += nt)
+        q[k] = (uint32_t)((((uint64_t)p[k + 1] << 32) | p[k]) >> (8 * sh));
+}
+static_assert(SLOT >= (size_t)CAPA + CAPB + 8, "room behind block B's last byte");
+
+// Writes each chunk's image: header, then block A, then block B.  ASM workgroups
+// a chunk (of bytes by one workgroup a chunk: 107 us for 256 chunks, 17 MB; so
+// 8.7).
+constexpr int ASM = 8;
 __global__ __launch_bounds__(256) void k_pack_assemble(const uint8_t *slots, const int32_t *sizes,
                                                        const int64_t *off, const int8_t *phase, uint8_t *img) {
-    const int c = blockIdx.x, t = threadIdx.x;
+    const int c = blockIdx.x, t = (int)(blockIdx.y * 256 + threadIdx.x);
     if (off[gridDim.x] < 0) return;
     const int a = sizes[2 * c], b = sizes[2 * c + 1];
     uint8_t *o = img + off[c];
@@ -418,8 +453,8 @@ __global__ __launch_bounds__(256) void k_pack_assemble(const uint8_t *slots, con
         put_i32(o + 9, NB);
         put_i32(o + 13, b);
     }
-    for (int k = t; k < a; k += 256) o[HDR + k] = sa[k];
-    for (int k = t; k < b; k += 256) o[HDR + a + k] = sb[k];
+    copy_words(o + HDR, sa, a, t, 256 * ASM);
+    copy_words(o + HDR + a, sb, b, t, 256 * ASM);
 }
 
 // Decoder input: per block, its bytes in[off, off + n) (n < 0: no block, the
@@ -758,7 +793,7 @@ extern "C" int fsg_world_pack(fsg_world *w, int32_t x0, int32_t y0, int32_t ncx,
     uint8_t *slots = static_cast<uint8_t *>(w->d_pack_slots), *img = static_cast<uint8_t *>(w->d_pack_img);
     k_pack_encode<<<dim3((unsigned)n, 2), PT, 0, c->stream>>>(s, slots, d_sizes);
     k_pack_offsets<<<1, 1024, 0, c->stream>>>(d_sizes, (int)n, d_off);
-    k_pack_assemble<<<(unsigned)n, 256, 0, c->stream>>>(slots, d_sizes, d_off, d_phase, img);
+    k_pack_assemble<<<dim3((unsigned)n, ASM), 256, 0, c->stream>>>(slots, d_sizes, d_off, d_phase, img);
     HIPCHK(hipGetLastError());
     w->pack_sizes.resize(2 * n);
     int64_t total = 0;
