@@ -51,11 +51,11 @@ def build_cpp_tests(verbose: bool = True) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
-    # the LZ4 block decoder of the device codec, built for the host
-    src = os.path.join(ROOT, "tests", "cpp", "lz4_host.cpp")
+    # the LZ4 block decoders of the device codec, built for the host
+    srcs = [os.path.join(ROOT, "tests", "cpp", f) for f in ("lz4_host.cpp", "lz4_wide_host.cpp")]
     lz4 = os.path.join(outdir, "liblz4host.so")
-    cmd = [HIPCC, "--offload-host-only", "-x", "hip", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", CSRC, src,
-           "-o", lz4]
+    cmd = [HIPCC, "--offload-host-only", "-x", "hip", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", CSRC] + srcs + [
+        "-o", lz4]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.run(cmd, check=True)
