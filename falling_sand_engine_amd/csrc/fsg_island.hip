@@ -7,9 +7,12 @@
 // component of at most 1000 cells is cleared to Tiles_NOTHING and, above 10
 // cells, becomes a rigid body textured with its colours.  The outcome does not
 // depend on the fill order: either the whole component (<= 1000 cells) or
-// "more than 1000".  So here each seed gets one workgroup running a BFS with
-// its visited set in LDS (a hash set, never more than half full) and its
-// frontier as a range of the visited list, reading the grid only; the host
+// "more than 1000".  So here each seed gets one workgroup.  It reads a window of
+// 64 x 64 cells around the seed as bits and one wave fills the component in
+// its registers, a row a lane; a component that leaves the window with at most
+// 1000 cells inside is found by a BFS with its visited set in LDS (a hash set,
+// never more than half full) and its frontier as a range of the visited list.
+// Both read the grid only; the host
 // then keeps, in seed order, the first seed of each island (later seeds of a
 // removed island find air, as consecutive calls would), and one more launch
 // writes the body images and clears the islands.
@@ -50,7 +53,38 @@ __device__ __forceinline__ int wave_max(int v) {
     return v;
 }
 
+// Fill of a row: the seeds' runs of m, to both sides.
+__device__ __forceinline__ uint64_t fill_row(uint64_t f, uint64_t m) {
+    uint64_t u = f, d = f, pu = m, pd = m;
+#pragma unroll
+    for (int k = 1; k < 64; k <<= 1) {
+        u |= pu & (u << k);
+        pu &= pu << k;
+        d |= pd & (d >> k);
+        pd &= pd >> k;
+    }
+    return u | d;
+}
+
+__device__ __forceinline__ uint64_t from_lane_below(uint64_t v) {  // lane 0: 0
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0u, (uint32_t)v, 0x138, 0xF, 0xF, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0u, (uint32_t)(v >> 32), 0x138, 0xF, 0xF, true);
+    return (uint64_t)hi << 32 | lo;
+}
+__device__ __forceinline__ uint64_t from_lane_above(uint64_t v) {  // lane 63: 0
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0u, (uint32_t)v, 0x130, 0xF, 0xF, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0u, (uint32_t)(v >> 32), 0x130, 0xF, 0xF, true);
+    return (uint64_t)hi << 32 | lo;
+}
+__device__ __forceinline__ int wave_total(int v) {
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
 // One workgroup per seed; read-only on the grid.  lists: CAP cells per seed.
+// Bound by one wave's chain: the window's load, then a fill step a row of the
+// component's height (more for winding ones).  A seed in solid ground 12 us;
+// by the BFS alone, a memory latency and two barriers a level, 56.
 __global__ __launch_bounds__(IT) void k_island_search(const uint64_t *__restrict__ cells, int W, int H,
                                                       uint32_t solid, const int32_t *__restrict__ xy,
                                                       uint32_t *__restrict__ lists, SeedOut *__restrict__ out) {
@@ -58,7 +92,71 @@ __global__ __launch_bounds__(IT) void k_island_search(const uint64_t *__restrict
     __shared__ uint32_t list[LIST];
     __shared__ uint32_t cnt;
     __shared__ int red[5][IT / 64];
+    __shared__ uint64_t rows[64];
+    __shared__ int outside;  // the component goes on outside the window
     const int tid = threadIdx.x, s = blockIdx.x;
+    const int sx = xy[2 * s], sy = xy[2 * s + 1];
+    if (sx >= 0 && sy >= 0 && sx < W && sy < H) {
+        const int lane = tid & 63, wv = tid >> 6;
+        const int x0 = max(0, min(sx - 32, W - 64)), y0 = max(0, min(sy - 32, H - 64));
+        constexpr int PER = 64 / (IT / 64);  // rows of a wave
+        uint32_t m[PER];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int y = y0 + wv * PER + k, x = x0 + lane;
+            m[k] = y < H && x < W ? (uint32_t)cells[(size_t)y * W + x] & 15u : 32u;
+        }
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const uint64_t b = __ballot(m[k] < 32u && ((solid >> (m[k] & 31u)) & 1u));
+            if (lane == 0) rows[wv * PER + k] = b;
+        }
+        __syncthreads();
+        if (wv == 0) {
+            const uint64_t mask = rows[lane];
+            uint64_t f = lane == sy - y0 ? mask & (1ull << (sx - x0)) : 0ull;
+            int n = 0;
+            for (int step = 0;; step++) {
+                const uint64_t g = fill_row((f | from_lane_below(f) | from_lane_above(f)) & mask, mask);
+                const bool more = __ballot(g != f) != 0;
+                f = g;
+                if (more && (step & 3) != 3) continue;
+                n = wave_total(__popcll(f));
+                if (!more || n > (int)CAP) break;
+            }
+            // the component's cells on a side of the window that is not the grid's
+            uint64_t side = (x0 > 0 ? 1ull : 0ull) | (x0 + 64 < W ? 1ull << 63 : 0ull);
+            if ((lane == 0 && y0 > 0) || (lane == 63 && y0 + 64 < H)) side = ~0ull;
+            const bool goes_on = n <= (int)CAP && __ballot((f & side) != 0) != 0;
+            if (lane == 0) outside = goes_on;
+            if (!goes_on) {
+                SeedOut r{};
+                r.status = n == 0 ? FSG_ISLAND_NONE : n > (int)CAP ? FSG_ISLAND_ATTACHED
+                                  : n < FSG_ISLAND_MIN_BODY ? FSG_ISLAND_REMOVED : FSG_ISLAND_BODY;
+                r.count = (uint32_t)n;
+                if (n > 0 && n <= (int)CAP) {
+                    const int own = __popcll(f);
+                    int at = own;
+                    for (int d = 1; d < 64; d <<= 1) {
+                        const int o = __shfl_up(at, d, 64);
+                        at += lane >= d ? o : 0;
+                    }
+                    at -= own;
+                    const uint32_t row = (uint32_t)(y0 + lane) * (uint32_t)W + (uint32_t)x0;
+                    for (uint64_t b = f; b; b &= b - 1) lists[(size_t)s * CAP + at++] = row + (uint32_t)__builtin_ctzll(b);
+                    r.minx = wave_min(f ? x0 + __builtin_ctzll(f) : INT32_MAX);
+                    r.maxx = wave_max(f ? x0 + 63 - __builtin_clzll(f) : -1);
+                    const uint64_t used = __ballot(f != 0);
+                    r.miny = y0 + __builtin_ctzll(used);
+                    r.maxy = y0 + 63 - __builtin_clzll(used);
+                    r.minidx = (uint32_t)wave_min(f ? (int)(row + (uint32_t)__builtin_ctzll(f)) : INT32_MAX);
+                }
+                if (lane == 0) out[s] = r;
+            }
+        }
+        __syncthreads();
+        if (!outside) return;
+    }
     for (uint32_t i = tid; i < HT; i += IT) ht[i] = 0;
     if (tid == 0) cnt = 0;
     __syncthreads();
@@ -77,7 +175,6 @@ __global__ __launch_bounds__(IT) void k_island_search(const uint64_t *__restrict
             h = (h + 1) & (HT - 1);
         }
     };
-    const int sx = xy[2 * s], sy = xy[2 * s + 1];
     const bool ok = sx >= 0 && sy >= 0 && sx < W && sy < H && is_solid((uint32_t)sy * (uint32_t)W + (uint32_t)sx);
     if (ok && tid == 0) insert((uint32_t)sy * (uint32_t)W + (uint32_t)sx);
     __syncthreads();
