@@ -9,7 +9,7 @@
 // phase, so no atomics are needed; halo cells are recomputed redundantly and
 // shrink by one ring per phase), then lays the colours out in LDS, gathers
 // each output cell's colour from its origin and writes the chunk interior
-// once.  About 24 KB of LDS per workgroup keeps several workgroups resident
+// once.  26.6 KB of LDS per workgroup keeps six workgroups resident
 // per CU, so one workgroup's loads and stores overlap the others' phases.
 // HBM traffic is one read and one write of each cell per tick plus the halo
 // re-read that the L2/MALL mostly absorbs.  This replaces the reference's
