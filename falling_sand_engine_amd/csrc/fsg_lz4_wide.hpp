@@ -4,7 +4,9 @@
 // output bytes, about 1300 cycles each; with fewer blocks than the chip has
 // wave slots that chain is the whole time (256 chunks of 128 x 128, 17 MB of
 // images: 3.4 ms).  Here a workgroup of WT threads
-// takes a block by batches of up to WT input and TOUT output bytes:
+// takes a block by batches of up to WIN input and TOUT output bytes (two input
+// bytes a thread; one: 1.29 ms for those 256 chunks, two 1.13; 512 threads with
+// one: 1.85):
 //   1. every input byte of the batch is parsed as if a sequence began there
 //      (length, literals, offset, match, where the next one begins);
 //   2. the positions each 64-byte segment is left at are found for every
@@ -30,11 +32,13 @@
 
 namespace fsg_lz4 {
 
-constexpr int WT = 1024;           // threads, and input positions parsed per batch
+constexpr int WT = 1024;           // threads
+constexpr int CAND = 2;            // input positions parsed by a thread per batch
+constexpr int WIN = CAND * WT;     // and by all: position c * WT + t is thread t's c-th
 constexpr int IBUF = 16 * WT;      // block bytes in LDS
 constexpr int TOUT = 8192;         // output bytes per batch at most
 constexpr int ORING = 8192;        // the last output bytes in LDS
-constexpr int MAXSEQ = WT / 3 + 2; // sequences of a batch (each takes 3 bytes or more)
+constexpr int MAXSEQ = WIN / 3 + 2; // sequences of a batch (each takes 3 bytes or more)
 constexpr int MAXEXT = 8;          // length bytes of a batched sequence
 constexpr uint32_t STOP = 0x8000u; // no sequence is parsed at this position
 constexpr uint64_t RESOLVED = 0x8000800080008000ull;
@@ -46,9 +50,9 @@ struct WideLds {
     uint32_t H[TOUT / 32];     // bit: a sequence's output starts
     int last[TOUT / 32 + 1];   // the last sequence starting before each word of H
     uint32_t sa[MAXSEQ], sb[MAXSEQ];          // start | literals << 16; literals' place in `in` | offset << 16
-    uint16_t leave[WT];        // where the chain from this position leaves its segment
-    uint32_t wcount[WT / 64], wout[WT / 64];
-    uint32_t cut;              // start << 10 | position of the first sequence left out
+    uint16_t leave[WIN];       // where the chain from this position leaves its segment
+    uint32_t wcount[WIN / 64], wout[WIN / 64];
+    uint32_t cut;              // start << 11 | position of the first sequence left out
 };
 
 // m mod o for 0 <= m < 2^20, o > 0 (the quotient's estimate is off by at most one).
@@ -71,9 +75,9 @@ __host__ __device__ inline int decode_wide(const uint8_t *src, int n, uint8_t *d
     const int adst = (int)((uintptr_t)dst & 3);
     int ip = 0, op = 0, ib = 0;
     bool loaded = false;
-    typename G::template Reg<uint32_t> nx;
-    typename G::template Reg<int> ll, lp, off, len, entry, before;
-    typename G::template Reg<uint64_t> mask;
+    typename G::template Reg<uint32_t> nx[CAND];
+    typename G::template Reg<int> ll[CAND], lp[CAND], off[CAND], len[CAND], entry[CAND], before[CAND];
+    typename G::template Reg<uint64_t> mask[CAND];
     for (;;) {
         if (ip >= n) return -1;
         if (!loaded || (ib + IBUF < n && ip + IBUF / 4 > ib + IBUF)) {
@@ -92,38 +96,40 @@ __host__ __device__ inline int decode_wide(const uint8_t *src, int n, uint8_t *d
         // 1. candidates; every byte read lies in [ip, lim), inside the buffer
         const int lim = n - 16 < ib + IBUF ? n - 16 : ib + IBUF;
         g.each([&](int t) {
-            const int p = ip + t;
-            auto b = [&](int i) { return (uint32_t)S.in[i - ib]; };
-            uint32_t to = STOP;
-            int l = 0, m = 0, q = p + 1, o = 0, e = 0;
-            auto more = [&](int &v, int &at) -> bool {  // length bytes; false: too many, or past lim
-                uint32_t s = 255;
-                for (int k = 0; k < MAXEXT && s == 255; k++) {
-                    if (at >= lim) return false;
-                    s = b(at++);
-                    v += (int)s;
-                }
-                return s != 255;
-            };
-            if (p < lim) {
-                const uint32_t token = b(p);
-                l = (int)(token >> 4);
-                m = (int)(token & 15u);
-                if (l != RUN_MASK || more(l, q)) {
-                    e = q + l;
-                    if (e + 2 <= lim) {
-                        o = (int)(b(e) | b(e + 1) << 8);
-                        int r = e + 2;
-                        if ((m != 15 || more(m, r)) && r <= lim) to = (uint32_t)(r - ip);
+            for (int c = 0; c < CAND; c++) {
+                const int p = ip + c * WT + t;
+                auto b = [&](int i) { return (uint32_t)S.in[i - ib]; };
+                uint32_t to = STOP;
+                int l = 0, m = 0, q = p + 1, o = 0, e = 0;
+                auto more = [&](int &v, int &at) -> bool {  // length bytes; false: too many, or past lim
+                    uint32_t s = 255;
+                    for (int k = 0; k < MAXEXT && s == 255; k++) {
+                        if (at >= lim) return false;
+                        s = b(at++);
+                        v += (int)s;
+                    }
+                    return s != 255;
+                };
+                if (p < lim) {
+                    const uint32_t token = b(p);
+                    l = (int)(token >> 4);
+                    m = (int)(token & 15u);
+                    if (l != RUN_MASK || more(l, q)) {
+                        e = q + l;
+                        if (e + 2 <= lim) {
+                            o = (int)(b(e) | b(e + 1) << 8);
+                            int r = e + 2;
+                            if ((m != 15 || more(m, r)) && r <= lim) to = (uint32_t)(r - ip);
+                        }
                     }
                 }
+                nx[c][t] = to;
+                ll[c][t] = l;
+                lp[c][t] = q - ib;
+                off[c][t] = o;
+                len[c][t] = l + m + MINMATCH;
+                S.leave[c * WT + t] = (uint16_t)(to == STOP ? STOP | (uint32_t)(c * WT + t) : to);
             }
-            nx[t] = to;
-            ll[t] = l;
-            lp[t] = q - ib;
-            off[t] = o;
-            len[t] = l + m + MINMATCH;
-            S.leave[t] = (uint16_t)(to == STOP ? STOP | (uint32_t)t : to);
             if (t < TOUT / 32) S.H[t] = 0;
             if (t == 0) {
                 S.cut = ~0u;
@@ -134,51 +140,61 @@ __host__ __device__ inline int decode_wide(const uint8_t *src, int n, uint8_t *d
         // 2. each position's way out of its segment (a step more is 3 bytes on
         // or more; others' progress, read in any order, only shortens it)
         g.each([&](int t) {
-            const uint32_t end = (uint32_t)(t | 63) + 1;
-            uint32_t e = S.leave[t];
-            while (e < end) {  // STOP lies above every position
-                e = S.leave[e];
-                S.leave[t] = (uint16_t)e;
+            for (int c = 0; c < CAND; c++) {
+                const int at = c * WT + t;
+                const uint32_t end = (uint32_t)(at | 63) + 1;
+                uint32_t e = S.leave[at];
+                while (e < end) {  // STOP lies above every position
+                    e = S.leave[e];
+                    S.leave[at] = (uint16_t)e;
+                }
             }
         });
         g.sync();
         uint32_t last = 0;  // where the real chain ends: past the batch, or STOP | position
         g.each([&](int t) {
-            const uint32_t seg = (uint32_t)t & ~63u;
             uint32_t e = 0;
-            while (e < seg) e = g.uniform(S.leave[e]);
-            entry[t] = e < seg + 64 ? (int)(e - seg) : -1;
-            while (e < (uint32_t)WT) e = g.uniform(S.leave[e]);
+            for (int c = 0; c < CAND; c++) {
+                const uint32_t seg = (uint32_t)(c * WT + (t & ~63));
+                while (e < seg) e = g.uniform(S.leave[e]);
+                entry[c][t] = e < seg + 64 ? (int)(e - seg) : -1;
+            }
+            while (e < (uint32_t)WIN) e = g.uniform(S.leave[e]);
             last = e;
         });
-        g.chain(nx, entry, mask);
+        for (int c = 0; c < CAND; c++) g.chain(nx[c], entry[c], mask[c], c * WT);
         // 3. output positions
-        g.prefix([&](int t) { return (mask[t] >> (t & 63)) & 1u ? len[t] : 0; }, before, S.wout);
+        for (int c = 0; c < CAND; c++)
+            g.prefix([&](int t) { return (mask[c][t] >> (t & 63)) & 1u ? len[c][t] : 0; }, before[c],
+                     S.wout + c * (WT / 64));
         g.each([&](int t) {
-            if ((t & 63) == 0) S.wcount[t >> 6] = (uint32_t)popc64(mask[t]);
+            if ((t & 63) == 0)
+                for (int c = 0; c < CAND; c++) S.wcount[c * (WT / 64) + (t >> 6)] = (uint32_t)popc64(mask[c][t]);
         });
         g.sync();
         int total = 0;
         g.each([&](int t) {
-            const int c = g.waves_before(t, S.wcount, total), o = g.waves_before(t, S.wout, total);
-            before[t] += o;
-            const int at = before[t], end = at + len[t];
-            const bool in = (mask[t] >> (t & 63)) & 1u, fits = end <= TOUT;
-            const int r = c + popc64(mask[t] & ((1ull << (t & 63)) - 1));
-            // (a sequence after the cut stands past the batch's last byte)
-            g.cover(t, S.last, r, (at >> 5) + 1, in && fits ? (end >> 5) + 1 : 0);
-            if (!in) return;
-            if (off[t] == 0 || off[t] > op + at + ll[t] || !fits || op + end + 16 > cap)
-                g.min(&S.cut, (uint32_t)at << 10 | (uint32_t)t);
-            if (!fits) return;
-            S.sa[r] = (uint32_t)at | (uint32_t)ll[t] << 16;
-            S.sb[r] = (uint32_t)lp[t] | (uint32_t)off[t] << 16;
-            g.or_(&S.H[at >> 5], 1u << (at & 31));
+            for (int c = 0; c < CAND; c++) {
+                int none;
+                const int at = before[c][t] + g.waves_before(t, c, S.wout, total), end = at + len[c][t];
+                const bool in = (mask[c][t] >> (t & 63)) & 1u, fits = end <= TOUT;
+                const int r = g.waves_before(t, c, S.wcount, none) +
+                              popc64(mask[c][t] & ((1ull << (t & 63)) - 1));
+                // (a sequence after the cut stands past the batch's last byte)
+                g.cover(t, S.last, r, (at >> 5) + 1, in && fits ? (end >> 5) + 1 : 0);
+                if (!in) continue;
+                if (off[c][t] == 0 || off[c][t] > op + at + ll[c][t] || !fits || op + end + 16 > cap)
+                    g.min(&S.cut, (uint32_t)(at < 2 * TOUT ? at : 2 * TOUT) << 11 | (uint32_t)(c * WT + t));
+                if (!fits) continue;
+                S.sa[r] = (uint32_t)at | (uint32_t)ll[c][t] << 16;
+                S.sb[r] = (uint32_t)lp[c][t] | (uint32_t)off[c][t] << 16;
+                g.or_(&S.H[at >> 5], 1u << (at & 31));
+            }
         });
         g.sync();
         const uint32_t cut = g.uniform(S.cut);
-        const int T = cut == ~0u ? total : (int)(cut >> 10);
-        const int next = cut != ~0u ? (int)(cut & 1023u) : last >= STOP ? (int)(last & ~STOP) : (int)last;
+        const int T = cut == ~0u ? total : (int)(cut >> 11);
+        const int next = cut != ~0u ? (int)(cut & 2047u) : last >= STOP ? (int)(last & ~STOP) : (int)last;
         if (T == 0) {
             // one sequence by decode_block's rules, read through `byte` and
             // copied by all threads; its sources are in the output itself

@@ -559,8 +559,8 @@ struct WideGroup {
     __device__ void min(uint32_t *p, uint32_t v) { atomicMin(p, v); }
     __device__ void or_(uint32_t *p, uint32_t v) { atomicOr(p, v); }
     // the sequences on the chain from the wave's entry
-    __device__ void chain(Reg<uint32_t> &nx, Reg<int> &entry, Reg<uint64_t> &mask) {
-        const int seg = __builtin_amdgcn_readfirstlane(t & ~63);
+    __device__ void chain(Reg<uint32_t> &nx, Reg<int> &entry, Reg<uint64_t> &mask, int base) {
+        const int seg = __builtin_amdgcn_readfirstlane(t & ~63) + base;
         uint64_t m = 0;
         for (int at = __builtin_amdgcn_readfirstlane(entry.v); at >= 0 && at < 64;) {
             const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)nx.v, at);
@@ -586,9 +586,10 @@ struct WideGroup {
         before.v = s - v;
         if ((t & 63) == 63) sums[t >> 6] = (uint32_t)s;
     }
-    __device__ int waves_before(int, const uint32_t *sums, int &total) {
-        constexpr int NW = fsg_lz4::WT / 64;
-        const int s = inclusive((t & 63) < NW ? (int)sums[t & 63] : 0), wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    __device__ int waves_before(int, int c, const uint32_t *sums, int &total) {
+        constexpr int NW = fsg_lz4::WIN / 64;
+        const int s = inclusive((t & 63) < NW ? (int)sums[t & 63] : 0);
+        const int wv = __builtin_amdgcn_readfirstlane(t >> 6) + c * (fsg_lz4::WT / 64);
         total = __builtin_amdgcn_readlane(s, NW - 1);
         return wv ? __builtin_amdgcn_readlane(s, wv - 1) : 0;
     }
@@ -604,9 +605,9 @@ struct WideGroup {
     }
 };
 
-// A workgroup per block (fsg_lz4_wide.hpp): about 22 000 cycles a batch of 1 KB of
-// block, a third of them the output bytes' lookups (VALU issue), a sixth the
-// barriers, the rest LDS latency of the parse and the chains.
+// A workgroup per block (fsg_lz4_wide.hpp): a third of the time is the output
+// bytes' lookups (VALU issue), a sixth the barriers, the rest LDS latency of the
+// parse and the chains.
 __global__ __launch_bounds__(fsg_lz4::WT) void k_pack_decode_wide(const uint8_t *in, const DecDesc *desc, uint8_t *out,
                                                                   int32_t *result) {
     __shared__ __align__(16) fsg_lz4::WideLds S;
@@ -619,8 +620,8 @@ __global__ __launch_bounds__(fsg_lz4::WT) void k_pack_decode_wide(const uint8_t 
 
 // A workgroup per block up to six blocks per compute unit (two at a time are
 // resident, and half of an unpack's blocks are short), else a wave per block.
-// Unpack of 1 chunk 3.3 ms by waves, 1.1 by workgroups; of 256 (512 blocks) 3.7
-// and 1.3; of 576 3.8 and 2.8; of 1024 3.8 and 4.1, as a workgroup does more
+// Unpack of 1 chunk 3.3 ms by waves, 1.0 by workgroups; of 256 (512 blocks) 3.7
+// and 1.1; of 576 3.8 and 2.7; of 1024 3.8 and 4.1, as a workgroup does more
 // work for a block than a wave.
 void launch_decode(const fsg_ctx *c, const uint8_t *in, const DecDesc *desc, uint8_t *out, int32_t *result, int n) {
     if (n <= 6 * c->n_cu)

@@ -21,10 +21,10 @@ struct HostGroup {
     uint32_t uniform(uint32_t x) { return x; }
     void min(uint32_t *p, uint32_t v) { *p = v < *p ? v : *p; }
     void or_(uint32_t *p, uint32_t v) { *p |= v; }
-    void chain(Reg<uint32_t> &nx, Reg<int> &entry, Reg<uint64_t> &mask) {
+    void chain(Reg<uint32_t> &nx, Reg<int> &entry, Reg<uint64_t> &mask, int base) {
         for (int seg = 0; seg < N; seg += 64) {
             uint64_t m = 0;
-            for (int at = entry[seg]; at >= 0 && at < 64 && nx[seg + at] != fsg_lz4::STOP; at = (int)nx[seg + at] - seg)
+            for (int at = entry[seg]; at >= 0 && at < 64 && nx[seg + at] != fsg_lz4::STOP; at = (int)nx[seg + at] - seg - base)
                 m |= 1ull << at;
             for (int k = 0; k < 64; k++) mask[seg + k] = m;
         }
@@ -38,11 +38,11 @@ struct HostGroup {
             sums[t >> 6] = (uint32_t)s;
         }
     }
-    int waves_before(int t, const uint32_t *sums, int &total) {
+    int waves_before(int t, int c, const uint32_t *sums, int &total) {
         int before = 0;
         total = 0;
-        for (int w = 0; w < N / 64; w++) {
-            if (w == (t >> 6)) before = total;
+        for (int w = 0; w < fsg_lz4::WIN / 64; w++) {
+            if (w == c * (N / 64) + (t >> 6)) before = total;
             total += (int)sums[w];
         }
         return before;
