@@ -1296,10 +1296,6 @@ int batch_prepare(fsg_ctx *c, fsg_world *const *ws, int n, bool *graph_ok) {
     const std::vector<fsg_world *> key(ws, ws + n);
     *graph_ok = c->graph && key == c->graph_key && start == c->graph_tiles && c->graph_ticks == c->tune.graph_ticks &&
                 c->graph_occ == c->tune.occupancy && c->graph_form == c->batch_form;
-    if (!*graph_ok) {
-        c->graph_key = key;
-        c->graph_tiles = start;
-    }
     c->total_tiles = (uint32_t)total;
     return FSG_OK;
 }
@@ -1327,6 +1323,7 @@ int batch_run(fsg_ctx *c, fsg_world *const *ws, int n, int ticks, bool graph_ok)
         if (!graph_ok) {
             if (c->graph) (void)hipGraphExecDestroy(c->graph);
             c->graph = nullptr;
+            c->graph_key.clear();
             hipGraph_t g;
             HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             for (int k = 0; k < T; k++) tick_launch((uint32_t)k);
@@ -1338,6 +1335,10 @@ int batch_run(fsg_ctx *c, fsg_world *const *ws, int n, int ticks, bool graph_ok)
                 c->graph = nullptr;
                 return FSG_ERR_DEVICE;
             }
+            // what the graph was captured with, noted here only: a batch of
+            // fewer ticks runs without one and must leave the key as it is
+            c->graph_key.assign(ws, ws + n);
+            c->graph_tiles.assign(c->h_tile_start, c->h_tile_start + n + 1);
             c->graph_ticks = T;
             c->graph_occ = c->tune.occupancy;
             c->graph_form = c->batch_form;

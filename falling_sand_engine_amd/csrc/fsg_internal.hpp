@@ -47,6 +47,7 @@ struct fsg_ctx {
     uint32_t *h_tile_start = nullptr;
     hipEvent_t staged = nullptr;
     bool staged_pending = false;
+    // the worlds and chunk prefix sums the cached graph was captured with
     std::vector<fsg_world *> graph_key;
     std::vector<uint32_t> graph_tiles;
     hipGraphExec_t graph = nullptr;

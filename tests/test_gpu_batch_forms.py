@@ -57,3 +57,29 @@ def test_batch_form_changes_between_calls(ctx):
             assert np.array_equal(a.download(), b.download()), (zone, a.width)
     for w in together + alone:
         w.close()
+
+
+@pytest.mark.parametrize("first,second", [(SIZES[:2], SIZES[2:]), (SIZES, SIZES[:1])])  # more worlds then, and fewer
+@pytest.mark.parametrize("skip", [0, 1])
+def test_a_batch_too_short_for_a_graph_leaves_the_cached_one_alone(ctx, first, second, skip):
+    """A graph captured over one set of worlds is not replayed for another set
+    whose last call had fewer ticks than a graph has."""
+    print(f"graph of {len(first)} worlds, then {len(second)} others, skip={skip}", flush=True)
+    a, b, alone = (batch_of(ctx, (skip,), (1,), False, s) for s in (first, second, second))
+    fsg.batch_step(ctx, a, 16)
+    for n in (5, 16, 33):
+        fsg.batch_step(ctx, b, n)
+        for w in alone:
+            w.tick(n)
+        for x, y in zip(b, alone):
+            assert np.array_equal(x.download(), y.download()), (n, x.width, x.height)
+    ref = [w.download() for w in a]
+    for w in b:
+        w.close()
+    fsg.batch_step(ctx, a, 16)  # the first set's own graph or a new one
+    again = batch_of(ctx, (skip,), (1,), False, first)
+    fsg.batch_step(ctx, again, 32)
+    for x, y, r in zip(a, again, ref):
+        assert not np.array_equal(r, x.download()) and np.array_equal(x.download(), y.download())
+    for w in a + alone + again:
+        w.close()
