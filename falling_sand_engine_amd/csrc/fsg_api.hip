@@ -174,17 +174,29 @@ int copy_out(fsg_ctx *c, std::initializer_list<CopyOut> parts) {
 
 // Whole rows are one copy.  A narrower rectangle is gathered on the device
 // first: the runtime's rectangle copy costs 3.3 ms whatever its size (a 64x64
-// page of getTile's mirror 3.5 ms, now 0.02).
+// page of getTile's mirror 3.5 ms, now 0.02).  The gather goes by bands of rows
+// of at most RECT_BAND bytes, so a download never needs more device memory than
+// that, and without even that the rectangle copy is used.
+constexpr size_t RECT_BAND = (size_t)64 << 20;
 template <typename T>
 int copy_rect_out(fsg_ctx *c, T *dst, const T *src, size_t pitch, int rw, int rh) {
-    const size_t n = (size_t)rw * (size_t)rh;
-    if ((size_t)rw == pitch || rh == 1) return copy_out(c, {{dst, src, n * sizeof(T)}});
+    const size_t row = (size_t)rw * sizeof(T);
+    if ((size_t)rw == pitch || rh == 1) return copy_out(c, {{dst, src, row * (size_t)rh}});
+    const int band = (int)std::min<size_t>((size_t)rh, std::max<size_t>(RECT_BAND / row, 1));
     void *tmp = nullptr;
-    if (dev_alloc(c, &tmp, n * sizeof(T))) return FSG_ERR_NOMEM;
-    fsg::k_gather_rect<T><<<dim3((unsigned)((rw + 255) / 256), (unsigned)std::min(rh, 65535)), 256, 0, c->stream>>>(
-        src, pitch, rw, rh, static_cast<T *>(tmp));
-    int rc = hipGetLastError() == hipSuccess ? FSG_OK : FSG_ERR_DEVICE;
-    if (!rc) rc = copy_out(c, {{dst, tmp, n * sizeof(T)}});
+    if (dev_alloc(c, &tmp, row * (size_t)band)) {
+        HIPCHK(hipMemcpy2DAsync(dst, row, src, pitch * sizeof(T), row, (size_t)rh, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        return FSG_OK;
+    }
+    int rc = FSG_OK;
+    for (int y = 0; y < rh && !rc; y += band) {
+        const int n = std::min(band, rh - y);
+        fsg::k_gather_rect<T><<<dim3((unsigned)((rw + 255) / 256), (unsigned)std::min(n, 65535)), 256, 0, c->stream>>>(
+            src + (size_t)y * pitch, pitch, rw, n, static_cast<T *>(tmp));
+        rc = hipGetLastError() == hipSuccess ? FSG_OK : FSG_ERR_DEVICE;
+        if (!rc) rc = copy_out(c, {{dst + (size_t)y * (size_t)rw, tmp, row * (size_t)n}});
+    }
     dev_free(tmp);
     return rc;
 }

@@ -49,3 +49,33 @@ def test_uploads_in_flight(ctx, n):
             fsg.check(fsg.lib().fsg_world_set_cells(w.handle, arr, n))
             ref.ravel()[at] = vals
         assert np.array_equal(w.download(), ref)
+
+
+def test_rectangles_without_device_memory(ctx):
+    """A download of part of a world succeeds when no device memory can be had
+    for it."""
+    W, H = 300, 200
+    cells = cells_of(W, H, 3)
+    with fsg.World(ctx, W, H, 0) as w:
+        w.upload(cells)
+        w.render()
+        layer = w.layer(fsg.LAYER_CELLS)
+        for x0, y0, rw, rh in [(0, 0, 299, 200), (17, 50, 200, 120), (299, 0, 1, 200)]:
+            print(f"rectangle {x0},{y0} {rw}x{rh} without device memory", flush=True)
+            try:
+                ctx.inject_alloc_failures(1)
+                assert np.array_equal(w.download(x0, y0, rw, rh), cells[y0:y0 + rh, x0:x0 + rw])
+                ctx.inject_alloc_failures(1)
+                assert np.array_equal(w.layer(fsg.LAYER_CELLS, x0, y0, rw, rh), layer[y0:y0 + rh, x0:x0 + rw])
+            finally:
+                ctx.inject_alloc_failures(0)
+
+
+@pytest.mark.parametrize("rw,rh", [(4095, 2049), (4095, 4096), (2047, 4096)])  # bands of 2,048 and 4,098 rows
+def test_rectangles_of_several_bands(ctx, rw, rh):
+    W = H = 4096
+    cells = cells_of(W, H, 4)
+    with fsg.World(ctx, W, H, 0) as w:
+        w.upload(cells)
+        print(f"rectangle {rw}x{rh}", flush=True)
+        assert np.array_equal(w.download(1, H - rh, rw, rh), cells[H - rh:, 1:1 + rw])
