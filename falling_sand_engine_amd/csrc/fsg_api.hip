@@ -119,6 +119,7 @@ int copy_in(fsg_ctx *c, void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return FSG_OK;
     if (bytes > fsg_ctx::STAGE) {
         HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));  // the source may go when this returns
         return FSG_OK;
     }
     std::lock_guard<std::mutex> lk(c->stage_in_mu);
@@ -628,10 +629,10 @@ extern "C" int fsg_world_create(fsg_ctx *c, int W, int H, uint64_t seed, const f
     fill_pair_table(w->d);
     w->d.ct = nullptr;
     if (conf.n_materials <= 8) {
-        w->ct_host = class_tables(w->d);  // kept until the world goes (the copy is asynchronous)
-        if (dev_alloc(c, &p, w->ct_host.size() * 4)) return fail(FSG_ERR_NOMEM);
+        const std::vector<uint32_t> ct = class_tables(w->d);
+        if (dev_alloc(c, &p, ct.size() * 4)) return fail(FSG_ERR_NOMEM);
         w->d.ct = (const uint32_t *)p;
-        if (copy_in(c, p, w->ct_host.data(), w->ct_host.size() * 4)) return fail(FSG_ERR_DEVICE);
+        if (copy_in(c, p, ct.data(), ct.size() * 4)) return fail(FSG_ERR_DEVICE);
     }
     const uint64_t air = conf.mat_air;
     fsg::k_fill<<<grid_for(cells, 256), 256, 0, c->stream>>>(w->d.buf[0], cells, air);
@@ -1062,8 +1063,7 @@ int ensure_stamp_buffers(fsg_world *w, size_t npix, int nb) {
 }
 
 // Validates bodies/pixels and uploads them; the pixel -> body map is made on
-// the device.  Pixels beyond fsg_ctx::STAGE bytes must stay valid until the
-// stream is synchronised.  `zero`: result words to clear on the way.
+// the device.  `zero`: result words to clear on the way.
 int set_bodies(fsg_world *w, const fsg_body *bodies, int nb, const fsg_cell *pixels, size_t npix, uint32_t *zero,
                uint32_t nzero) {
     if (npix >= 0xFFFFFFFFull) return FSG_ERR_INVALID;

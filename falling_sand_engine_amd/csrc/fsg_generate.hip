@@ -162,11 +162,10 @@ extern "C" int fsg_world_generate(fsg_world *w, int kind, uint64_t seed) {
         }
         int32_t *d_h = static_cast<int32_t *>(w->d_gen);
         fsg_gen_disc *d_d = reinterpret_cast<fsg_gen_disc *>(static_cast<char *>(w->d_gen) + b_h);
-        w->gen_discs = std::move(discs);  // the host copy outlives the asynchronous upload
-        if (int rc = fsg_impl::copy_in(c, d_d, w->gen_discs.data(), b_d)) return rc;
+        if (int rc = fsg_impl::copy_in(c, d_d, discs.data(), b_d)) return rc;
         k_gen_heights<<<fsg_impl::grid_for((size_t)W, 256), 256, 0, c->stream>>>(W, H, seed, d_h);
         k_gen_basin<<<(unsigned)(w->d.tiles_x * w->d.tiles_y), GT, 0, c->stream>>>(
-            cur, W, H, g, d_h, d_d, (int)w->gen_discs.size(), w->d.tiles_x);
+            cur, W, H, g, d_h, d_d, (int)discs.size(), w->d.tiles_x);
         HIPCHK(hipGetLastError());
     }
     // a new grid, as after fsg_world_upload

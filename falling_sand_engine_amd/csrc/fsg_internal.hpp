@@ -96,7 +96,6 @@ struct fsg_world {
     // tick) or for any tick (list_any: both zero)
     bool list_any = true;
     uint64_t list_next = 0;
-    std::vector<uint32_t> ct_host;  // host copy of the class tables (DevWorld::ct)
     uint32_t *d_layer[3] = {nullptr, nullptr, nullptr};  // texture layers (fsg_world_render)
     unsigned long long *d_tally = nullptr;                 // render census replicas
     void *d_isl = nullptr;                                 // island check scratch
@@ -105,7 +104,6 @@ struct fsg_world {
     size_t isl_pix_cap = 0, isl_pix_used = 0;
     void *d_gen = nullptr;                                 // device generator scratch
     size_t gen_cap = 0;
-    std::vector<fsg_gen_disc> gen_discs;                   // host copy of the last disc upload
     // chunk .pack codec (fsg_pack.hip): encoder slots, assembled images, sizes/offsets,
     // layer2/background upload, decoder input, record staging, descriptors/statuses
     void *d_pack_slots = nullptr, *d_pack_img = nullptr, *d_pack_small = nullptr, *d_pack_aux = nullptr;
@@ -175,7 +173,7 @@ void dev_free(void *p);
 void trim_cache(fsg_ctx *c, size_t keep);  // hipFree cached blocks down to `keep` bytes
 unsigned grid_for(size_t n, unsigned block);
 // Host -> device copy in stream order; the source may change when it returns
-// if bytes <= fsg_ctx::STAGE, else only once the stream has been synchronised.
+// (waits for a copy of more than fsg_ctx::STAGE bytes).
 int copy_in(fsg_ctx *c, void *dst, const void *src, size_t bytes);
 // Device -> host copies, behind everything on the stream; waits for them.
 struct CopyOut {

@@ -971,9 +971,7 @@ extern "C" int fsg_world_particles_add(fsg_world *w, const fsg_particle *p, size
     fsg_ctx *c = w->ctx;
     HIPCHK(hipSetDevice(c->device));
     if (int rc = grow_lists(w, w->npart + n)) return rc;
-    const size_t bytes = n * sizeof(fsg_particle);
-    if (int rc = fsg_impl::copy_in(c, w->d_part + w->npart, p, bytes)) return rc;
-    if (bytes > fsg_ctx::STAGE) HIPCHK(hipStreamSynchronize(c->stream));
+    if (int rc = fsg_impl::copy_in(c, w->d_part + w->npart, p, n * sizeof(fsg_particle))) return rc;
     w->npart += n;
     return FSG_OK;
 }

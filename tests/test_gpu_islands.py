@@ -91,3 +91,23 @@ def test_ticks_after_a_check_stay_bit_exact(ctx, orc, skip):
     assert got[0]["status"] == _abi.ISLAND_BODY and got[1]["status"] == _abi.ISLAND_REMOVED
     orc.run(c_ref, cfg, 7, 30, 30)
     assert np.array_equal(grid, c_ref)
+
+
+def test_more_kept_islands_than_the_upload_staging_holds(ctx, orc):
+    """40,000 islands removed by one call: their list (1.28 MB) is past the
+    staging's 1 MiB, so the call's own memory is what the device copy reads."""
+    W = H = 400
+    c = np.full((H, W), fsg.make_cell(fsg.MAT_AIR, 320, 0), np.uint64)
+    c[::2, ::2] = fsg.make_cell(fsg.MAT_STONE, 300, 0xFF445566)
+    seeds = [(x, y) for y in range(0, H, 2) for x in range(0, W, 2)]
+    cfg = orc.default_config()
+    print(f"islands {len(seeds)} in one call", flush=True)
+    with fsg.World(ctx, W, H, 1, cfg) as w:
+        w.upload(c)
+        got = w.physicsCheck(seeds)
+        junk = [np.full(1 << 18, 0xAB, np.uint8) for _ in range(64)]  # memory the call gave back, in use again
+        grid = w.download()
+    del junk
+    compare(got, orc.physics_check(c, cfg, seeds))
+    assert np.array_equal(grid, c)
+    assert not np.any(grid & np.uint64(0xFF))
