@@ -64,10 +64,16 @@ size_t size_class(size_t bytes) {
     return (bytes + step - 1) & ~(step - 1);
 }
 
+// True if an injected failure is due.
+static bool take_injected(fsg_ctx *c) {
+    for (int k = c->inject.load(); k > 0;)
+        if (c->inject.compare_exchange_weak(k, k - 1)) return true;
+    return false;
+}
+
 int dev_alloc(fsg_ctx *c, void **p, size_t bytes) {
     *p = nullptr;
-    for (int k = c->inject.load(); k > 0;)
-        if (c->inject.compare_exchange_weak(k, k - 1)) return FSG_ERR_NOMEM;
+    if (take_injected(c)) return FSG_ERR_NOMEM;
     if (bytes == 0) bytes = 8;
     bytes = size_class(bytes);
     {
@@ -111,22 +117,31 @@ void dev_free(void *p) {
     if (c->cached > c->cache_cap) trim_cache_locked(c, c->cache_cap);
 }
 
+// Pinned staging, allocated at first use; null if it cannot be had, and then
+// the copies go without it.
+static char *staging(fsg_ctx *c, char *&at, size_t bytes) {
+    if (at) return at;
+    if (take_injected(c)) return nullptr;
+    void *p = nullptr;
+    if (hipHostMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return at = static_cast<char *>(p);
+}
+
 // A copy from or to pageable memory below 1 MiB goes through the runtime's own
 // staging in small pieces (512 KiB: 213 us in, 233 us out; 64 KiB: 35 and 37);
 // through pinned memory and one memcpy it takes 30 and 30 (9 and 11).  Larger
 // ones are pinned in place by the runtime and gain nothing from a second copy.
 int copy_in(fsg_ctx *c, void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return FSG_OK;
-    if (bytes > fsg_ctx::STAGE) {
+    std::unique_lock<std::mutex> lk(c->stage_in_mu, std::defer_lock);
+    if (bytes <= fsg_ctx::STAGE) lk.lock();
+    if (!lk || !staging(c, c->h_in, fsg_ctx::IN_SLOTS * fsg_ctx::STAGE)) {
         HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));  // the source may go when this returns
         return FSG_OK;
-    }
-    std::lock_guard<std::mutex> lk(c->stage_in_mu);
-    if (!c->h_in) {
-        void *p;
-        if (hipHostMalloc(&p, fsg_ctx::IN_SLOTS * fsg_ctx::STAGE) != hipSuccess) return FSG_ERR_NOMEM;
-        c->h_in = static_cast<char *>(p);
     }
     if (c->in_used + bytes > fsg_ctx::STAGE) {  // the next slot, once its uploads are over
         HIPCHK(hipEventRecord(c->in_ev[c->in_slot], c->stream));
@@ -147,17 +162,13 @@ int copy_in(fsg_ctx *c, void *dst, const void *src, size_t bytes) {
 int copy_out(fsg_ctx *c, std::initializer_list<CopyOut> parts) {
     size_t total = 0;
     for (const CopyOut &p : parts) total += p.bytes;
-    if (total > fsg_ctx::STAGE) {
+    std::unique_lock<std::mutex> lk(c->stage_out_mu, std::defer_lock);
+    if (total <= fsg_ctx::STAGE) lk.lock();
+    if (!lk || !staging(c, c->h_out, fsg_ctx::STAGE)) {
         for (const CopyOut &p : parts)
             if (p.bytes) HIPCHK(hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(hipStreamSynchronize(c->stream));
         return FSG_OK;
-    }
-    std::lock_guard<std::mutex> lk(c->stage_out_mu);
-    if (!c->h_out) {
-        void *p;
-        if (hipHostMalloc(&p, fsg_ctx::STAGE) != hipSuccess) return FSG_ERR_NOMEM;
-        c->h_out = static_cast<char *>(p);
     }
     size_t o = 0;
     for (const CopyOut &p : parts) {

@@ -136,7 +136,8 @@ int fsg_ctx_create(const fsg_ctx_config *cfg, fsg_ctx **out);
 int fsg_ctx_destroy(fsg_ctx *ctx);
 /* Bytes of world state currently held by the context. */
 int fsg_ctx_usage(fsg_ctx *ctx, uint64_t *bytes_used);
-/* Test hook: make the next n device allocations of this ctx fail. */
+/* Test hook: make the next n allocations of this ctx (device memory, pinned
+ * staging) fail. */
 int fsg_ctx_inject_alloc_failures(fsg_ctx *ctx, int n);
 /* Plain device-to-device copy of `bytes` bytes by a streaming kernel, timed
  * with HIP events (ms = mean over `reps`).  It has no counterpart in the

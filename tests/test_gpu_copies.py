@@ -79,3 +79,27 @@ def test_rectangles_of_several_bands(ctx, rw, rh):
         w.upload(cells)
         print(f"rectangle {rw}x{rh}", flush=True)
         assert np.array_equal(w.download(1, H - rh, rw, rh), cells[H - rh:, 1:1 + rw])
+
+
+def test_copies_without_pinned_memory():
+    """Small uploads and downloads succeed when the pinned staging cannot be
+    had, and use it once it can."""
+    W, H = 200, 100
+    cells = cells_of(W, H, 6)
+    cfg = fsg.default_config()
+    cfg.n_materials = 9  # no class tables, whose upload would take the staging at creation
+    cfg.materials[8] = cfg.materials[fsg.MAT_STONE]
+    ps = [fsg.make_particle(fsg.make_cell(fsg.MAT_SAND, 320, i), 5.0 + i % 90, 5.0, 0.0, 0.0) for i in range(20000)]
+    with fsg.Context(0) as c, fsg.World(c, W, H, 0, cfg) as w:
+        w.upload(cells)
+        w.particles_add(ps)  # 1.1 MB each: past the staging's size
+        w.particles_add(ps[:19000])  # (and the list grows to 40,000)
+        for fails in (1, 0):
+            print(f"staging fails={fails}", flush=True)
+            c.inject_alloc_failures(fails)
+            w.particles_add(ps[:10])  # staged up; the list has room
+            c.inject_alloc_failures(fails)
+            assert np.array_equal(w.download(), cells)
+            c.inject_alloc_failures(0)
+        got = w.particles()
+        assert [(p.x, p.tile.rgba) for p in got] == [(p.x, p.tile.rgba) for p in ps + ps[:19000] + ps[:10] + ps[:10]]
