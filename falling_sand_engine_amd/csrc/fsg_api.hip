@@ -1124,11 +1124,11 @@ extern "C" int fsg_world_stamp_bodies(fsg_world *w, const fsg_body *bodies, int 
     // 110,000 pixels: a stamp took 0.81 ms while 17 bytes per pixel came back
     // and the host walked them, and a 4-byte body map went up; now 0.25)
     fsg::StampRes r{};
-    const size_t words = 4 + 2 * (size_t)nb, blocks = grid_for(npix, 256);
+    const size_t words = 4 + 2 * (size_t)nb, blocks = grid_for(npix, 256), groups = (blocks + 255) / 256;
     const uint32_t cap = res && res->displaced_out ? (uint32_t)std::min<size_t>(res->displaced_cap, npix) : 0u;
     if (res && npix) {
         HIPCHK(hipSetDevice(c->device));
-        const size_t head = ((words + blocks) * 4 + 15) & ~(size_t)15, need = head + (size_t)cap * sizeof(fsg_cell_edit);
+        const size_t head = ((words + groups + blocks) * 4 + 15) & ~(size_t)15, need = head + (size_t)cap * sizeof(fsg_cell_edit);
         if (w->sres_cap < need) {
             dev_free(w->d_sres);
             w->d_sres = nullptr;
@@ -1138,12 +1138,13 @@ extern "C" int fsg_world_stamp_bodies(fsg_world *w, const fsg_body *bodies, int 
         }
         r.count = static_cast<uint32_t *>(w->d_sres);
         r.hits = r.count + 4;
-        r.block = r.count + words;
+        r.group = r.count + words;
+        r.block = r.group + groups;
         r.list = reinterpret_cast<fsg_cell_edit *>(static_cast<char *>(w->d_sres) + head);
         r.nb = (uint32_t)nb;
         r.cap = cap;
     }
-    if (int rc = set_bodies(w, bodies, nb, pixels, npix, r.count, r.count ? (uint32_t)words : 0u)) return rc;
+    if (int rc = set_bodies(w, bodies, nb, pixels, npix, r.count, r.count ? (uint32_t)(words + groups) : 0u)) return rc;
     if (npix)
         if (int rc = stamp_single(w, false, r)) return rc;
     std::vector<uint32_t> h(words, 0u);

@@ -38,6 +38,7 @@ struct StampRes {
     uint32_t *count;           // [0] placed, [1] unplaced, [2] displaced
     uint32_t *hits;            // [nb] displaced SAND per body, then [nb] displaced SOUP
     uint32_t *block;           // displaced pixels per workgroup of k_claims_restore
+    uint32_t *group;           // and per 256 of them (zero on entry)
     fsg_cell_edit *list;       // displaced cells in pixel order, at most cap
     uint32_t nb, cap;
 };

@@ -66,3 +66,29 @@ def test_overlapping_bodies_refused(ctx):
             assert e.value.status == -1
         assert w.stamp_bodies(ok, px)["placed"] > 0
         w.unstamp_bodies(px.size)
+
+
+@pytest.mark.parametrize("cap", [1000, 400000])
+def test_displaced_list_of_many_workgroups(ctx, orc, cap):
+    """Three bodies of 100,000 pixels over sand and water: 1,172 workgroups
+    count them, in groups of 256."""
+    W, H = 900, 700
+    cells = np.full((H, W), fsg.make_cell(fsg.MAT_SAND, 320, 5), np.uint64)
+    cells[:, ::3] = fsg.make_cell(fsg.MAT_AIR, 320, 0)
+    cells[::7] = fsg.make_cell(fsg.MAT_WATER, 320, 6)
+    rng = np.random.default_rng(1)
+    px = np.full(300000, fsg.make_cell(fsg.MAT_STONE, 320, 7), np.uint64)
+    px[rng.random(px.size) < 0.2] = 0
+    px[100000:170000] = 0  # (workgroups and a whole group with none displaced)
+    bodies = [fsg.body_from_pose(250 + 180 * k, 200 + 150 * k, 0.3 * k, 400, 250, 100000 * k) for k in range(3)]
+    cfg = orc.default_config()
+    print(f"stamp 300,000 pixels cap={cap}", flush=True)
+    ref = cells.copy()
+    rs = orc.stamp(ref, cfg, bodies, px, displaced_cap=cap)
+    with fsg.World(ctx, W, H, 3, cfg) as w:
+        w.upload(cells)
+        gs = w.stamp_bodies(bodies, px, displaced_cap=cap)
+        assert np.array_equal(w.download(), ref)
+    assert rs["displaced"] > 65536 and len(gs["displaced_cells"]) == min(cap, rs["displaced"])
+    for k in ("placed", "displaced", "hits_sand", "hits_soup", "displaced_cells"):
+        assert gs[k] == rs[k], k
