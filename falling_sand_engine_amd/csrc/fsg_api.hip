@@ -982,10 +982,18 @@ int stamp_rounds(fsg_ctx *c, const fsg::StampWorld *d_table, int n, uint32_t tot
     const int resolve = unstamp ? fsg::OP_UNRESOLVE : fsg::OP_RESOLVE;
     const dim3 g(grid_for(max_npix, 256), (unsigned)n);  // y: world, x: its pixels
     // every target slot is cleared up front; with save its old contents are
-    // copied out first and put back after the last round
-    fsg::k_claims_init<<<g, 256, 0, c->stream>>>(a, save ? 1 : 0);
+    // taken out first and put back after the last round.  By exchanges that is
+    // one launch, but they cost more than a read and a write: unstamp of 62,500
+    // pixels 100 us by exchange, 105 by copy; 98,000 128 and 128; 393,000 357
+    // and 325; 1.6 M 1,161 and 1,084 (of the kernels 264 and 123).
+    const fsg::ClaimSave how = !save ? fsg::SAVE_NONE : total <= 1u << 16 ? fsg::SAVE_EXCHANGE : fsg::SAVE_COPY;
+    fsg::k_claims_init<<<g, 256, 0, c->stream>>>(a, how);
+    if (how == fsg::SAVE_COPY) fsg::k_claims_clear<<<g, 256, 0, c->stream>>>(a);
     fsg::k_stamp_step<<<g, 256, 0, c->stream>>>(a, propose, 0);
-    if (total <= 1u << 20) {  // up to 4,096 reservations of the open list, by the resolve itself
+    // the open list's reservations, one per 256 pixels, are the resolve's own
+    // while they are few (unstamp, so / by k_stamp_compact: 10,000 pixels 80 /
+    // 90 us, 250,000 212 / 219; 393,000 331 / 320, 467,000 375 / 361)
+    if (total <= 1u << 18) {
         fsg::k_stamp_resolve0<<<g, 256, 0, c->stream>>>(a, resolve);
     } else {
         fsg::k_stamp_step<<<g, 256, 0, c->stream>>>(a, resolve, 0);

@@ -1418,9 +1418,10 @@ __device__ __forceinline__ void mark_tiles_wave(uint32_t *flags, bool on, uint32
 // the atomicMin to the earlier round's claim still in the slot -- so the
 // earliest round and then the lowest pixel win, as a round-by-round pass
 // over the pixels gives.  With save the slots' contents (the state before
-// the last tick) are taken out by the exchange that clears them: of the
-// pixels sharing a slot one gets its cell and the others ~0, which no cell
-// is; k_claims_restore puts the cells back.
+// the last tick) are first taken out: by the exchange that clears them, where
+// of the pixels sharing a slot one gets its cell and the others ~0, which no
+// cell is; or by a copy, and then k_claims_clear clears them in a launch of its
+// own, after every copy.  k_claims_restore puts the cells back.
 __device__ __forceinline__ void slot_at(const StampWorld &W, uint64_t t, int d, bool live, bool &on, int &wx,
                                         int &wy) {
     wx = (int)(uint32_t)t + kDX[d];
@@ -1445,11 +1446,30 @@ __global__ void k_claims_init(StampArgs a, int save) {
         int wx, wy;
         slot_at(W, t, d, live, on, wx, wy);
         uint64_t *slot = &W.claims[(size_t)wy * W.W + wx];
-        if (on && save) {
+        if (save == SAVE_COPY) {
+            if (on) W.save[5 * (size_t)p + d] = *slot;
+            continue;
+        }
+        if (on && save == SAVE_EXCHANGE) {
             W.save[5 * (size_t)p + d] = atomicExch(reinterpret_cast<unsigned long long *>(slot), ~0ull);
         } else if (on) {
             *slot = ~0ull;
         }
+        if (W.flags) mark_tiles_wave(W.flags, on, on ? (uint32_t)((wy / TH) * W.tiles_x + wx / TW) : 0u);
+    }
+}
+
+__global__ void k_claims_clear(StampArgs a) {
+    const StampWorld &W = a.worlds[blockIdx.y];
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool in = p < W.npix;
+    const uint64_t t = in ? W.tgt[p] : NOT_LIVE;
+    const bool live = in && (uint32_t)t != NOT_LIVE;
+    for (int d = 0; d < 5; d++) {
+        bool on;
+        int wx, wy;
+        slot_at(W, t, d, live, on, wx, wy);
+        if (on) W.claims[(size_t)wy * W.W + wx] = ~0ull;
         if (W.flags) mark_tiles_wave(W.flags, on, on ? (uint32_t)((wy / TH) * W.tiles_x + wx / TW) : 0u);
     }
 }

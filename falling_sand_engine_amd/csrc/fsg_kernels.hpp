@@ -72,7 +72,10 @@ __global__ void k_set_cells(uint64_t *cells, int W, int H, const int32_t *xy, co
 // and `zero` words of zeroed result.
 __global__ void k_pix_body(const fsg_body *bodies, const uint32_t *order, uint32_t nb, uint32_t npix,
                            uint32_t *pix_body, uint32_t *zero, uint32_t nzero);
+// What happens to the contents of the slots that are cleared.
+enum ClaimSave { SAVE_NONE, SAVE_EXCHANGE, SAVE_COPY /* k_claims_clear follows */ };
 __global__ void k_claims_init(StampArgs a, int save);
+__global__ void k_claims_clear(StampArgs a);
 __global__ void k_claims_restore(StampArgs a, StampRes r);
 __global__ void k_displaced(StampWorld W, StampRes r);
 // Per-pixel steps of a stamp claim round (k_stamp_step, k_stamp_step_list).

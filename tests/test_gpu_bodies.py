@@ -127,6 +127,38 @@ def test_tick_after_unstamp_and_census(ctx, orc):
     assert np.array_equal(got_after, after), int(np.count_nonzero(got_after != after))
 
 
+@pytest.mark.parametrize("npix", [(1 << 16), (1 << 16) + 1, (1 << 18), (1 << 18) + 1])
+def test_claim_slots_saved_by_exchange_and_by_copy(ctx, orc, npix):
+    """On either side of the pixel counts where the claim slots are saved
+    another way and the open pixels are listed another way (unused pixels
+    fill the array up): grid, pixels and the census of the spare buffer."""
+    W, H, seed = 640, 512, 21
+    rng = np.random.default_rng(seed)
+    cells = fsg.generate(2, W, H, seed)
+    bodies, used = random_bodies(rng, W, H, 150, max_side=28, mats=MIXED_MATS)
+    pixels = np.full(npix, fsg.make_cell(fsg.MAT_STONE, 100), np.uint64)
+    assert used.size < npix
+    pixels[:used.size] = used
+    cfg = orc.default_config(chunk_skip=1)
+    print(f"claim slots of {npix} pixels, {used.size} used", flush=True)
+    ref = cells.copy()
+    orc.stamp(ref, cfg, bodies, pixels)
+    pre_tick = ref.copy()
+    orc.run(ref, cfg, seed, 0, 1)
+    ref_px = orc.unstamp(ref, cfg, bodies, pixels)
+    _layers, ref_st = orc.render(ref, cfg, _render_params(), prev=pre_tick)
+    with fsg.World(ctx, W, H, seed, cfg) as w:
+        w.upload(cells)
+        w.stamp_bodies(bodies, pixels)
+        assert np.array_equal(w.download(), pre_tick)
+        w.tick(1)
+        got_px = w.unstamp_bodies(pixels.size)
+        st = w.render(fsg.LAYER_CELLS, stats=True)
+        assert np.array_equal(w.download(), ref)
+    assert np.array_equal(got_px, ref_px)
+    assert st["moved"] == [int(v) for v in ref_st.moved] and sum(st["moved"]) > 0
+
+
 def _render_params():
     from falling_sand_engine_amd._abi import RenderParams
     p = RenderParams()
