@@ -361,11 +361,19 @@ int launch_tick(fsg_world *w) {
         // of 512 15.0; 289 chunks of 512 threads 15.6, of 256 18.2; 484 of
         // 512 19.6, of 256 20.1, and 1024 of 512 27.2, of 256 24.5: with
         // more chunks per compute unit the wider workgroups take more rounds
-        const unsigned slots = (unsigned)(fsg::WGS_PER_CU - (zoned ? 1 : 0)) * cu, rest = tiles % slots;
+        // One phase a tick on a world that the last-level cache (256 MB) does
+        // not hold is bound by memory, and five workgroups per CU disturb each
+        // other's lines less than six: 5000x4200 67.7 us a tick by five, 69.0 by
+        // six, 6144x6000 117.9 and 120.9, 8192^2 199.2 and 204.2, all-active
+        // 198.1 and 201.8; 4096^2 49.4 and 46.8.  With two phases it depends on
+        // the cells (6144x6000 119.5 and 121.4, all-active 128.4 and 125.4).
+        const bool five = zoned || (w->d.mat.cell_iter == 1 && (size_t)w->d.W * w->d.H * 16 > (size_t)256 << 20);
+        const unsigned slots = (unsigned)(fsg::WGS_PER_CU - (five ? 1 : 0)) * cu, rest = tiles % slots;
         // whole chunks in full rounds of resident workgroups, a remainder of
-        // at most a quarter round as quarters, which then fill one round (a
-        // larger one as whole chunks: 4096^2 world, 1024 left over, 59 us a
-        // tick instead of 68)
+        // at most a quarter round as quarters, which then fill one round.  Left
+        // over from rounds of 1536, us a tick as quarters / whole: 32 29.9 /
+        // 32.2, 256 33.2 / 33.7, 384 35.6 / 35.2, 512 37.9 / 36.3, 1024 66.9 /
+        // 58.9; all-active 384 41.2 / 41.7, 448 42.6 / 42.6, 512 44.6 / 43.4
         const unsigned nfull = tiles <= slots || 4 * rest > slots ? tiles : tiles - rest;
         auto launch = [&](auto re_, auto zn_) {
             constexpr int R = decltype(re_)::value, Z = decltype(zn_)::value;
@@ -376,7 +384,8 @@ int launch_tick(fsg_world *w) {
             else if (tiles <= 2 * cu)
                 fsg::k_tick_small<0, R, Z, fsg::MEDIUM_NT><<<tiles, fsg::MEDIUM_NT, 0, st>>>(w->d, 0u);
             else
-                fsg::k_tick_world<R, Z><<<nfull + 4u * (tiles - nfull), fsg::NT, 0, st>>>(w->d, 0u, (int)nfull);
+                fsg::k_tick_world<R, Z><<<nfull + 4u * (tiles - nfull), fsg::NT, five && !Z ? fsg::FIVE_LDS : 0, st>>>(
+                    w->d, 0u, (int)nfull);
         };
         if (zoned) re ? launch(Yes{}, Yes{}) : launch(No{}, Yes{});
         else re ? launch(Yes{}, No{}) : launch(No{}, No{});

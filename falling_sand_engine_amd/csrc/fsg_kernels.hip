@@ -138,6 +138,7 @@ template <int N> struct TileLds {
     uint16_t queue[queue_end<N>(N / 64 - 1)];
 };
 static_assert(sizeof(TileLds<NT>) + 256 <= 26880, "six workgroups per CU");
+static_assert(sizeof(TileLds<NT>) + FIVE_LDS > 26880, "five with FIVE_LDS");
 
 // perm[y]: in byte k, the LDS offset (from the block's top-left cell) of the
 // place cell k goes to under scatter mask y, k ^ ((y >> 2k) & 3).
