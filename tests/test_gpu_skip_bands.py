@@ -48,3 +48,32 @@ def test_skip_forms_equal_oracle(ctx, orc, tx, ty, react, trim, zoned):
             ref[y, x] = fsg.make_cell(fsg.MAT_SAND, 320, 5)
         st = w.stats()
         assert zoned or tx * ty < 200 or st.tiles_processed < st.tiles_offered
+
+
+@pytest.mark.parametrize("zoned", [0, 1])
+def test_listed_world_across_jumps_and_batches(ctx, orc, zoned):
+    """2,561 chunks are the fewest whose awake ones are listed by tick parity:
+    ticks run by the batch path, or a jump of the tick counter by an odd or
+    even number, in between listed ticks."""
+    tx, ty = BANDS[-1]
+    cells = mostly_asleep(tx, ty, 0)
+    H, W = cells.shape
+    assert -(-W // 64) * -(-H // 64) == 2561
+    cfg = orc.default_config(chunk_skip=1)
+    zone = (W // 7, 0, W // 2, H - 70) if zoned else None
+    print(f"listed world across jumps zoned={zoned}", flush=True)
+    with fsg.World(ctx, W, H, 9, cfg) as w:
+        w.upload(cells)
+        if zone:
+            w.tickZone = zone
+        ref, t = cells, 0
+        for jump, how, n in ((0, "tick", 3), (0, "batch", 2), (0, "tick", 2), (0, "batch", 3), (0, "tick", 1),
+                             (51, "tick", 3), (30, "tick", 2), (0, "batch", 1), (7, "batch", 2), (1, "tick", 3)):
+            if jump:
+                t += jump
+                w.set_tick(t)
+            w.tick(n) if how == "tick" else fsg.batch_step(ctx, [w], n)
+            ref = orc.run(ref, cfg, 9, t, n, zone)
+            t += n
+            assert np.array_equal(w.download(), ref), (t, how)
+        assert zoned or w.stats().tiles_processed < w.stats().tiles_offered
