@@ -1553,10 +1553,16 @@ extern "C" int fsg_autotune_batch(fsg_ctx *c, fsg_world *const *ws, int n, int s
         for (int skip : {1, 0})
             for (int T : {16, 32, 8, 4, 1}) cand.push_back(fsg_tuning{T, skip, occ, 0});
     double best_ms = 1e30;
+    // batches of few chunks run kernels that have no second register budget:
+    // such a candidate has the time of the first one, so that the choice (which
+    // is cached for larger batches of its class too) is not left to noise
+    const size_t budgets = cand.size() / 2;
+    std::vector<char> one_budget(budgets, 0);
     for (size_t k = 0; k < cand.size() && !rc; k++) {
         c->tune = cand[k];
-        float f = 0.f;
-        for (int pass = 0; pass < 2 && !rc; pass++) {  // pass 0 builds the graph, pass 1 is timed
+        const bool twin = k >= budgets && one_budget[k - budgets];
+        float f = twin ? (float)r.ms[k - budgets] : 0.f;
+        for (int pass = twin ? 2 : 0; pass < 2 && !rc; pass++) {  // pass 0 builds the graph, pass 1 is timed
             for (int i = 0; i < n && !rc; i++) rc = copy_state(cl[i], ws[i]);
             bool graph_ok = false;
             if (!rc) rc = batch_prepare(c, cl.data(), n, &graph_ok);
@@ -1567,6 +1573,7 @@ extern "C" int fsg_autotune_batch(fsg_ctx *c, fsg_world *const *ws, int n, int s
                 rc = FSG_ERR_DEVICE;
         }
         if (rc) break;
+        if (k < budgets) one_budget[k] = batch_threads(c) != fsg::NT;
         r.candidate[k] = cand[k];
         r.ms[k] = f;
         r.n_candidates = (int)k + 1;

@@ -525,18 +525,21 @@ int fsg_perworld_step_timed(fsg_ctx *ctx, fsg_world *const *worlds, int n, int t
 typedef struct fsg_tuning {
     int32_t graph_ticks; /* ticks per captured HIP graph block: 1 (no graph), 4, 8, 16 or 32 */
     int32_t chunk_skip;  /* dirty-chunk skipping in batches: -1 each world's own setting, 0 off, 1 on */
-    int32_t occupancy;   /* tick-kernel register budget: 4 workgroups per CU, or 5: the most it can have (5 or 6) */
+    int32_t occupancy;   /* register budget of the 256-thread tick kernel: 4 workgroups per CU, or 5: the most
+                          * it can have (5 or 6).  Batches of few chunks (at most two per CU, with skipping
+                          * three and a half) run wider workgroups, to which it does not apply. */
     int32_t reserved;    /* 0 */
 } fsg_tuning;
 
 #define FSG_TUNE_MAX_CANDIDATES 32
 typedef struct fsg_tune_report {
     fsg_tuning best;
-    int32_t n_candidates;  /* candidates timed (0 when the choice came from the cache) */
+    int32_t n_candidates;  /* candidates compared (0 when the choice came from the cache) */
     int32_t from_cache;    /* 1: the cache held a choice for this GPU and world-size class */
     uint64_t size_class;   /* the cache key's world-size signature */
     fsg_tuning candidate[FSG_TUNE_MAX_CANDIDATES];
-    double ms[FSG_TUNE_MAX_CANDIDATES]; /* device time of sample_ticks ticks per candidate */
+    double ms[FSG_TUNE_MAX_CANDIDATES]; /* device time of sample_ticks ticks per candidate; one that differs
+                                         * only in an occupancy that does not apply has the other's */
 } fsg_tune_report;
 
 /* Current batch tuning of the context (default {16, -1, 5, 0}). */
