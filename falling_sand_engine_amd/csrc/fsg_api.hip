@@ -995,9 +995,14 @@ int stamp_rounds(fsg_ctx *c, const fsg::StampWorld *d_table, int n, uint32_t tot
     // one launch, but they cost more than a read and a write: unstamp of 62,500
     // pixels 100 us by exchange, 105 by copy; 98,000 128 and 128; 393,000 357
     // and 325; 1.6 M 1,161 and 1,084 (of the kernels 264 and 123).
-    const fsg::ClaimSave how = !save ? fsg::SAVE_NONE : total <= 1u << 16 ? fsg::SAVE_EXCHANGE : fsg::SAVE_COPY;
-    fsg::k_claims_init<<<g, 256, 0, c->stream>>>(a, how);
-    if (how == fsg::SAVE_COPY) fsg::k_claims_clear<<<g, 256, 0, c->stream>>>(a);
+    if (!save) {
+        fsg::k_claims_init<fsg::SAVE_NONE><<<g, 256, 0, c->stream>>>(a);
+    } else if (total <= 1u << 16) {
+        fsg::k_claims_init<fsg::SAVE_EXCHANGE><<<g, 256, 0, c->stream>>>(a);
+    } else {
+        fsg::k_claims_init<fsg::SAVE_COPY><<<g, 256, 0, c->stream>>>(a);
+        fsg::k_claims_clear<<<g, 256, 0, c->stream>>>(a);
+    }
     fsg::k_stamp_step<<<g, 256, 0, c->stream>>>(a, propose, 0);
     // the open list's reservations, one per 256 pixels, are the resolve's own
     // while they are few (unstamp, so / by k_stamp_compact: 10,000 pixels 80 /

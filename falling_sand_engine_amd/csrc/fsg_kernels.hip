@@ -1430,7 +1430,8 @@ __device__ __forceinline__ void slot_at(const StampWorld &W, uint64_t t, int d, 
     on = live && wx >= 0 && wy >= 0 && wx < W.W && wy < W.H;
 }
 
-__global__ void k_claims_init(StampArgs a, int save) {
+template <ClaimSave SAVE>
+__global__ void k_claims_init(StampArgs a) {
     const StampWorld &W = a.worlds[blockIdx.y];
     const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p == 0 && blockIdx.y == 0) *a.nopen = 0;
@@ -1447,11 +1448,11 @@ __global__ void k_claims_init(StampArgs a, int save) {
         int wx, wy;
         slot_at(W, t, d, live, on, wx, wy);
         uint64_t *slot = &W.claims[(size_t)wy * W.W + wx];
-        if (save == SAVE_COPY) {
+        if (SAVE == SAVE_COPY) {
             if (on) W.save[5 * (size_t)p + d] = *slot;
             continue;
         }
-        if (on && save == SAVE_EXCHANGE) {
+        if (on && SAVE == SAVE_EXCHANGE) {
             W.save[5 * (size_t)p + d] = atomicExch(reinterpret_cast<unsigned long long *>(slot), ~0ull);
         } else if (on) {
             *slot = ~0ull;
@@ -1459,6 +1460,9 @@ __global__ void k_claims_init(StampArgs a, int save) {
         if (W.flags) mark_tiles_wave(W.flags, on, on ? (uint32_t)((wy / TH) * W.tiles_x + wx / TW) : 0u);
     }
 }
+template __global__ void k_claims_init<SAVE_NONE>(StampArgs);
+template __global__ void k_claims_init<SAVE_EXCHANGE>(StampArgs);
+template __global__ void k_claims_init<SAVE_COPY>(StampArgs);
 
 __global__ void k_claims_clear(StampArgs a) {
     const StampWorld &W = a.worlds[blockIdx.y];

@@ -74,7 +74,8 @@ __global__ void k_pix_body(const fsg_body *bodies, const uint32_t *order, uint32
                            uint32_t *pix_body, uint32_t *zero, uint32_t nzero);
 // What happens to the contents of the slots that are cleared.
 enum ClaimSave { SAVE_NONE, SAVE_EXCHANGE, SAVE_COPY /* k_claims_clear follows */ };
-__global__ void k_claims_init(StampArgs a, int save);
+template <ClaimSave SAVE>
+__global__ void k_claims_init(StampArgs a);
 __global__ void k_claims_clear(StampArgs a);
 __global__ void k_claims_restore(StampArgs a, StampRes r);
 __global__ void k_displaced(StampWorld W, StampRes r);
