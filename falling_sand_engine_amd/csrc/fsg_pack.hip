@@ -618,16 +618,36 @@ __global__ __launch_bounds__(fsg_lz4::WT) void k_pack_decode_wide(const uint8_t 
     if (threadIdx.x == 0) result[blockIdx.x] = r;
 }
 
-// A workgroup per block up to six blocks per compute unit (two at a time are
-// resident, and half of an unpack's blocks are short), else a wave per block.
-// Unpack of 1 chunk 3.3 ms by waves, 1.0 by workgroups; of 256 (512 blocks) 3.7
-// and 1.1; of 576 3.8 and 2.7; of 1024 3.8 and 4.1, as a workgroup does more
-// work for a block than a wave.
-void launch_decode(const fsg_ctx *c, const uint8_t *in, const DecDesc *desc, uint8_t *out, int32_t *result, int n) {
-    if (n <= 6 * c->n_cu)
-        k_pack_decode_wide<<<(unsigned)n, fsg_lz4::WT, 0, c->stream>>>(in, desc, out, result);
+// A workgroup per block or a wave per block.  By waves a call takes what its
+// longest block takes, by its input bytes mostly; by workgroups, of which two
+// are resident on a compute unit, it grows with the blocks past that, as a
+// workgroup does more work for a block than a wave.  So up to two blocks per
+// compute unit it is workgroups, and up to six if the longest block's input is
+// long enough for the number of blocks.  us for
+// chunk images (two blocks each, half of them short), waves / workgroups: 1
+// chunk 3233 / 925, 256 3535 / 947, 400 3527 / 1599, 576 3522 / 2425, 768 3513
+// / 2577 (1024: 3.8 / 4.1 ms a call); nearly empty ones, of 3,003 bytes, 1 853
+// / 498, 256 876 / 595, 400 877 / 1019, 768 884 / 1732; 400 of 4.6 KB 976 /
+// 1053, of 7.9 KB 1168 / 1064; 576 of 7.7 KB 1163 / 1583, of 15.5 KB 1642 /
+// 1555; 768 of 15.5 KB 1636 / 1775, of 39 KB 2909 / 1728.  (Raw blocks as small
+// as 1,000 bytes, 512 of them, take 7 to 34 by waves and 14 to 43 so, which is
+// lost in such a call's copies; 1,500 go by waves.)
+bool decode_wide_pays(const fsg_ctx *c, const std::vector<DecDesc> &desc) {
+    const int64_t n = (int64_t)desc.size(), cu = c->n_cu;
+    if (n <= 2 * cu || n > 6 * cu) return n <= 2 * cu;
+    int32_t longest = 0;
+    for (const DecDesc &d : desc) longest = std::max(longest, d.n);
+    return longest * cu >= (n - 2 * cu) * 5120;
+}
+
+// desc: the blocks as d_desc has them.
+void launch_decode(const fsg_ctx *c, const uint8_t *in, const std::vector<DecDesc> &desc, const DecDesc *d_desc,
+                   uint8_t *out, int32_t *result) {
+    const unsigned n = (unsigned)desc.size();
+    if (decode_wide_pays(c, desc))
+        k_pack_decode_wide<<<n, fsg_lz4::WT, 0, c->stream>>>(in, d_desc, out, result);
     else
-        k_pack_decode<<<(unsigned)((n + DW - 1) / DW), 64 * DW, 0, c->stream>>>(in, desc, out, result, n);
+        k_pack_decode<<<(n + DW - 1) / DW, 64 * DW, 0, c->stream>>>(in, d_desc, out, result, (int)n);
 }
 
 // Little-endian u32 at a 4-byte aligned staging address (records are 12 or
@@ -890,7 +910,7 @@ extern "C" int fsg_world_unpack(fsg_world *w, int32_t x0, int32_t y0, int32_t nc
     if (int rc = fsg_impl::copy_in(c, d_desc, desc.data(), 2 * n * sizeof(DecDesc))) return rc;
     if (b_l2 + b_bg) HIPCHK(hipMemsetAsync(dec + b_desc + b_st, 0, b_l2 + b_bg, c->stream));  // failed chunks: 0
     uint8_t *raw = static_cast<uint8_t *>(w->d_pack_raw);
-    launch_decode(c, src, d_desc, raw, d_bst, (int)(2 * n));
+    launch_decode(c, src, desc, d_desc, raw, d_bst);
     k_pack_cells<<<(unsigned)n, 256, 0, c->stream>>>(raw, d_bst, d, d_cst);
     HIPCHK(hipGetLastError());
     if (int rc = fsg_impl::copy_out(c, {{status, d_cst, n * 4},
@@ -936,8 +956,8 @@ extern "C" int fsg_lz4_decode_blocks(fsg_ctx *c, const void *src, size_t src_len
     if (src_len) HIPCHK(hipMemcpyAsync(d_src.p, src, src_len, hipMemcpyHostToDevice, c->stream));
     if (out_len) HIPCHK(hipMemcpyAsync(d_out.p, out, out_len, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(d_desc.p, desc.data(), (size_t)n * sizeof(DecDesc), hipMemcpyHostToDevice, c->stream));
-    launch_decode(c, static_cast<const uint8_t *>(d_src.p), static_cast<const DecDesc *>(d_desc.p),
-                  static_cast<uint8_t *>(d_out.p), static_cast<int32_t *>(d_res.p), n);
+    launch_decode(c, static_cast<const uint8_t *>(d_src.p), desc, static_cast<const DecDesc *>(d_desc.p),
+                  static_cast<uint8_t *>(d_out.p), static_cast<int32_t *>(d_res.p));
     HIPCHK(hipGetLastError());
     if (out_len) HIPCHK(hipMemcpyAsync(out, d_out.p, out_len, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipMemcpyAsync(result, d_res.p, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));

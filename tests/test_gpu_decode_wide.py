@@ -65,3 +65,34 @@ def test_wide_decoder_matches_oracle_on_the_device(ctx, orc, per_call):
             want = orc.lz4_decode(src, cap)
             assert (out[:cap] if r == cap else None) == want, (a + k, len(src), cap, r)
             assert out[cap:] == b"\xa5" * 64, a + k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cx,cy", [(16, 16), (20, 20), (32, 24), (40, 20)])  # up to two blocks per CU, six, more
+@pytest.mark.parametrize("features", ["none", "few", "one chunk", "one bad"])
+def test_unpack_of_nearly_empty_chunks(ctx, cx, cy, features):
+    """Between two and six blocks per compute unit the longest input decides
+    between a wave and a workgroup per block: chunks of air, with scattered
+    cells, with one chunk of noise among them, and with one image cut short."""
+    W, H = 128 * cx, 128 * cy
+    rng = np.random.default_rng(cx)
+    cells = np.zeros((H, W), np.uint64)
+    noise = (rng.integers(0, 8, (H, W)).astype(np.uint64) | (rng.integers(0, 2**32, (H, W), dtype=np.uint64) << np.uint64(32)))
+    if features == "few":
+        at = rng.random((H, W)) < 0.01
+        cells[at] = noise[at]
+    elif features != "none":
+        cells[256:384, 128:256] = noise[256:384, 128:256]
+    print(f"unpack {cx}x{cy} {features}", flush=True)
+    with fsg.World(ctx, W, H, 1) as w:
+        w.upload(cells)
+        images = w.pack(0, 0, cx, cy)
+        w.generate(2, 3)
+        want = cells
+        if features == "one bad":
+            images[2 * cx + 1] = images[2 * cx + 1][:-1]
+            want = cells.copy()
+            want[256:384, 128:256] = w.download()[256:384, 128:256]
+        status = w.unpack(0, 0, cx, cy, images)[0]
+        assert [k for k, s in enumerate(status) if s] == ([2 * cx + 1] if features == "one bad" else [])
+        assert np.array_equal(w.download(), want)
