@@ -120,6 +120,7 @@ struct RowParse {
     int next;                  // first run start past the lane
     int pe;                    // end of the last match that starts before the lane (-1: none)
     uint64_t lanes;            // lanes in which a match starts
+    bool one;                  // the whole row is one match with the record before; nothing else is set
 
     // End of the run that starts at bit b of the lane.
     __device__ int end_of(int lane, int b) const {
@@ -135,6 +136,8 @@ struct RowParse {
         uint64_t left = __shfl_up(v1, 1, 64);
         const uint64_t wrap = __shfl(u1, 63, 64);  // the row above's last record comes before this row's first
         if (lane == 0) left = wrap;
+        one = row > 0 && (row + 1) * S <= n - fsg_lz4::MFLIMIT && !__ballot(((v1 ^ v0) | (v0 ^ left)) != 0);
+        if (one) return;
         uint32_t mL = eqmask<R>(v1 ^ v0) << R, mU = 0;
         if (i > 0) mL |= eqmask<R>(v0 ^ left);
         if (row) mU = eqmask<R>(v0 ^ u0) | eqmask<R>(v1 ^ u1) << R;
@@ -242,9 +245,10 @@ __device__ __forceinline__ int rows_before(int v, int *sums, int *total) {
 
 // A workgroup of PT threads encodes a block: its waves take the record rows in
 // turn, first for the rows' sizes, then to write them.  Bound by the VALU work of
-// the run loops, whose trips are the lane's with the most runs.  (A thread per
-// row walking its records: 1095 us for 256 chunks, so 190; a pack of 16384
-// chunks 11.0 ms, so 10.7.)
+// the run loops, whose trips are the lane's with the most runs, and of a row's
+// fixed part, which rows of one value do without.  (A thread per row walking its
+// records: 1326 us for 256 basin chunks, so 191, for 2304 1577 and 893; for 256
+// chunks of air 197 and 51, for 2304 881 and 459, 1282 with every row parsed.)
 template <int R, class Rec>
 __device__ void encode_block(int n, const Rec &rec, uint8_t *out, int cap, int32_t *size_out) {
     constexpr int S = CW * R, NW = PT / 64;
@@ -252,9 +256,19 @@ __device__ void encode_block(int n, const Rec &rec, uint8_t *out, int cap, int32
     __shared__ int hm[ROWS], lead[ROWS], trail[ROWS], rest[ROWS], carry[ROWS], start[ROWS], nxt[ROWS], sums[ROWS / 64];
     __shared__ int psum[ROWS + 1];
     __shared__ uint64_t has[ROWS / 64];
+    __shared__ uint8_t one[ROWS];  // rows that are one match: sized without a parse, and not read again
     for (int r = wv; r < rows; r += NW) {
         RowParse<R> p;
         p.parse(r, lane, n, rec);
+        if (lane == 0) one[r] = p.one;
+        if (p.one) {
+            if (lane == 0) {
+                hm[r] = 1;
+                lead[r] = trail[r] = 0;
+                rest[r] = 3 + extlen(S - fsg_lz4::MINMATCH);
+            }
+            continue;
+        }
         const int sum = wave_sum(p.size(lane), lane);
         const uint64_t lanes = p.lanes;
         // the row's first match, and the end of its last one
@@ -315,6 +329,17 @@ __device__ void encode_block(int n, const Rec &rec, uint8_t *out, int cap, int32
     }
     const Out o{out, cap};
     for (int r = wv; r < rows; r += NW) {
+        if (one[r]) {
+            if (lane == 0) {
+                constexpr int ml = S - fsg_lz4::MINMATCH;
+                o.put(start[r], (uint32_t)(min(carry[r], 15) << 4 | min(ml, 15)));
+                int oc = put_len(o, start[r] + 1, carry[r]) + carry[r];
+                o.put(oc++, (uint32_t)R);
+                o.put(oc++, 0u);
+                put_len(o, oc, ml);
+            }
+            continue;
+        }
         RowParse<R> p;
         p.parse(r, lane, n, rec);
         constexpr int W = RowParse<R>::W;

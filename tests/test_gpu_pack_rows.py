@@ -61,3 +61,37 @@ def test_row_patterns(ctx, orc, name, aux):
     assert (st == 0).all() and np.array_equal(back, cells)
     assert l2 is None or np.array_equal(l2b, l2)
     assert bg is None or np.array_equal(bgb, bg)
+
+
+def one_value_rows(rng, shape):
+    """Rows of one value, that of the record before them, which are not parsed."""
+    base = noise(rng, shape)
+    after = base.copy()
+    after[1::3] = base[0:-1:3, -1:][:after[1::3].shape[0]]   # behind rows that end in literals
+    pairs = base.copy()
+    pairs[3::5] = pairs[4::5] = base[2:-1:5, -1:][:pairs[4::5].shape[0]]  # two in a row, then literals again
+    most = np.full(shape, base[0, 0])
+    most[40, 17:19] = base[1, :2]                            # one row of many with something in it
+    ends = np.full(shape, base[0, 0])
+    ends[0, 0] = base[1, 1]                                  # the block's first record
+    ends[-1, -1] = base[2, 2]                                # and its last one
+    return dict(after=after, pairs=pairs, most=most, ends=ends)
+
+
+@pytest.mark.parametrize("name", ["after", "pairs", "most", "ends"])
+@pytest.mark.parametrize("aux", ["none", "same"])
+def test_rows_of_one_value(ctx, orc, name, aux):
+    print("pack rows of one value", name, aux, flush=True)
+    cells = one_value_rows(np.random.default_rng(5), (128, 128))[name]
+    cells = np.concatenate([cells, one_value_rows(np.random.default_rng(6), (128, 128))[name]], axis=1)
+    l2 = None if aux == "none" else cells.copy()
+    bg = None if aux == "none" else (cells >> np.uint64(32)).astype(np.uint32)
+    with fsg.World(ctx, 256, 128, 1, orc.default_config()) as w:
+        w.upload(cells)
+        got = w.pack(0, 0, 2, 1, layer2=l2, background=bg)
+        w.upload(np.zeros_like(cells))
+        st, _ph, l2b, bgb = w.unpack(0, 0, 2, 1, got, want_layer2=True, want_background=True)
+        back = w.download()
+    assert got == oracle_images(orc, cells, 0, 0, 2, 1, None, l2, bg)
+    assert (st == 0).all() and np.array_equal(back, cells)
+    assert l2 is None or (np.array_equal(l2b, l2) and np.array_equal(bgb, bg))
