@@ -322,13 +322,14 @@ int launch_tick(fsg_world *w) {
     using Yes = std::integral_constant<int, 1>;
     const unsigned cu = (unsigned)w->ctx->n_cu;
     if (sk && tiles <= 10 * cu) {
-        // skipping, tested by each workgroup.  us a tick (test and list as two
-        // launches of 256 threads / this): 64 chunks of 1024 threads 22.4 /
-        // 16.8, 256 29.8 / 18.3; 484 of 512 threads 30.6 / 22.3, 784 33.2 /
-        // 26.1 (of 256 threads 30.7); 1024 of 256 threads, all awake, 33.0 (of
-        // 512 34.0; half asleep 35.1 / 32.6); 2500 44.1 / 42.8.  From two
-        // rounds of resident workgroups on the sleeping ones' slots cost as
-        // much as the second launch: 4096 54.0 / 55.8, 16384 65 / 86.
+        // skipping, tested by each workgroup.  us a tick with a tenth of the
+        // chunks awake, test and list as two launches of 256 threads / this: 64
+        // chunks of 1024 threads 19.6 / 12.3, 256 20.3 / 12.6; 400 of 512 threads
+        // 20.1 / 13.4, 896 22.0 / 18.1; 1600 of 256 threads 25.4 / 21.7, 2560
+        // 26.7 / 25.4; all awake 896 30.2 / 28.9, 1600 43.4 / 44.3, 2560 55.9 /
+        // 54.0; none 896 5.5 / 5.2, 1600 5.5 / 5.5, 2560 5.4 / 7.1.  Above, the
+        // sleeping ones' slots cost as much as the second launch: 4096^2 basin
+        // world 54.0 / 55.8, 16384 chunks with a tenth awake 65 / 86.
         auto launch = [&](auto re_, auto zn_) {
             constexpr int R = decltype(re_)::value, Z = decltype(zn_)::value;
             if (tiles <= cu)

@@ -556,10 +556,7 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
     const uint64_t *__restrict__ in = w.buf[tick & 1];
     uint64_t *__restrict__ out = w.buf[(tick + 1) & 1];
     const bool skip = SK == 2 ? w.skip != 0 : SK != 0;
-    bool prev_changed = true, sleeps = false;
-    // a small world's tick is one chunk's latency: its region is loaded
-    // before the flags are waited for
-    constexpr bool LATE = SK == 1 && N != NT;
+    bool prev_changed = true;
     // Tick zone: no block of the region holds a zone cell (the chunk cannot
     // change), or some do and some do not (blocks are tested one by one).
     ZoneTest zt{};
@@ -571,11 +568,10 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
         const uint32_t *fr = w.flags[(tick + 1) & 1];
         const uint32_t self = fr[tile];
         const bool forced = tick == w.force_tick;
-        sleeps = SK != 3 && !chunk_awake<!LATE>(w, fr, tx, ty, forced);
+        const bool sleeps = SK != 3 && !chunk_awake<true>(w, fr, tx, ty, forced);
         // both state buffers hold this chunk unless it changed last tick
         prev_changed = forced || (self & F_ANY);
-        sleeps |= zt.dead && !prev_changed;
-        if (!LATE && sleeps) {
+        if (sleeps || (zt.dead && !prev_changed)) {
             if (tid == 0) w.flags[tick & 1][tile] = 0;
             return;
         }
@@ -639,10 +635,6 @@ __device__ __forceinline__ void tile_update(const DevWorld &w, uint64_t tick, in
                 if (row_in(k)) v[k] = load(1 + rr + RS * k, c2);
         }
         if (edge) ve = load(ey, ec2);
-    }
-    if (LATE && sleeps) {
-        if (tid == 0) w.flags[tick & 1][tile] = 0;
-        return;
     }
     // compact cells into LDS (origin residues in bits 9-14), colours kept in
     // registers until the write-back
