@@ -134,13 +134,13 @@ static char *staging(fsg_ctx *c, char *&at, size_t bytes) {
 // staging in small pieces (512 KiB: 213 us in, 233 us out; 64 KiB: 35 and 37);
 // through pinned memory and one memcpy it takes 30 and 30 (9 and 11).  Larger
 // ones are pinned in place by the runtime and gain nothing from a second copy.
-int copy_in(fsg_ctx *c, void *dst, const void *src, size_t bytes) {
+int copy_in(fsg_ctx *c, void *dst, const void *src, size_t bytes, bool kept) {
     if (bytes == 0) return FSG_OK;
     std::unique_lock<std::mutex> lk(c->stage_in_mu, std::defer_lock);
     if (bytes <= fsg_ctx::STAGE) lk.lock();
     if (!lk || !staging(c, c->h_in, fsg_ctx::IN_SLOTS * fsg_ctx::STAGE)) {
         HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));  // the source may go when this returns
+        if (!kept || bytes <= fsg_ctx::STAGE) HIPCHK(hipStreamSynchronize(c->stream));
         return FSG_OK;
     }
     if (c->in_used + bytes > fsg_ctx::STAGE) {  // the next slot, once its uploads are over
@@ -1097,7 +1097,9 @@ int ensure_stamp_buffers(fsg_world *w, size_t npix, int nb) {
 }
 
 // Validates bodies/pixels and uploads them; the pixel -> body map is made on
-// the device.  `zero`: result words to clear on the way.
+// the device.  Pixels beyond fsg_ctx::STAGE bytes must stay until the stream is
+// synchronised: a wait here would hold up a serving loop that admits worlds
+// while others tick.  `zero`: result words to clear on the way.
 int set_bodies(fsg_world *w, const fsg_body *bodies, int nb, const fsg_cell *pixels, size_t npix, uint32_t *zero,
                uint32_t nzero) {
     if (npix >= 0xFFFFFFFFull) return FSG_ERR_INVALID;
@@ -1127,7 +1129,7 @@ int set_bodies(fsg_world *w, const fsg_body *bodies, int nb, const fsg_cell *pix
     if (int rc = copy_in(c, w->d_bodies, w->bodies.data(), (size_t)nb * sizeof(fsg_body))) return rc;
     if (!npix) return FSG_OK;
     if (int rc = copy_in(c, w->d_order, order.data(), (size_t)nb * 4)) return rc;
-    if (int rc = copy_in(c, w->d_pixels, pixels, npix * 8)) return rc;
+    if (int rc = copy_in(c, w->d_pixels, pixels, npix * 8, true)) return rc;
     fsg::k_pix_body<<<grid_for(std::max<size_t>(npix, nzero), 256), 256, 0, c->stream>>>(
         w->d_bodies, w->d_order, (uint32_t)nb, (uint32_t)npix, w->d_pixbody, zero, nzero);
     HIPCHK(hipGetLastError());
@@ -1169,7 +1171,10 @@ extern "C" int fsg_world_stamp_bodies(fsg_world *w, const fsg_body *bodies, int 
     }
     if (int rc = set_bodies(w, bodies, nb, pixels, npix, r.count, r.count ? (uint32_t)(words + groups) : 0u)) return rc;
     if (npix)
-        if (int rc = stamp_single(w, false, r)) return rc;
+        if (int rc = stamp_single(w, false, r)) {
+            (void)hipStreamSynchronize(c->stream);  // the caller's pixels may go
+            return rc;
+        }
     std::vector<uint32_t> h(words, 0u);
     if (r.count) {
         if (cap) fsg::k_displaced<<<(unsigned)blocks, 256, 0, c->stream>>>(w->sw_host, r);

@@ -172,9 +172,10 @@ int dev_alloc(fsg_ctx *c, void **p, size_t bytes);
 void dev_free(void *p);
 void trim_cache(fsg_ctx *c, size_t keep);  // hipFree cached blocks down to `keep` bytes
 unsigned grid_for(size_t n, unsigned block);
-// Host -> device copy in stream order; the source may change when it returns
-// (waits for a copy of more than fsg_ctx::STAGE bytes).
-int copy_in(fsg_ctx *c, void *dst, const void *src, size_t bytes);
+// Host -> device copy in stream order; the source may change when it returns:
+// a copy of more than fsg_ctx::STAGE bytes is waited for, unless it is `kept`,
+// which promises that the source stays until the stream is synchronised.
+int copy_in(fsg_ctx *c, void *dst, const void *src, size_t bytes, bool kept = false);
 // Device -> host copies, behind everything on the stream; waits for them.
 struct CopyOut {
     void *dst;

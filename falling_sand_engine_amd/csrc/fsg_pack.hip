@@ -898,7 +898,6 @@ extern "C" int fsg_world_unpack(fsg_world *w, int32_t x0, int32_t y0, int32_t nc
             in_total += len;
         }
         if (grow(c, &w->d_pack_in, &w->pack_in_cap, std::max<size_t>(in_total, 1))) return FSG_ERR_NOMEM;
-        if (int rc = fsg_impl::copy_in(c, w->d_pack_in, images, in_total)) return rc;
         src = static_cast<const uint8_t *>(w->d_pack_in);
     } else {
         int64_t o = 0;
@@ -916,6 +915,8 @@ extern "C" int fsg_world_unpack(fsg_world *w, int32_t x0, int32_t y0, int32_t nc
     if (grow(c, &w->d_pack_raw, &w->pack_raw_cap, n * RAW) ||
         grow(c, &w->d_pack_dec, &w->pack_dec_cap, b_desc + b_st + b_l2 + b_bg))
         return FSG_ERR_NOMEM;
+    if (images)  // the last thing that can fail for want of memory is behind it
+        if (int rc = fsg_impl::copy_in(c, w->d_pack_in, images, in_total, true)) return rc;
     char *dec = static_cast<char *>(w->d_pack_dec);
     DecDesc *d_desc = reinterpret_cast<DecDesc *>(dec);
     int32_t *d_bst = reinterpret_cast<int32_t *>(dec + b_desc), *d_cst = d_bst + 2 * n;
