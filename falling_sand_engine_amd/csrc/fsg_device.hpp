@@ -20,7 +20,7 @@ constexpr int NT = 256;              // threads per workgroup (4 wave64)
 constexpr int WGS_PER_CU = 6;        // 256-thread tick workgroups resident per compute unit
 constexpr int FIVE_LDS = 2048;       // LDS beyond theirs with which one fewer fits
 constexpr int SMALL_NT = 1024;       // threads per chunk of a world with at most one chunk per CU
-constexpr int MEDIUM_NT = 512;       // threads per chunk of a world with at most two chunks per CU
+constexpr int MEDIUM_NT = 512;       // and with at most two (with skipping three and a half)
 constexpr int QUARTER_NT = 1024;     // threads per quarter chunk of a world with at most a quarter chunk per CU
 constexpr int MAX_IT = 3;            // largest cell_iter the fused kernel supports
 constexpr uint64_t MOVED = 0x100;

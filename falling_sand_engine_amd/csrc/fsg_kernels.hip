@@ -835,7 +835,8 @@ __device__ __forceinline__ int xcd_order(int i, int n, int g) {
 }
 
 // Small worlds: the same update with SMALL_NT (1024) threads per chunk (at
-// most one chunk per compute unit) or MEDIUM_NT (512, at most two).  A small
+// most one chunk per compute unit) or MEDIUM_NT (512, at most two, with
+// skipping three and a half).  A small
 // world leaves compute units idle, so a tick lasts one workgroup's latency;
 // more waves per chunk cut each wave's share of the phases and hide each
 // other's LDS latency.  With skipping (SK = 1) each workgroup tests its own

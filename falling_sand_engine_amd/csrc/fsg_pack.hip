@@ -26,7 +26,8 @@
 // bytes of a block are literals, as the format requires.
 //
 // Decoding: one wave per block (fsg_lz4.hpp), four waves per workgroup, or for
-// few blocks a workgroup each (fsg_lz4_wide.hpp), into a record staging area;
+// few blocks with enough input a workgroup each (fsg_lz4_wide.hpp), into a
+// record staging area;
 // then one workgroup per chunk checks every record and
 // writes the cells.
 #include "fsg_internal.hpp"

@@ -885,7 +885,12 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 // are for are bounded by one lane's chain of loads whatever their number, so
 // up to 2^25 cells they are always built (a pass of 10 particles on 4096^2
 // took 206 us with the on-demand map, of 1000 745; with the planes and the
-// launches below 84 and 115), and above for one particle per 2^17 cells.
+// launches below 84 and 115), and above for one particle per 2^17 cells, from
+// where they are ahead everywhere.  us a pass, planes / map, over ground: 8192^2
+// 200 particles 201 / 247, 400 208 / 492; 16384 x 8192 200 316 / 253, 800 329 /
+// 676; 16384^2 800 563 / 599, 3000 576 / 744; in the air 8192^2 200 183 / 130, 400
+// 196 / 332; 16384 x 8192 200 301 / 127, 400 311 / 338; 16384^2 1500 546 / 456,
+// 3000 552 / 584.
 bool want_planes(const fsg_world *w, size_t n) {
     const size_t cells = (size_t)w->d.W * w->d.H;
     return cells <= (size_t)1 << 25 || n >= cells >> 17;
